@@ -109,14 +109,82 @@ __global__ __launch_bounds__(kBlock) void support_kernel(d3d_scene s,
     out[3 * pid + 2] = ok ? p.z : NAN;
 }
 
-// collider.aabb() (containment.py:6-229), lane per collider.
-__global__ __launch_bounds__(kBlock) void aabb_kernel(d3d_scene s, const int32_t *__restrict__ shape,
-                                                      int64_t n, double *__restrict__ out) {
-    const int64_t pid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (pid >= n) return;
+// Box of the posed hull of lane `src` of the wavefront, by its 64 lanes: the
+// running minimum and maximum of the world vertices, lanes striding over the
+// hull, then butterfly merges (min and max are exact, so the box does not
+// depend on the order).  Every lane returns the box.
+__device__ __forceinline__ void hull_box_wave(const d3d_scene &s, const Shape &mine, int src,
+                                              double (&mn)[3], double (&mx)[3]) {
     Shape h;
+#pragma unroll
+    for (int j = 0; j < 9; ++j) h.R[j] = readlane_f64(mine.R[j], src);
+#pragma unroll
+    for (int j = 0; j < 3; ++j) h.t[j] = readlane_f64(mine.t[j], src);
+    const int nv = readlane_i32(mine.nv, src);
+    const int voff = readlane_i32(mine.voff, src), voff64 = readlane_i32(mine.voff64, src);
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        mn[a] = INFINITY;
+        mx[a] = -INFINITY;
+    }
+#pragma unroll 4
+    for (int j = lane_id(); j < nv; j += kWave) {
+        const v3 w = to_world(h, hull_vertex(s, voff, voff64, j));
+        mn[0] = w.x < mn[0] ? w.x : mn[0];
+        mx[0] = w.x > mx[0] ? w.x : mx[0];
+        mn[1] = w.y < mn[1] ? w.y : mn[1];
+        mx[1] = w.y > mx[1] ? w.y : mx[1];
+        mn[2] = w.z < mn[2] ? w.z : mn[2];
+        mx[2] = w.z > mx[2] ? w.z : mx[2];
+    }
+    for_butterfly<kWave>([&](auto o) {
+        constexpr int OFF = decltype(o)::value;
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+            double p, q;
+            xpair<OFF>(mn[a], p, q);
+            mn[a] = q < p ? q : p;
+            xpair<OFF>(mx[a], p, q);
+            mx[a] = q > p ? q : p;
+        }
+    });
+}
+
+// collider.aabb() (containment.py:6-229): a wavefront takes S colliders, one
+// per lane; analytic boxes and hulls of at most serial_max vertices are the
+// lane's own work, the larger hulls are swept by the whole wavefront, one
+// after the other.
+// Bound: memory for large batches of analytic colliders (1,048,576 boxes: 200
+// MB in and out in 32 us); with hulls, the longest chain of hull sweeps a
+// wavefront holds (a lane that walks its own hull takes one load round per
+// vertex: 5,003 mixed colliders with hulls of up to 4,096 vertices took 1,280
+// us that way, 42 us swept by the wavefront).
+template <int S>
+__global__ __launch_bounds__(kBlock) void aabb_kernel(d3d_scene s, const int32_t *__restrict__ shape,
+                                                      int64_t n, int serial_max,
+                                                      double *__restrict__ out) {
+    const int lane = lane_id();
+    const int64_t wave = ((int64_t)blockIdx.x * kBlock + threadIdx.x) / kWave;
+    const int64_t pid = wave * S + lane;
+    const bool valid = lane < S && pid < n;
+    Shape h = empty_shape();
+    const bool ok = valid && load_checked(s, shape[pid], h);
     double mn[3], mx[3];
-    if (!load_checked(s, shape[pid], h)) {
+    const bool coop = ok && h.type == D3D_HULL && h.nv > serial_max;
+    unsigned long long m = __ballot(coop);
+    while (m) {
+        const int src = __ffsll((long long)m) - 1;
+        m &= m - 1;
+        double bmn[3], bmx[3];
+        hull_box_wave(s, h, src, bmn, bmx);
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+            mn[a] = lane == src ? bmn[a] : mn[a];
+            mx[a] = lane == src ? bmx[a] : mx[a];
+        }
+    }
+    if (!valid) return;
+    if (!ok) {
 #pragma unroll
         for (int a = 0; a < 6; ++a) out[6 * pid + a] = NAN;
         return;
@@ -124,6 +192,7 @@ __global__ __launch_bounds__(kBlock) void aabb_kernel(d3d_scene s, const int32_t
     const double *R = h.R, *t = h.t;
     switch (h.type) {
     case D3D_HULL: {
+        if (coop) break;
 #pragma unroll
         for (int a = 0; a < 3; ++a) {
             mn[a] = INFINITY;
@@ -294,8 +363,20 @@ extern "C" int d3d_aabb_batch(const d3d_scene *scene, const int32_t *shape, int6
     D3D_CHECK_ARG(n >= 0, "n must be >= 0");
     if (n == 0) return D3D_OK;
     D3D_CHECK_ARG(shape && out, "NULL buffer");
-    hipLaunchKernelGGL(aabb_kernel, dim3(grid_for(n, kBlock)), dim3(kBlock), 0, (hipStream_t)stream,
-                       *scene, shape, n, out);
+    // Few colliders per wavefront keep its chain of hull sweeps short, many keep
+    // its lanes busy on analytic boxes; the line moves with the batch because a
+    // large one has wavefronts to spare.  4 / 16 / 64 colliders per wavefront:
+    // 16,384 mixed 37 / 67 / 89 us, 131,072 mixed 146 / 125 / 165 us, 262,144
+    // mixed 272 / 250 / 241 us; boxes alone 20,000 10.5 / 10.4 / 10.3 us, 200,000
+    // 36 / 14 / 11 us, 1,048,576 165 / 52 / 32 us.
+    const int serial_max = default_params().hull_serial_max;
+    auto launch = [&](auto kernel, int per_wave) {
+        hipLaunchKernelGGL(kernel, dim3(grid_for(n, kBlock / kWave * per_wave)), dim3(kBlock), 0,
+                           (hipStream_t)stream, *scene, shape, n, serial_max, out);
+    };
+    if (n < 65536) launch(aabb_kernel<4>, 4);
+    else if (n < 524288) launch(aabb_kernel<16>, 16);
+    else launch(aabb_kernel<64>, 64);
     D3D_CHECK_LAUNCH("aabb_kernel");
     return D3D_OK;
 }
