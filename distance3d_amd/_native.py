@@ -91,6 +91,8 @@ _SIGNATURES = {
     "d3d_instance_pairs": [_SCENE, _P, _P, _P, _P, _P, _P, _I64, _I64, _P, _P, _P, _P, _P],
     "d3d_bvh_build": [_P, _I64, _P, _I64, _P],
     "d3d_bvh_query": [_P, _I64, _P, _P, _I64, _P, _I64, _P, _P],
+    "d3d_bvh_query_sorted": [_P, _I64, _P, _P, _I64, _P, _I64, _P, _P, _I64, _P],
+    "d3d_bvh_query_sorted_finish": [_I64, _P, _I64, _P, _P, _I64, _P],
     "d3d_bvh_refit": [_P, _I64, _P, _I64, _P],
     "d3d_overlap_dense": [_P, _I64, _P, _I64, _P, _I64, _P, _P, _I64, _P],
     "d3d_mpr_batch": [_P, _P, _P, _P, _I64, _D, _I32, _I32, _P, _P, _P],
@@ -114,7 +116,7 @@ def exported_symbols():
     """Names of the C-ABI functions this binding uses."""
     return (["d3d_abi_version", "d3d_last_error", "d3d_init", "d3d_gjk_workspace_bytes",
              "d3d_bvh_bytes", "d3d_gjk_epa_workspace_bytes", "d3d_tet_pairs_workspace_bytes",
-             "d3d_overlap_dense_workspace_bytes"]
+             "d3d_overlap_dense_workspace_bytes", "d3d_bvh_query_sorted_workspace_bytes"]
             + list(_SIGNATURES))
 
 
@@ -140,6 +142,8 @@ def load_library(path=LIB_PATH):
                          "d3d_overlap_dense_workspace_bytes"):
                 getattr(lib, name).argtypes = [ctypes.c_int64]
                 getattr(lib, name).restype = ctypes.c_int64
+            lib.d3d_bvh_query_sorted_workspace_bytes.argtypes = [ctypes.c_int64, ctypes.c_int64]
+            lib.d3d_bvh_query_sorted_workspace_bytes.restype = ctypes.c_int64
             for name, argtypes in _SIGNATURES.items():
                 fn = getattr(lib, name)
                 fn.argtypes = argtypes

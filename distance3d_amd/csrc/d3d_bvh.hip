@@ -1,21 +1,19 @@
-// d3d_bvh.hip -- AABB broad phase on gfx950: linear BVH build and stackless
-// overlap queries.
+// d3d_bvh.hip -- AABB broad phase on gfx950: a packed 8-wide tree over
+// Morton-sorted boxes, its refit and its overlap queries.
 //
 // Build (all on the caller's stream, inside a caller-owned buffer):
-//   1. scene bounds of the AABB centres (block reduction)
+//   1. bounds of the AABB centres (block partials)
 //   2. 30-bit Morton codes of the centres
-//   3. radix sort of (code, index), 4 passes of 8 bits (LDS histograms; the
-//      order among equal codes is arbitrary, which the hierarchy tolerates)
-//   4. Karras hierarchy: internal node i covers a range of sorted leaves and
-//      splits at the highest differing code bit (ties broken by position)
-//   5. bottom-up refit: node boxes in FP32 rounded outward, so a node box
-//      contains the exact FP64 boxes below it
-//   6. ropes: every node stores the node to visit after its subtree
-// Query: one lane per query AABB walks left child / rope without a stack;
-// FP32 node tests are conservative, and each leaf hit is confirmed with the
-// reference's closed-interval FP64 test (aabb_tree.py:503-527), so the pair
-// set equals the brute-force set of all_aabbs_overlap exactly.  Hits are
-// appended with one atomic per wavefront (ballot compaction).
+//   3. radix sort of (code, index), 3 stable passes of 10 bits
+//   4. levels: level 0 holds the boxes in Morton order (FP32, rounded outward),
+//      a record of level k + 1 the union of 8 consecutive records of level k
+// The tree has no pointers: its shape follows from n alone, so a refit is step
+// 4 again, and a level-k record is found by its index.
+// Query: 8 lanes test the 8 children of a node in one coalesced load and push
+// the overlapping ones on an LDS stack; FP32 tests are conservative, and each
+// leaf hit is confirmed with the reference's closed-interval FP64 test
+// (aabb_tree.py:503-527), so the pair set equals the brute-force set of
+// all_aabbs_overlap exactly.
 #include "d3d_bvh_core.hpp"
 #include "d3d_device.hpp"
 #include "d3d_runtime.hpp"
@@ -23,94 +21,71 @@
 namespace d3d {
 
 constexpr int kBvhBlock = 256;
-constexpr int kSortItems = 16;  // items per thread in the radix sort
-constexpr int kSortTile = kBvhBlock * kSortItems;
+constexpr int kDigitBits = 10;
+constexpr int kDigits = 1 << kDigitBits;
+constexpr int kSortPasses = 3;  // 30-bit codes
 
+// A box of the tree: level 0 carries the original box index.  Rows that pad a
+// level to a multiple of 8 are NaN: no comparison with them holds.
 struct BvhNode {
     float lo[3];
-    int left;
+    int32_t id;
     float hi[3];
-    int escape;
+    int32_t pad;
 };
-
-struct BvhHeader {
-    int64_t n;
-    double slo[3], shi[3];
-    int64_t reserved[9];
-};
+static_assert(sizeof(BvhNode) == 32, "a node's 8 children are 256 consecutive bytes");
 
 struct BvhView {
-    BvhHeader *hdr;
-    BvhNode *nodes;     // 2n-1: internal 0..n-2, leaves n-1..2n-2
-    int32_t *leaf_orig; // sorted position -> original index
-    int32_t *parent;    // 2n-1
-    int32_t *right;     // n-1 (refit / ropes)
-    int32_t *flags;     // n-1 refit arrival counters
-    uint32_t *keys, *keys_alt;
-    int32_t *vals_alt;
-    int32_t *hist;      // tiles * 256
-    double *bpart;      // bound partials 6 * kBoundBlocks
+    BvhNode *nodes;
+    uint64_t *items, *items_alt;  // code << 32 | index
+    int32_t *order;               // sorted position -> original index
+    int32_t *hist;                // tiles x kDigits
+    int32_t *dtot;                // kDigits
+    double *bpart;                // bound partials 6 * kBoundBlocks
 };
 
 constexpr int kBoundBlocks = 256;
 
-__host__ __device__ inline int64_t sort_tiles(int64_t n) { return (n + kSortTile - 1) / kSortTile; }
+// Items of a sort tile per thread: a tile per block, so a small set takes
+// small tiles to have blocks for more than a few compute units, a large one
+// fewer columns to scan.  The whole build with 4 / 8 / 16 items: 5,003 boxes
+// 41 / 50 / 66 us, 262,144 boxes 66 / 69 / 86 us, 524,288 boxes 93 / 89 / 100
+// us, 1,048,576 boxes 152 / 138 / 137 us.
+__host__ __device__ inline int sort_items(int64_t n) { return n < 393216 ? 4 : 8; }
+__host__ __device__ inline int64_t sort_tiles(int64_t n) {
+    const int64_t tile = (int64_t)kBvhBlock * sort_items(n);
+    return (n + tile - 1) / tile;
+}
 
 __host__ __device__ inline int64_t align256(int64_t b) { return (b + 255) / 256 * 256; }
 
-__host__ __device__ inline int64_t bvh_bytes(int64_t n) {
+// One walk over the buffer's parts, for its size and for its pointers.
+inline int64_t bvh_layout(int64_t n, char *base, BvhView *v) {
     const int64_t m = n > 0 ? n : 1;
-    int64_t b = align256(sizeof(BvhHeader));
-    b += align256((2 * m - 1) * (int64_t)sizeof(BvhNode));
-    b += align256(m * 4);           // leaf_orig
-    b += align256((2 * m - 1) * 4); // parent
-    b += align256(m * 4);           // right
-    b += align256(m * 4);           // flags
-    b += 2 * align256(m * 4);       // keys, keys_alt
-    b += align256(m * 4);           // vals_alt
-    b += align256(sort_tiles(m) * 256 * 4);
-    b += align256(6 * kBoundBlocks * 8);
+    int64_t b = 0;
+    auto part = [&](int64_t bytes) {
+        char *p = base ? base + b : nullptr;
+        b += align256(bytes);
+        return p;
+    };
+    BvhView w;
+    w.nodes = (BvhNode *)part(bvh_levels(m).nodes * (int64_t)sizeof(BvhNode));
+    w.items = (uint64_t *)part(m * 8);
+    w.items_alt = (uint64_t *)part(m * 8);
+    w.order = (int32_t *)part(m * 4);
+    w.hist = (int32_t *)part(sort_tiles(m) * kDigits * 4);
+    w.dtot = (int32_t *)part(kDigits * 4);
+    w.bpart = (double *)part(6 * kBoundBlocks * 8);
+    if (v) *v = w;
     return b;
 }
 
-inline BvhView bvh_view(void *base, int64_t n) {
-    const int64_t m = n > 0 ? n : 1;
-    char *p = (char *)base;
-    BvhView v;
-    v.hdr = (BvhHeader *)p;
-    p += align256(sizeof(BvhHeader));
-    v.nodes = (BvhNode *)p;
-    p += align256((2 * m - 1) * (int64_t)sizeof(BvhNode));
-    v.leaf_orig = (int32_t *)p;
-    p += align256(m * 4);
-    v.parent = (int32_t *)p;
-    p += align256((2 * m - 1) * 4);
-    v.right = (int32_t *)p;
-    p += align256(m * 4);
-    v.flags = (int32_t *)p;
-    p += align256(m * 4);
-    v.keys = (uint32_t *)p;
-    p += align256(m * 4);
-    v.keys_alt = (uint32_t *)p;
-    p += align256(m * 4);
-    v.vals_alt = (int32_t *)p;
-    p += align256(m * 4);
-    v.hist = (int32_t *)p;
-    p += align256(sort_tiles(m) * 256 * 4);
-    v.bpart = (double *)p;
-    return v;
-}
+inline int64_t bvh_bytes(int64_t n) { return bvh_layout(n, nullptr, nullptr); }
 
-static int cu_count_bvh() {
-    static int cus = 0;
-    if (!cus) {
-        int dev = 0;
-        if (hipGetDevice(&dev) != hipSuccess ||
-            hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-            cus <= 0)
-            cus = 256;
-    }
-    return cus;
+inline BvhView bvh_view(void *base, int64_t n) {
+    BvhView v;
+    bvh_layout(n, (char *)base, &v);
+    return v;
 }
 
 // ------------------------------------------------------------- bounds
@@ -147,23 +122,6 @@ __global__ __launch_bounds__(kBvhBlock) void bvh_bounds_partial(const double *__
     if (threadIdx.x < 6) part[6 * blockIdx.x + threadIdx.x] = red[threadIdx.x][0];
 }
 
-__global__ __launch_bounds__(64) void bvh_bounds_final(const double *__restrict__ part, int nparts,
-                                                       BvhHeader *__restrict__ hdr, int64_t n) {
-    if (threadIdx.x == 0) {
-        double lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
-        for (int b = 0; b < nparts; ++b)
-            for (int a = 0; a < 3; ++a) {
-                lo[a] = fmin(lo[a], part[6 * b + a]);
-                hi[a] = fmax(hi[a], part[6 * b + 3 + a]);
-            }
-        hdr->n = n;
-        for (int a = 0; a < 3; ++a) {
-            hdr->slo[a] = lo[a];
-            hdr->shi[a] = hi[a];
-        }
-    }
-}
-
 __device__ __forceinline__ uint32_t spread10(uint32_t v) {
     v &= 0x3ffu;
     v = (v | (v << 16)) & 0x030000FFu;
@@ -173,310 +131,582 @@ __device__ __forceinline__ uint32_t spread10(uint32_t v) {
     return v;
 }
 
+__device__ __forceinline__ int item_digit(uint64_t item, int pass) {
+    return (int)(item >> (32 + kDigitBits * pass)) & (kDigits - 1);
+}
+
+// Morton codes of a sort tile, and the tile's counts of the first digit.  The
+// at most kBoundBlocks bound partials are merged again by every block (one per
+// thread, butterflies, then the wavefronts'): a launch of its own for that took
+// 5 us, and 51 us where one thread walked the partials.
 __global__ __launch_bounds__(kBvhBlock) void bvh_morton_kernel(const double *__restrict__ aabbs,
-                                                               int64_t n,
-                                                               const BvhHeader *__restrict__ hdr,
-                                                               uint32_t *__restrict__ keys,
-                                                               int32_t *__restrict__ vals) {
-    const int64_t i = (int64_t)blockIdx.x * kBvhBlock + threadIdx.x;
-    if (i >= n) return;
-    uint32_t q[3];
+                                                               int64_t n, int items,
+                                                               const double *__restrict__ part,
+                                                               int nparts, uint64_t *__restrict__ out,
+                                                               int32_t *__restrict__ hist) {
+    static_assert(kBoundBlocks == kBvhBlock, "one partial per thread");
+    constexpr int kWaves = kBvhBlock / kWave;
+    __shared__ double wred[kWaves][6];
+    __shared__ int32_t h[kDigits];
+    const int t = threadIdx.x;
+    for (int d = t; d < kDigits; d += kBvhBlock) h[d] = 0;
+    double b[6];
+#pragma unroll
+    for (int k = 0; k < 6; ++k) b[k] = t < nparts ? part[6 * t + k] : (k < 3 ? INFINITY : -INFINITY);
+    for_butterfly<kWave>([&](auto o) {
+        constexpr int OFF = decltype(o)::value;
+#pragma unroll
+        for (int k = 0; k < 6; ++k) {
+            double p, q;
+            xpair<OFF>(b[k], p, q);
+            b[k] = k < 3 ? fmin(p, q) : fmax(p, q);
+        }
+    });
+    if ((t & (kWave - 1)) == 0)
+#pragma unroll
+        for (int k = 0; k < 6; ++k) wred[t / kWave][k] = b[k];
+    __syncthreads();
+    double lo[3], ext[3];
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
-        const double c = (aabbs[6 * i + 2 * a] + aabbs[6 * i + 2 * a + 1]) * 0.5;
-        const double ext = hdr->shi[a] - hdr->slo[a];
-        double t = ext > 0.0 ? (c - hdr->slo[a]) / ext : 0.0;
-        t = fmin(fmax(t, 0.0), 1.0);
-        q[a] = (uint32_t)fmin(t * 1024.0, 1023.0);
+        double mn = wred[0][a], mx = wred[0][3 + a];
+#pragma unroll
+        for (int w = 1; w < kWaves; ++w) {
+            mn = fmin(mn, wred[w][a]);
+            mx = fmax(mx, wred[w][3 + a]);
+        }
+        lo[a] = mn;
+        ext[a] = mx - mn;
     }
-    keys[i] = (spread10(q[0]) << 2) | (spread10(q[1]) << 1) | spread10(q[2]);
-    vals[i] = (int32_t)i;
+    const int64_t base = (int64_t)blockIdx.x * kBvhBlock * items;
+    for (int j = 0; j < items; ++j) {
+        const int64_t i = base + (int64_t)j * kBvhBlock + t;
+        if (i >= n) break;
+        uint32_t q[3];
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+            const double c = (aabbs[6 * i + 2 * a] + aabbs[6 * i + 2 * a + 1]) * 0.5;
+            double u = ext[a] > 0.0 ? (c - lo[a]) / ext[a] : 0.0;
+            u = fmin(fmax(u, 0.0), 1.0);
+            q[a] = (uint32_t)fmin(u * 1024.0, 1023.0);
+        }
+        const uint32_t key = (spread10(q[0]) << 2) | (spread10(q[1]) << 1) | spread10(q[2]);
+        const uint64_t item = ((uint64_t)key << 32) | (uint32_t)i;
+        out[i] = item;
+        atomicAdd(&h[item_digit(item, 0)], 1);
+    }
+    __syncthreads();
+    for (int d = t; d < kDigits; d += kBvhBlock) hist[(int64_t)blockIdx.x * kDigits + d] = h[d];
 }
 
 // --------------------------------------------------------- radix sort
+//
+// Three passes over (code, index) items of 8 bytes, each: counts per tile
+// (rows of kDigits, tile-major, so both the count and the scatter read and
+// write whole rows), an exclusive scan of every digit's column, the scatter.
 
-__global__ __launch_bounds__(kBvhBlock) void rs_hist_kernel(const uint32_t *__restrict__ keys,
-                                                            int64_t n, int shift,
+__global__ __launch_bounds__(kBvhBlock) void rs_hist_kernel(const uint64_t *__restrict__ in, int64_t n,
+                                                            int items, int pass,
                                                             int32_t *__restrict__ hist) {
-    __shared__ int32_t h[256];
-    h[threadIdx.x] = 0;
+    __shared__ int32_t h[kDigits];
+    for (int d = threadIdx.x; d < kDigits; d += kBvhBlock) h[d] = 0;
     __syncthreads();
-    const int64_t base = (int64_t)blockIdx.x * kSortTile;
-    for (int j = 0; j < kSortItems; ++j) {
+    const int64_t base = (int64_t)blockIdx.x * kBvhBlock * items;
+    for (int j = 0; j < items; ++j) {
         const int64_t i = base + (int64_t)j * kBvhBlock + threadIdx.x;
-        if (i < n) atomicAdd(&h[(keys[i] >> shift) & 255u], 1);
+        if (i < n) atomicAdd(&h[item_digit(in[i], pass)], 1);
     }
     __syncthreads();
-    // digit-major layout: hist[digit * tiles + tile]
-    hist[(int64_t)threadIdx.x * gridDim.x + blockIdx.x] = h[threadIdx.x];
+    for (int d = threadIdx.x; d < kDigits; d += kBvhBlock) hist[(int64_t)blockIdx.x * kDigits + d] = h[d];
 }
 
-// exclusive scan of hist (digit-major) in place, one block
-__global__ __launch_bounds__(1024) void rs_scan_kernel(int32_t *__restrict__ hist, int64_t len) {
-    __shared__ int32_t part[1024];
-    const int t = threadIdx.x;
-    const int64_t per = (len + 1023) / 1024;
-    const int64_t b0 = t * per, b1 = (b0 + per < len) ? b0 + per : len;
-    int32_t s = 0;
-    for (int64_t i = b0; i < b1; ++i) s += hist[i];
-    part[t] = s;
+// Exclusive scan of every digit's column over the tiles, in place, and the
+// column sums: a block takes 64 digits, its 16 wavefronts a sixteenth of the
+// tiles each, so a wavefront's loads are whole 256-byte rows and independent of
+// each other.  (One block walking all columns in order took 112 us for 256
+// tiles of 256 digits; this takes 5 us for 256 tiles of 1,024.)
+constexpr int kScanSegs = 16;
+__global__ __launch_bounds__(kWave * kScanSegs) void rs_scan_kernel(int32_t *__restrict__ hist,
+                                                                    int64_t tiles,
+                                                                    int32_t *__restrict__ dtot) {
+    __shared__ int32_t seg[kScanSegs][kWave];
+    const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
+    const int d = blockIdx.x * kWave + lane;
+    const int64_t per = (tiles + kScanSegs - 1) / kScanSegs;
+    const int64_t t0 = min(per * w, tiles), t1 = min(t0 + per, tiles);
+    int32_t sum = 0;
+#pragma unroll 8
+    for (int64_t k = t0; k < t1; ++k) sum += hist[k * kDigits + d];
+    seg[w][lane] = sum;
     __syncthreads();
-    for (int off = 1; off < 1024; off <<= 1) {
-        const int32_t v = t >= off ? part[t - off] : 0;
-        __syncthreads();
-        part[t] += v;
-        __syncthreads();
-    }
-    int32_t run = part[t] - s;
-    for (int64_t i = b0; i < b1; ++i) {
-        const int32_t c = hist[i];
-        hist[i] = run;
+    int32_t run = 0;
+    for (int k = 0; k < w; ++k) run += seg[k][lane];
+    if (w == kScanSegs - 1) dtot[d] = run + sum;
+#pragma unroll 8
+    for (int64_t k = t0; k < t1; ++k) {
+        const int32_t c = hist[k * kDigits + d];
+        hist[k * kDigits + d] = run;
         run += c;
     }
 }
 
-// Stable scatter: items of a tile are ranked in index order.  Per chunk of
-// 256 items, each wavefront finds the lanes holding the same digit by
-// matching the 8 digit bits with ballots; a lane's position is the tile's
-// running count for its digit, plus the counts of the same digit in earlier
-// wavefronts of the chunk, plus its rank among the earlier lanes of its own
-// wavefront.  (LSD radix sort needs every pass to be stable.)
-__global__ __launch_bounds__(kBvhBlock) void rs_scatter_kernel(
-    const uint32_t *__restrict__ keys, const int32_t *__restrict__ vals, int64_t n, int shift,
-    const int32_t *__restrict__ offs, uint32_t *__restrict__ keys_out, int32_t *__restrict__ vals_out) {
+// Stable scatter of a tile (an LSD sort needs every pass to be stable).  A
+// wavefront owns a run of kItems * 64 consecutive items; it finds the lanes
+// holding the same digit by matching the digit bits with ballots, and its rank
+// is its own running count of the digit plus the earlier lanes' matches, with
+// no barrier between chunks.  Then the wavefronts' counts become positions:
+// digits before (the scan of the column sums, redone by every block), tiles
+// before (hist) and wavefronts before.  The last pass keeps the index only.
+template <int kItems, bool kLast>
+__global__ __launch_bounds__(kBvhBlock) void rs_scatter_kernel(const uint64_t *__restrict__ in,
+                                                               int64_t n, int pass,
+                                                               const int32_t *__restrict__ hist,
+                                                               const int32_t *__restrict__ dtot,
+                                                               uint64_t *__restrict__ out,
+                                                               int32_t *__restrict__ order) {
     constexpr int kWaves = kBvhBlock / kWave;
-    __shared__ int32_t run[256];
-    __shared__ int32_t wcnt[kWaves][256];
-    const int t = threadIdx.x;
-    const int lane = t & (kWave - 1);
-    const int wave = t / kWave;
-    run[t] = offs[(int64_t)t * gridDim.x + blockIdx.x];
-#pragma unroll
-    for (int w = 0; w < kWaves; ++w) wcnt[w][t] = 0;
-    __syncthreads();
+    constexpr int kPer = kDigits / kBvhBlock;  // digits per thread
+    __shared__ int32_t wcnt[kWaves][kDigits];
+    __shared__ int32_t wsum[kWaves];
+    const int t = threadIdx.x, lane = t & (kWave - 1), wave = t / kWave;
     const unsigned long long lt = lane == 0 ? 0ull : (~0ull >> (kWave - lane));
-    const int64_t base = (int64_t)blockIdx.x * kSortTile;
-    for (int j = 0; j < kSortItems; ++j) {
-        const int64_t i = base + (int64_t)j * kBvhBlock + t;
-        const bool valid = i < n;
-        const uint32_t k = valid ? keys[i] : 0u;
-        const int dig = (int)((k >> shift) & 255u);
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w)
+        for (int d = t; d < kDigits; d += kBvhBlock) wcnt[w][d] = 0;
+    const int64_t base = ((int64_t)blockIdx.x * kWaves + wave) * kItems * kWave + lane;
+    uint64_t item[kItems];
+    int rank[kItems];
+#pragma unroll
+    for (int j = 0; j < kItems; ++j) item[j] = base + j * kWave < n ? in[base + j * kWave] : 0ull;
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < kItems; ++j) {
+        const bool valid = base + j * kWave < n;
+        const int dig = item_digit(item[j], pass);
         unsigned long long same = __ballot(valid);
 #pragma unroll
-        for (int b = 0; b < 8; ++b) {
+        for (int b = 0; b < kDigitBits; ++b) {
             const unsigned long long m = __ballot((dig >> b) & 1);
             same &= ((dig >> b) & 1) ? m : ~m;
         }
-        const int rank = __popcll(same & lt);
-        if (valid && rank == 0) wcnt[wave][dig] = __popcll(same);
-        __syncthreads();
-        if (valid) {
-            int pos = run[dig] + rank;
-            for (int w = 0; w < wave; ++w) pos += wcnt[w][dig];
-            keys_out[pos] = k;
-            vals_out[pos] = vals[i];
-        }
-        __syncthreads();
-        int add = 0;
+        const int before = __popcll(same & lt);
+        rank[j] = wcnt[wave][dig] + before;
+        // the digit's lanes have read the count before its first lane raises it
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        if (valid && before == 0) wcnt[wave][dig] += __popcll(same);
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    }
+    // digits [kPer t, kPer t + kPer): start of the digit over all tiles
+    int32_t start[kPer];
+    int32_t sum = 0;
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) {
+        start[k] = sum;
+        sum += dtot[kPer * t + k];
+    }
+    int32_t incl = sum;
+#pragma unroll
+    for (int off = 1; off < kWave; off <<= 1) {
+        const int32_t v = __shfl_up(incl, off);
+        if (lane >= off) incl += v;
+    }
+    if (lane == kWave - 1) wsum[wave] = incl;
+    __syncthreads();
+    int32_t first = incl - sum;
+    for (int w = 0; w < wave; ++w) first += wsum[w];
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) {
+        const int d = kPer * t + k;
+        int32_t pos = first + start[k] + hist[(int64_t)blockIdx.x * kDigits + d];
 #pragma unroll
         for (int w = 0; w < kWaves; ++w) {
-            add += wcnt[w][t];
-            wcnt[w][t] = 0;
+            const int32_t c = wcnt[w][d];
+            wcnt[w][d] = pos;
+            pos += c;
         }
-        run[t] += add;
-        __syncthreads();
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < kItems; ++j) {
+        if (base + j * kWave >= n) break;
+        const int32_t pos = wcnt[wave][item_digit(item[j], pass)] + rank[j];
+        if (kLast) order[pos] = (int32_t)(uint32_t)item[j];
+        else out[pos] = item[j];
     }
 }
 
-// ---------------------------------------------------------- hierarchy
+// -------------------------------------------------------------- levels
 
-__global__ __launch_bounds__(kBvhBlock) void bvh_hierarchy_kernel(const uint32_t *__restrict__ keys,
-                                                                  int64_t n,
-                                                                  BvhNode *__restrict__ nodes,
-                                                                  int32_t *__restrict__ parent,
-                                                                  int32_t *__restrict__ right,
-                                                                  int32_t *__restrict__ flags) {
-    const int64_t ii = (int64_t)blockIdx.x * kBvhBlock + threadIdx.x;
-    if (ii >= n - 1) return;
-    const int i = (int)ii;
-    int lc, rc;
-    karras_children(keys, n, i, &lc, &rc);
-    nodes[i].left = lc;
-    right[i] = rc;
-    parent[lc] = i;
-    parent[rc] = i;
-    flags[i] = 0;
-    if (i == 0) parent[0] = -1;
+// Up to four consecutive levels in one launch: a thread makes one record of
+// level `base` (base 0: the outward-rounded FP32 box of its leaf; otherwise it
+// reads the record an earlier launch made), then 8 lanes, the 64 of the
+// wavefront and the block's 8 wavefronts merge theirs into records of the next
+// three.  Lanes past a level's count write the rows that pad it to a multiple
+// of 8.  Bound: the gather of the boxes in Morton order (1,048,576 boxes: 32
+// us, 48 bytes at random per box; the refit of the pointer tree this replaced
+// took 62 launches and 595 us).
+constexpr int kLevelBlock = 512;
+
+__device__ __forceinline__ void put_node(BvhNode *nd, const float (&lo)[3], const float (&hi)[3], int id) {
+    float4 *p = reinterpret_cast<float4 *>(nd);
+    p[0] = make_float4(lo[0], lo[1], lo[2], __int_as_float(id));
+    p[1] = make_float4(hi[0], hi[1], hi[2], 0.0f);
 }
 
-__device__ __forceinline__ void store_box(BvhNode *nd, const float lo[3], const float hi[3]) {
-    nd->lo[0] = lo[0];
-    nd->lo[1] = lo[1];
-    nd->lo[2] = lo[2];
-    nd->hi[0] = hi[0];
-    nd->hi[1] = hi[1];
-    nd->hi[2] = hi[2];
-}
-
-// Refit, level by level without device-wide fences: the leaf launch writes
-// the leaf boxes; each internal node keeps an arrival counter (flags) and the
-// child that arrives second appends the node to the next frontier list.  A
-// level launch gives every node of its frontier the union of its children's
-// boxes (written by earlier launches, so visible) and builds the next
-// frontier the same way.  A node splits its leaf range at the highest
-// differing bit of (30-bit Morton code, leaf index), so the tree has at most
-// 60 internal levels for n < 2^30 and kRefitLevels launches reach the root.
-constexpr int kRefitLevels = 62;
-
-__global__ __launch_bounds__(kBvhBlock) void bvh_refit_leaves(const double *__restrict__ aabbs,
-                                                              int64_t n,
-                                                              const int32_t *__restrict__ sorted_vals,
-                                                              int32_t *__restrict__ leaf_orig,
-                                                              BvhNode *__restrict__ nodes,
-                                                              const int32_t *__restrict__ parent,
-                                                              int32_t *__restrict__ flags,
-                                                              int32_t *__restrict__ front,
-                                                              int32_t *__restrict__ count) {
-    const int64_t i = (int64_t)blockIdx.x * kBvhBlock + threadIdx.x;
-    if (i >= n) return;
-    const int orig = sorted_vals[i];
-    leaf_orig[i] = orig;
-    float lo[3], hi[3];
+template <bool kLeaf>
+__global__ __launch_bounds__(kLevelBlock) void bvh_level_kernel(BvhLevels lv, int base,
+                                                                const double *__restrict__ aabbs,
+                                                                const int32_t *__restrict__ order,
+                                                                BvhNode *__restrict__ nodes) {
+    __shared__ float wlo[kLevelBlock / kWave][3], whi[kLevelBlock / kWave][3];
+    const int lane = lane_id(), wave = threadIdx.x / kWave;
+    int64_t i = (int64_t)blockIdx.x * kLevelBlock + threadIdx.x;
+    float lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
+    const float nan3[3] = {NAN, NAN, NAN};
+    const bool in = i < lv.count[base];
+    if (kLeaf) {
+        if (in) {
+            // a refit finds the order in the leaf records
+            const int32_t id = order ? order[i] : nodes[i].id;
+            const double *A = aabbs + 6 * (int64_t)id;
 #pragma unroll
-    for (int a = 0; a < 3; ++a) {
-        lo[a] = __double2float_rd(aabbs[6 * (int64_t)orig + 2 * a]);
-        hi[a] = __double2float_ru(aabbs[6 * (int64_t)orig + 2 * a + 1]);
-    }
-    const int leaf = (int)(n - 1 + i);
-    store_box(&nodes[leaf], lo, hi);
-    nodes[leaf].left = -1;
-    if (n == 1) return;
-    const int p = parent[leaf];
-    if (p >= 0 && atomicAdd(&flags[p], 1) == 1) front[atomicAdd(count, 1)] = p;
-}
-
-__global__ __launch_bounds__(kBvhBlock) void bvh_refit_level(BvhNode *__restrict__ nodes,
-                                                             const int32_t *__restrict__ parent,
-                                                             const int32_t *__restrict__ right,
-                                                             int32_t *__restrict__ flags,
-                                                             const int32_t *__restrict__ front_in,
-                                                             const int32_t *__restrict__ count_in,
-                                                             int32_t *__restrict__ front_out,
-                                                             int32_t *__restrict__ count_out) {
-    const int cnt = *count_in;
-    for (int i = blockIdx.x * kBvhBlock + threadIdx.x; i < cnt; i += gridDim.x * kBvhBlock) {
-        const int p = front_in[i];
-        const BvhNode na = nodes[nodes[p].left], nb = nodes[right[p]];
-        float lo[3], hi[3];
-#pragma unroll
-        for (int k = 0; k < 3; ++k) {
-            lo[k] = fminf(na.lo[k], nb.lo[k]);
-            hi[k] = fmaxf(na.hi[k], nb.hi[k]);
+            for (int a = 0; a < 3; ++a) {
+                lo[a] = __double2float_rd(A[2 * a]);
+                hi[a] = __double2float_ru(A[2 * a + 1]);
+            }
+            put_node(&nodes[i], lo, hi, id);
+        } else if (i < round8(lv.count[0])) {
+            put_node(&nodes[i], nan3, nan3, 0);
         }
-        store_box(&nodes[p], lo, hi);
-        const int q = parent[p];
-        if (q >= 0 && atomicAdd(&flags[q], 1) == 1) front_out[atomicAdd(count_out, 1)] = q;
+    } else if (in) {
+        const BvhNode nd = nodes[lv.off[base] + i];
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+            lo[a] = nd.lo[a];
+            hi[a] = nd.hi[a];
+        }
     }
+    auto merge = [&](auto o) {
+        constexpr int OFF = decltype(o)::value;
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+            float p, q;
+            xpair<OFF>(lo[a], p, q);
+            lo[a] = fminf(p, q);
+            xpair<OFF>(hi[a], p, q);
+            hi[a] = fmaxf(p, q);
+        }
+    };
+    auto put_level = [&](int level, bool mine) {
+        i >>= 3;
+        if (level > lv.top || !mine) return;
+        if (i < lv.count[level]) put_node(&nodes[lv.off[level] + i], lo, hi, -1);
+        else if (i < round8(lv.count[level])) put_node(&nodes[lv.off[level] + i], nan3, nan3, -1);
+    };
+    merge(IntC<1>{});
+    merge(IntC<2>{});
+    merge(IntC<4>{});
+    put_level(base + 1, (lane & 7) == 0);
+    merge(IntC<8>{});
+    merge(IntC<16>{});
+    merge(IntC<32>{});
+    put_level(base + 2, lane == 0);
+    if (lane == 0)
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+            wlo[wave][a] = lo[a];
+            whi[wave][a] = hi[a];
+        }
+    __syncthreads();
+    if (threadIdx.x == 0)
+#pragma unroll
+        for (int w = 1; w < kLevelBlock / kWave; ++w)
+#pragma unroll
+            for (int a = 0; a < 3; ++a) {
+                lo[a] = fminf(lo[a], wlo[w][a]);
+                hi[a] = fmaxf(hi[a], whi[w][a]);
+            }
+    put_level(base + 3, threadIdx.x == 0);
 }
 
-__global__ void bvh_zero_ints(int32_t *__restrict__ a, int64_t n) {
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-         i += (int64_t)gridDim.x * blockDim.x)
-        a[i] = 0;
-}
-
-// Boxes of every node from the leaf AABBs: leaf launch, then one launch per
-// tree level (see bvh_refit_leaves).  `flags` must be zero for the internal
-// nodes; leaf_orig holds the sorted permutation (read and rewritten in place
-// when sorted_vals == leaf_orig).
-static void refit_launches(const BvhView &v, const double *aabbs, int64_t n,
-                           const int32_t *sorted_vals, hipStream_t st) {
-    // frontiers ping-pong between keys_alt and vals_alt (free after the sort);
-    // per-level counters live in the histogram area
-    int32_t *fr[2] = {(int32_t *)v.keys_alt, v.vals_alt};
-    int32_t *cnt = v.hist;
-    const int nb = (int)((n + kBvhBlock - 1) / kBvhBlock);
-    hipLaunchKernelGGL(bvh_zero_ints, dim3(1), dim3(kBvhBlock), 0, st, cnt, (int64_t)(kRefitLevels + 1));
-    hipLaunchKernelGGL(bvh_refit_leaves, dim3(nb), dim3(kBvhBlock), 0, st, aabbs, n, sorted_vals,
-                       v.leaf_orig, v.nodes, v.parent, v.flags, fr[0], cnt);
-    if (n > 1) {
-        int lg = (int)((n / 2 + kBvhBlock - 1) / kBvhBlock);
-        const int cap = 4 * cu_count_bvh();
-        if (lg > cap) lg = cap;
-        if (lg < 1) lg = 1;
-        for (int L = 0; L < kRefitLevels; ++L)
-            hipLaunchKernelGGL(bvh_refit_level, dim3(lg), dim3(kBvhBlock), 0, st, v.nodes, v.parent,
-                               v.right, v.flags, fr[L & 1], cnt + L, fr[(L + 1) & 1], cnt + L + 1);
+// Every level from the boxes: order from the sort, or NULL for a refit.
+static void level_launches(const BvhView &v, const double *aabbs, int64_t n, const int32_t *order,
+                           hipStream_t st) {
+    const BvhLevels lv = bvh_levels(n);
+    for (int base = 0; base == 0 || base < lv.top; base += 3) {
+        // a block makes 512, 64, 8 and 1 rows of the four levels, so whole groups of
+        // 8 rows (with their padding) of the last one take a multiple of 8 blocks
+        int64_t blocks = (round8(lv.count[base]) + kLevelBlock - 1) / kLevelBlock;
+        if (base + 3 <= lv.top) blocks = round8(blocks);
+        if (base == 0)
+            hipLaunchKernelGGL(bvh_level_kernel<true>, dim3((unsigned)blocks), dim3(kLevelBlock), 0, st, lv, base,
+                               aabbs, order, v.nodes);
+        else
+            hipLaunchKernelGGL(bvh_level_kernel<false>, dim3((unsigned)blocks), dim3(kLevelBlock), 0, st, lv, base,
+                               aabbs, order, v.nodes);
     }
-}
-
-__global__ __launch_bounds__(kBvhBlock) void bvh_rope_kernel(int64_t n, BvhNode *__restrict__ nodes,
-                                                             const int32_t *__restrict__ parent,
-                                                             const int32_t *__restrict__ left,
-                                                             const int32_t *__restrict__ right) {
-    const int64_t k = (int64_t)blockIdx.x * kBvhBlock + threadIdx.x;
-    if (k >= 2 * n - 1) return;
-    nodes[k].escape = rope_of((int)k, n, parent, left, right);
-}
-
-// internal nodes' left children as a plain array for rope_of
-__global__ __launch_bounds__(kBvhBlock) void bvh_left_kernel(int64_t n, const BvhNode *__restrict__ nodes,
-                                                             int32_t *__restrict__ left) {
-    const int64_t k = (int64_t)blockIdx.x * kBvhBlock + threadIdx.x;
-    if (k < n - 1) left[k] = nodes[k].left;
 }
 
 // ------------------------------------------------------------- query
 
+// Rows of a query's own hit list; hits past it go to the overflow list.
+constexpr int kHitRows = 16;
+
+// Scratch of a sorted query (device pointers into the caller's workspace).
+struct QueryWs {
+    unsigned long long *base;  // per block: its queries' hits, then their start
+    int32_t *most;             // per block: most hits of one query
+    int32_t *count;            // per query
+    unsigned long long *off;   // per query: start of its pairs
+    int32_t *rows;             // per query kHitRows box indices, as found
+    int32_t *ovf;              // (query, rank, box) of the hits past the rows
+    int32_t *stage;            // per pair: box indices of long lists, as found
+};
+
+// Overlaps of the queries with the tree by groups of QL lanes: each round a
+// group pops QL / 8 nodes of its stack, 8 lanes each, one child per lane; the
+// overlapping children are pushed, or on level 0 tested exactly and reported.
+// A round costs one dependent load (a second one on level 0), so it is the
+// number of rounds in a row that bounds a query; many queries fill the chip
+// with 8 lanes each, a few take more nodes per round instead.  (One lane per
+// query on a pointer tree, a load per node: 65,536 queries of 1,048,576 boxes
+// 825 us; this kernel 126 us.)
+// kSorted: hits go to the query's rows (or the overflow list) with their
+// count; otherwise they are appended to `pairs` as they are found.
+//
+// The stack: popping one node of level k at a time never leaves more than
+// 7 k + 1 entries above its own place (each of its 8 children is finished
+// before the next is taken), so QL = 8 needs 7 kBvhMaxLevels + 1 rows.  Wider
+// groups take more than one node only while what they could push stays within
+// kWide rows, and one at a time above that.
+template <int QL, bool kSorted>
 __global__ __launch_bounds__(kBvhBlock) void bvh_query_kernel(
-    const BvhNode *__restrict__ nodes, const int32_t *__restrict__ leaf_orig, int64_t n,
-    const double *__restrict__ aabbs, const double *__restrict__ q, int64_t m,
-    int32_t *__restrict__ pairs, int64_t cap, unsigned long long *__restrict__ counter) {
-    const int64_t qi = (int64_t)blockIdx.x * kBvhBlock + threadIdx.x;
-    if (qi >= m) return;
+    BvhLevels lv, const BvhNode *__restrict__ nodes, const double *__restrict__ aabbs,
+    const double *__restrict__ q, int64_t m, int32_t *__restrict__ pairs, int64_t cap,
+    unsigned long long *__restrict__ counter, QueryWs ws) {
+    constexpr int kGroups = kBvhBlock / QL;
+    constexpr int W = QL / 8;
+    constexpr int kWide = W == 1 ? 0 : 20 * W;
+    constexpr int kStack = kWide + 7 * kBvhMaxLevels + 1;
+    __shared__ int32_t stack[kGroups][kStack];
+    __shared__ int64_t off[kBvhMaxLevels];
+    __shared__ int32_t found[kGroups];
+    const int t = threadIdx.x, g = t / QL, sub = t & (QL - 1);
+    const int slot = sub >> 3, child = sub & 7;
+    const int lane = lane_id();
+    if (t < kBvhMaxLevels) off[t] = lv.off[t];
+    const int64_t qi = (int64_t)blockIdx.x * kGroups + g;
+    const bool valid = qi < m;
     double Q[6];
-#pragma unroll
-    for (int k = 0; k < 6; ++k) Q[k] = q[6 * qi + k];
     float qlo[3], qhi[3];
+#pragma unroll
+    for (int k = 0; k < 6; ++k) Q[k] = valid ? q[6 * qi + k] : 0.0;
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
         qlo[a] = __double2float_rd(Q[2 * a]);
         qhi[a] = __double2float_ru(Q[2 * a + 1]);
     }
-    const int lane = lane_id();
-    const int leaf0 = (int)(n - 1);
-    int node = 0;
-    // a rope walk visits each node at most once; the cap only guards
-    // against a corrupted tree
-    for (int64_t steps = 0; node >= 0 && steps < 2 * n; ++steps) {
-        const BvhNode nd = nodes[node];
-        const bool ov = nd.lo[0] <= qhi[0] && nd.hi[0] >= qlo[0] && nd.lo[1] <= qhi[1] &&
-                        nd.hi[1] >= qlo[1] && nd.lo[2] <= qhi[2] && nd.hi[2] >= qlo[2];
-        bool hit = false;
-        int orig = 0;
-        if (ov && node >= leaf0) {
-            orig = leaf_orig[node - leaf0];
-            const double *A = aabbs + 6 * (int64_t)orig;
-            // aabb_overlap(tree_aabb, test_aabb), aabb_tree.py:520-527
-            hit = A[0] <= Q[1] && A[1] >= Q[0] && A[2] <= Q[3] && A[3] >= Q[2] && A[4] <= Q[5] &&
-                  A[5] >= Q[4];
-        }
-        const unsigned long long msk = __ballot(hit);
-        if (hit) {
-            const int first = __ffsll((long long)msk) - 1;
-            unsigned long long base = 0;
-            if (lane == first) base = atomicAdd(counter, (unsigned long long)__popcll(msk));
-            const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)base, first);
-            const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(base >> 32), first);
-            const unsigned long long pos =
-                (((unsigned long long)hi << 32) | lo) +
-                (unsigned long long)__popcll(msk & (lane == 0 ? 0ull : (~0ull >> (64 - lane))));
-            if (pos < (unsigned long long)cap) {
-                pairs[2 * pos] = (int32_t)qi;
-                pairs[2 * pos + 1] = orig;
+    if (sub == 0) stack[g][0] = lv.top << kNodeBits;
+    __syncthreads();
+    const unsigned long long lt = lane == 0 ? 0ull : (~0ull >> (kWave - lane));
+    int *const st = stack[g];
+    int sp = valid ? 1 : 0;
+    int cnt = 0;
+    while (sp > 0) {
+        const int take = sp + 7 * W <= kWide ? min(sp, W) : 1;
+        const int e = slot < take ? st[sp - 1 - slot] : -1;
+        sp -= take;
+        bool push = false, hit = false;
+        int level = 0, rec = 0, orig = 0;
+        if (e >= 0) {
+            level = e >> kNodeBits;
+            rec = 8 * (e & ((1 << kNodeBits) - 1)) + child;
+            const float4 *p = reinterpret_cast<const float4 *>(nodes + off[level] + rec);
+            const float4 lo = p[0], hi = p[1];
+            const bool ov = lo.x <= qhi[0] && hi.x >= qlo[0] && lo.y <= qhi[1] && hi.y >= qlo[1] &&
+                            lo.z <= qhi[2] && hi.z >= qlo[2];
+            push = ov && level > 0;
+            if (ov && level == 0) {
+                orig = __float_as_int(lo.w);
+                const double *A = aabbs + 6 * (int64_t)orig;
+                // aabb_overlap(tree_aabb, test_aabb), aabb_tree.py:520-527
+                hit = A[0] <= Q[1] && A[1] >= Q[0] && A[2] <= Q[3] && A[3] >= Q[2] && A[4] <= Q[5] &&
+                      A[5] >= Q[4];
             }
         }
-        node = (ov && node < leaf0) ? nd.left : nd.escape;
+        const unsigned long long pm = group_bits<QL>(__ballot(push), lane);
+        const unsigned long long below = group_bits<QL>(lt, lane);
+        if (push) st[sp + __popcll(pm & below)] = ((level - 1) << kNodeBits) | rec;
+        sp += __popcll(pm);
+        const unsigned long long all = __ballot(hit);
+        if (all != 0ull) {
+            const unsigned long long hm = group_bits<QL>(all, lane);
+            if constexpr (kSorted) {
+                if (hit) {
+                    const int r = cnt + __popcll(hm & below);
+                    if (r < kHitRows) {
+                        ws.rows[kHitRows * qi + r] = orig;
+                    } else {
+                        const unsigned long long pos = atomicAdd(counter, 1ull);
+                        if (pos < (unsigned long long)cap) {
+                            ws.ovf[3 * pos] = (int32_t)qi;
+                            ws.ovf[3 * pos + 1] = r;
+                            ws.ovf[3 * pos + 2] = orig;
+                        }
+                    }
+                }
+                cnt += __popcll(hm);
+            } else if (hit) {
+                const int first = __ffsll((long long)all) - 1;
+                unsigned long long b0 = 0;
+                if (lane == first) b0 = atomicAdd(counter, (unsigned long long)__popcll(all));
+                const unsigned l32 = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)b0, first);
+                const unsigned h32 = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(b0 >> 32), first);
+                const unsigned long long pos =
+                    (((unsigned long long)h32 << 32) | l32) + (unsigned long long)__popcll(all & lt);
+                if (pos < (unsigned long long)cap) {
+                    pairs[2 * pos] = (int32_t)qi;
+                    pairs[2 * pos + 1] = orig;
+                }
+            }
+        }
+        // the group's lanes read what the others pushed
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    }
+    if constexpr (kSorted) {
+        if (sub == 0) {
+            found[g] = cnt;
+            if (valid) ws.count[qi] = cnt;
+        }
+        __syncthreads();
+        if (t == 0) {
+            unsigned long long sum = 0;
+            int most = 0;
+            for (int k = 0; k < kGroups; ++k) {
+                sum += (unsigned long long)found[k];
+                most = max(most, found[k]);
+            }
+            ws.base[blockIdx.x] = sum;
+            ws.most[blockIdx.x] = most;
+        }
+    }
+}
+
+// Starts of the query blocks' pairs (exclusive scan of base in place) by one
+// block; result[0] the number of pairs, result[1] the most of one query.
+__global__ __launch_bounds__(1024) void query_scan_kernel(unsigned long long *__restrict__ base,
+                                                          const int32_t *__restrict__ most,
+                                                          int64_t blocks,
+                                                          unsigned long long *__restrict__ result) {
+    __shared__ unsigned long long part[1024];
+    __shared__ int32_t big[1024];
+    const int t = threadIdx.x;
+    const int64_t per = (blocks + 1023) / 1024;
+    const int64_t b0 = min((int64_t)t * per, blocks), b1 = min(b0 + per, blocks);
+    unsigned long long sum = 0;
+    int mx = 0;
+    for (int64_t k = b0; k < b1; ++k) {
+        sum += base[k];
+        mx = max(mx, most[k]);
+    }
+    part[t] = sum;
+    big[t] = mx;
+    __syncthreads();
+    for (int d = 1; d < 1024; d <<= 1) {
+        const unsigned long long v = t >= d ? part[t - d] : 0ull;
+        const int o = t >= d ? big[t - d] : 0;
+        __syncthreads();
+        part[t] += v;
+        big[t] = max(big[t], o);
+        __syncthreads();
+    }
+    unsigned long long run = part[t] - sum;
+    for (int64_t k = b0; k < b1; ++k) {
+        const unsigned long long c = base[k];
+        base[k] = run;
+        run += c;
+    }
+    if (t == 1023) {
+        result[0] = part[1023];
+        result[1] = (unsigned long long)big[1023];
+    }
+}
+
+// The pairs of kQueries queries (a block of the query kernel), 16 lanes each:
+// a list that fits the query's rows is ranked by counting the smaller indices
+// and written in order; of a longer one the rows are copied to its place in
+// `stage`, where query_spill_kernel adds the rest.
+template <int kQueries>
+__global__ __launch_bounds__(kQueries * kHitRows) void query_write_kernel(int64_t m, int64_t cap,
+                                                                          QueryWs ws,
+                                                                          int32_t *__restrict__ pairs) {
+    static_assert(kHitRows == 16 && kQueries >= 2 && kQueries <= 32, "16 lanes read at most two counts each");
+    __shared__ int32_t cnt[32];
+    __shared__ int32_t vals[kQueries][kHitRows];
+    const int t = threadIdx.x, g = t / kHitRows, sub = t & (kHitRows - 1);
+    const int64_t q0 = (int64_t)blockIdx.x * kQueries;
+    if (t < 32) cnt[t] = t < kQueries && q0 + t < m ? ws.count[q0 + t] : 0;
+    __syncthreads();
+    // hits of the block's earlier queries
+    int before = (sub < g ? cnt[sub] : 0) + (sub + 16 < g ? cnt[sub + 16] : 0);
+    for_butterfly<16>([&](auto o) {
+        int a, b;
+        xpair<decltype(o)::value>(before, a, b);
+        before = a + b;
+    });
+    const int64_t q = q0 + g;
+    const int k = cnt[g];
+    const unsigned long long off = ws.base[blockIdx.x] + (unsigned long long)before;
+    if (q < m && sub == 0) ws.off[q] = off;
+    const int b = sub < k ? ws.rows[kHitRows * q + sub] : 0x7fffffff;
+    vals[g][sub] = b;
+    __syncthreads();
+    if (sub >= k) return;
+    if (k > kHitRows) {
+        if (off + sub < (unsigned long long)cap) ws.stage[off + sub] = b;
+        return;
+    }
+    int rank = 0;
+#pragma unroll
+    for (int j = 0; j < kHitRows; ++j) rank += vals[g][j] < b ? 1 : 0;
+    const unsigned long long pos = off + (unsigned long long)rank;
+    if (pos < (unsigned long long)cap) {
+        pairs[2 * pos] = (int32_t)q;
+        pairs[2 * pos + 1] = b;
+    }
+}
+
+// The overflow list's hits to their places in `stage`.
+__global__ __launch_bounds__(kBvhBlock) void query_spill_kernel(
+    const unsigned long long *__restrict__ n_ovf, int64_t cap, QueryWs ws) {
+    const unsigned long long n = min(*n_ovf, (unsigned long long)cap);
+    for (unsigned long long i = (unsigned long long)blockIdx.x * kBvhBlock + threadIdx.x; i < n;
+         i += (unsigned long long)gridDim.x * kBvhBlock) {
+        const unsigned long long pos = ws.off[ws.ovf[3 * i]] + (unsigned long long)ws.ovf[3 * i + 1];
+        if (pos < (unsigned long long)cap) ws.stage[pos] = ws.ovf[3 * i + 2];
+    }
+}
+
+// Lists longer than a query's rows, ranked by counting in `stage` by one
+// wavefront each.
+__global__ __launch_bounds__(kBvhBlock) void query_long_kernel(int64_t m, int64_t cap, QueryWs ws,
+                                                               int32_t *__restrict__ pairs) {
+    const int lane = lane_id();
+    const int64_t waves = (int64_t)gridDim.x * (kBvhBlock / kWave);
+    for (int64_t q = ((int64_t)blockIdx.x * kBvhBlock + threadIdx.x) / kWave; q < m; q += waves) {
+        const int k = ws.count[q];
+        if (k <= kHitRows) continue;
+        const unsigned long long off = ws.off[q];
+        if (off + (unsigned long long)k > (unsigned long long)cap) continue;
+        const int32_t *list = ws.stage + off;
+        for (int i = lane; i < k; i += kWave) {
+            const int b = list[i];
+            int rank = 0;
+            for (int j = 0; j < k; ++j) rank += list[j] < b ? 1 : 0;
+            pairs[2 * (off + rank)] = (int32_t)q;
+            pairs[2 * (off + rank) + 1] = b;
+        }
     }
 }
 
@@ -583,6 +813,28 @@ extern "C" int64_t d3d_bvh_bytes(int64_t n) {
     return bvh_bytes(n);
 }
 
+template <int kItems>
+static void sort_launches(const BvhView &v, int64_t n, hipStream_t st) {
+    const int64_t tiles = sort_tiles(n);
+    uint64_t *in = v.items, *out = v.items_alt;
+    for (int pass = 0; pass < kSortPasses; ++pass) {
+        if (pass > 0)  // the code kernel counted the first digit
+            hipLaunchKernelGGL(rs_hist_kernel, dim3((unsigned)tiles), dim3(kBvhBlock), 0, st, in, n,
+                               kItems, pass, v.hist);
+        hipLaunchKernelGGL(rs_scan_kernel, dim3(kDigits / kWave), dim3(kWave * kScanSegs), 0, st, v.hist,
+                           tiles, v.dtot);
+        if (pass + 1 < kSortPasses)
+            hipLaunchKernelGGL(HIP_KERNEL_NAME(rs_scatter_kernel<kItems, false>), dim3((unsigned)tiles),
+                               dim3(kBvhBlock), 0, st, in, n, pass, v.hist, v.dtot, out, v.order);
+        else
+            hipLaunchKernelGGL(HIP_KERNEL_NAME(rs_scatter_kernel<kItems, true>), dim3((unsigned)tiles),
+                               dim3(kBvhBlock), 0, st, in, n, pass, v.hist, v.dtot, out, v.order);
+        uint64_t *x = in;
+        in = out;
+        out = x;
+    }
+}
+
 extern "C" int d3d_bvh_build(const double *aabbs, int64_t n, void *bvh, int64_t bvh_bytes_avail,
                              void *stream) {
     clear_error();
@@ -591,50 +843,19 @@ extern "C" int d3d_bvh_build(const double *aabbs, int64_t n, void *bvh, int64_t 
     D3D_CHECK_ARG(bvh_bytes_avail >= bvh_bytes(n), "bvh buffer smaller than d3d_bvh_bytes(n)");
     hipStream_t st = (hipStream_t)stream;
     BvhView v = bvh_view(bvh, n);
-    int nb = (int)((n + kBvhBlock - 1) / kBvhBlock);
-    const int nparts = nb < kBoundBlocks ? nb : kBoundBlocks;
+    const int64_t nb = (n + kBvhBlock - 1) / kBvhBlock;
+    const int nparts = (int)(nb < kBoundBlocks ? nb : kBoundBlocks);
     hipLaunchKernelGGL(bvh_bounds_partial, dim3(nparts), dim3(kBvhBlock), 0, st, aabbs, n, v.bpart);
     D3D_CHECK_LAUNCH("bvh_bounds_partial");
-    hipLaunchKernelGGL(bvh_bounds_final, dim3(1), dim3(64), 0, st, v.bpart, nparts, v.hdr, n);
-    D3D_CHECK_LAUNCH("bvh_bounds_final");
-    // codes into keys_alt/vals_alt, sorted back and forth; 4 passes end in keys/leaf_orig-source
-    uint32_t *kin = v.keys, *kout = v.keys_alt;
-    int32_t *vin = v.leaf_orig, *vout = v.vals_alt;
-    hipLaunchKernelGGL(bvh_morton_kernel, dim3(nb), dim3(kBvhBlock), 0, st, aabbs, n, v.hdr, kin, vin);
+    const int items = sort_items(n);
+    hipLaunchKernelGGL(bvh_morton_kernel, dim3((unsigned)sort_tiles(n)), dim3(kBvhBlock), 0, st, aabbs, n,
+                       items, v.bpart, nparts, v.items, v.hist);
     D3D_CHECK_LAUNCH("bvh_morton_kernel");
-    const int64_t tiles = sort_tiles(n);
-    for (int pass = 0; pass < 4; ++pass) {
-        const int shift = 8 * pass;
-        hipLaunchKernelGGL(rs_hist_kernel, dim3((unsigned)tiles), dim3(kBvhBlock), 0, st, kin, n,
-                           shift, v.hist);
-        D3D_CHECK_LAUNCH("rs_hist_kernel");
-        hipLaunchKernelGGL(rs_scan_kernel, dim3(1), dim3(1024), 0, st, v.hist, tiles * 256);
-        D3D_CHECK_LAUNCH("rs_scan_kernel");
-        hipLaunchKernelGGL(rs_scatter_kernel, dim3((unsigned)tiles), dim3(kBvhBlock), 0, st, kin, vin,
-                           n, shift, v.hist, kout, vout);
-        D3D_CHECK_LAUNCH("rs_scatter_kernel");
-        uint32_t *tk = kin; kin = kout; kout = tk;
-        int32_t *tv = vin; vin = vout; vout = tv;
-    }
-    // after 4 passes the sorted data is back in keys / leaf_orig's buffer
-    if (n > 1) {
-        const int ni = (int)((n - 1 + kBvhBlock - 1) / kBvhBlock);
-        hipLaunchKernelGGL(bvh_hierarchy_kernel, dim3(ni), dim3(kBvhBlock), 0, st, kin, n, v.nodes,
-                           v.parent, v.right, v.flags);
-        D3D_CHECK_LAUNCH("bvh_hierarchy_kernel");
-    }
-    refit_launches(v, aabbs, n, vin, st);
-    D3D_CHECK_LAUNCH("bvh_refit");
-    // ropes; the refit flags (no longer needed) hold the left-child array
-    if (n > 1) {
-        hipLaunchKernelGGL(bvh_left_kernel, dim3((unsigned)((n - 1 + kBvhBlock - 1) / kBvhBlock)),
-                           dim3(kBvhBlock), 0, st, n, v.nodes, v.flags);
-        D3D_CHECK_LAUNCH("bvh_left_kernel");
-    }
-    const int nn = (int)((2 * n - 1 + kBvhBlock - 1) / kBvhBlock);
-    hipLaunchKernelGGL(bvh_rope_kernel, dim3(nn), dim3(kBvhBlock), 0, st, n, v.nodes, v.parent,
-                       v.flags, v.right);
-    D3D_CHECK_LAUNCH("bvh_rope_kernel");
+    if (items == 4) sort_launches<4>(v, n, st);
+    else sort_launches<8>(v, n, st);
+    D3D_CHECK_LAUNCH("bvh_sort");
+    level_launches(v, aabbs, n, v.order, st);
+    D3D_CHECK_LAUNCH("bvh_level_kernel");
     return D3D_OK;
 }
 
@@ -644,18 +865,34 @@ extern "C" int d3d_bvh_refit(const double *aabbs, int64_t n, void *bvh, int64_t 
     D3D_CHECK_ARG(n >= 1 && n < (int64_t)0x40000000, "n must be in [1, 2^30)");
     D3D_CHECK_ARG(aabbs && bvh, "NULL buffer");
     D3D_CHECK_ARG(bvh_bytes_avail >= bvh_bytes(n), "bvh buffer smaller than d3d_bvh_bytes(n)");
-    hipStream_t st = (hipStream_t)stream;
-    BvhView v = bvh_view(bvh, n);
-    // the build left the ropes' left-child array in `flags`; the arrival
-    // counters of the refit need it zeroed (the ropes are already in the nodes)
-    if (n > 1) {
-        const int64_t zb = (n - 1 + kBvhBlock - 1) / kBvhBlock;
-        hipLaunchKernelGGL(bvh_zero_ints, dim3((unsigned)(zb < 1024 ? zb : 1024)), dim3(kBvhBlock), 0, st,
-                           v.flags, n - 1);
-    }
-    refit_launches(v, aabbs, n, v.leaf_orig, st);
-    D3D_CHECK_LAUNCH("bvh_refit");
+    level_launches(bvh_view(bvh, n), aabbs, n, nullptr, (hipStream_t)stream);
+    D3D_CHECK_LAUNCH("bvh_level_kernel");
     return D3D_OK;
+}
+
+// Lanes per query: few queries take wide groups (fewer rounds in a row each),
+// many fill the chip with narrow ones.  A sorted query of a tree of 1,048,576
+// boxes with 8 / 16 / 32 / 64 lanes: 300 queries 46 / 31 / 22 / 18 us, 5,003
+// queries 56 / 37 / 28 / 24, 16,384 queries 81 / 55 / 46 / 50, 32,768 queries
+// 94 / 73 / 74 / 88, 65,536 queries 130 / 132 / 138 / 173, 131,072 queries 232 /
+// 236 / 262 / 329 (the same order on trees of 5,003 and 100,003 boxes).
+static int query_lanes(int64_t m) { return m < 8192 ? 64 : m < 49152 ? 32 : 8; }
+
+template <bool kSorted>
+static void query_launch(const BvhView &v, int64_t n, const double *aabbs, const double *queries,
+                         int64_t m, int32_t *pairs, int64_t cap, unsigned long long *counter,
+                         const QueryWs &ws, hipStream_t st) {
+    const BvhLevels lv = bvh_levels(n);
+    auto go = [&](auto kernel, int lanes) {
+        const int per = kBvhBlock / lanes;
+        hipLaunchKernelGGL(kernel, dim3((unsigned)((m + per - 1) / per)), dim3(kBvhBlock), 0, st, lv,
+                           v.nodes, aabbs, queries, m, pairs, cap, counter, ws);
+    };
+    switch (query_lanes(m)) {
+    case 8: go(bvh_query_kernel<8, kSorted>, 8); break;
+    case 32: go(bvh_query_kernel<32, kSorted>, 32); break;
+    default: go(bvh_query_kernel<64, kSorted>, 64); break;
+    }
 }
 
 extern "C" int d3d_bvh_query(const void *bvh, int64_t n, const double *aabbs, const double *queries,
@@ -670,11 +907,89 @@ extern "C" int d3d_bvh_query(const void *bvh, int64_t n, const double *aabbs, co
     hipLaunchKernelGGL(bvh_zero_counter, dim3(1), dim3(1), 0, st, (unsigned long long *)n_pairs);
     D3D_CHECK_LAUNCH("bvh_zero_counter");
     if (m == 0) return D3D_OK;
-    BvhView v = bvh_view((void *)bvh, n);
-    const int nb = (int)((m + kBvhBlock - 1) / kBvhBlock);
-    hipLaunchKernelGGL(bvh_query_kernel, dim3(nb), dim3(kBvhBlock), 0, st, v.nodes, v.leaf_orig, n,
-                       aabbs, queries, m, pairs, cap, (unsigned long long *)n_pairs);
+    query_launch<false>(bvh_view((void *)bvh, n), n, aabbs, queries, m, pairs, cap,
+                        (unsigned long long *)n_pairs, QueryWs{}, st);
     D3D_CHECK_LAUNCH("bvh_query_kernel");
+    return D3D_OK;
+}
+
+// Parts of a sorted query's workspace, for its size and for its pointers.
+static int64_t query_layout(int64_t m, int64_t cap, char *base, QueryWs *ws) {
+    int64_t b = 0;
+    auto part = [&](int64_t bytes) {
+        char *p = base ? base + b : nullptr;
+        b += align256(bytes);
+        return p;
+    };
+    const int64_t per = m > 0 ? kBvhBlock / query_lanes(m) : 1;
+    const int64_t blocks = (m + per - 1) / per;
+    QueryWs w;
+    w.base = (unsigned long long *)part(blocks * 8);
+    w.most = (int32_t *)part(blocks * 4);
+    w.count = (int32_t *)part(m * 4);
+    w.off = (unsigned long long *)part(m * 8);
+    w.rows = (int32_t *)part(m * kHitRows * 4);
+    w.ovf = (int32_t *)part(cap * 12);
+    w.stage = (int32_t *)part(cap * 4);
+    if (ws) *ws = w;
+    return b;
+}
+
+extern "C" int64_t d3d_bvh_query_sorted_workspace_bytes(int64_t m, int64_t cap) {
+    if (m < 0 || cap < 0) return -1;
+    return query_layout(m, cap, nullptr, nullptr);
+}
+
+extern "C" int d3d_bvh_query_sorted(const void *bvh, int64_t n, const double *aabbs,
+                                    const double *queries, int64_t m, int32_t *pairs, int64_t cap,
+                                    uint64_t *result, void *workspace, int64_t workspace_bytes,
+                                    void *stream) {
+    clear_error();
+    D3D_CHECK_ARG(n >= 1 && n < (int64_t)0x40000000, "n must be in [1, 2^30)");
+    D3D_CHECK_ARG(m >= 1 && m < (int64_t)0x7fffffff, "m must be in [1, 2^31)");
+    D3D_CHECK_ARG(cap >= 1, "cap must be >= 1");
+    D3D_CHECK_ARG(bvh && aabbs && queries && pairs && result && workspace, "NULL buffer");
+    D3D_CHECK_ARG(workspace_bytes >= query_layout(m, cap, nullptr, nullptr), "workspace too small");
+    hipStream_t st = (hipStream_t)stream;
+    unsigned long long *res = (unsigned long long *)result;
+    QueryWs ws;
+    query_layout(m, cap, (char *)workspace, &ws);
+    hipLaunchKernelGGL(bvh_zero_counter, dim3(1), dim3(1), 0, st, res + 2);
+    D3D_CHECK_LAUNCH("bvh_zero_counter");
+    query_launch<true>(bvh_view((void *)bvh, n), n, aabbs, queries, m, pairs, cap, res + 2, ws, st);
+    D3D_CHECK_LAUNCH("bvh_query_kernel");
+    const int per = kBvhBlock / query_lanes(m);
+    const int64_t blocks = (m + per - 1) / per;
+    hipLaunchKernelGGL(query_scan_kernel, dim3(1), dim3(1024), 0, st, ws.base, ws.most, blocks, res);
+    D3D_CHECK_LAUNCH("query_scan_kernel");
+    auto write = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(per * kHitRows), 0, st, m, cap, ws, pairs);
+    };
+    if (per == 32) write(query_write_kernel<32>);
+    else if (per == 8) write(query_write_kernel<8>);
+    else write(query_write_kernel<4>);
+    D3D_CHECK_LAUNCH("query_write_kernel");
+    return D3D_OK;
+}
+
+extern "C" int d3d_bvh_query_sorted_finish(int64_t m, int32_t *pairs, int64_t cap,
+                                           const uint64_t *result, void *workspace,
+                                           int64_t workspace_bytes, void *stream) {
+    clear_error();
+    D3D_CHECK_ARG(m >= 1 && m < (int64_t)0x7fffffff, "m must be in [1, 2^31)");
+    D3D_CHECK_ARG(cap >= 1, "cap must be >= 1");
+    D3D_CHECK_ARG(pairs && result && workspace, "NULL buffer");
+    D3D_CHECK_ARG(workspace_bytes >= query_layout(m, cap, nullptr, nullptr), "workspace too small");
+    hipStream_t st = (hipStream_t)stream;
+    QueryWs ws;
+    query_layout(m, cap, (char *)workspace, &ws);
+    hipLaunchKernelGGL(query_spill_kernel, dim3(1024), dim3(kBvhBlock), 0, st,
+                       (const unsigned long long *)result + 2, cap, ws);
+    D3D_CHECK_LAUNCH("query_spill_kernel");
+    const int64_t blocks = (m * kWave + kBvhBlock - 1) / kBvhBlock;
+    hipLaunchKernelGGL(query_long_kernel, dim3((unsigned)(blocks < 4096 ? blocks : 4096)),
+                       dim3(kBvhBlock), 0, st, m, cap, ws, pairs);
+    D3D_CHECK_LAUNCH("query_long_kernel");
     return D3D_OK;
 }
 

@@ -1,12 +1,43 @@
-// d3d_bvh_core.hpp -- per-node logic of the linear BVH, written as plain
-// __host__ __device__ functions so the same code runs in the kernels and in a
-// host-side structural check (tests/bvh_host_check.hip).
+// d3d_bvh_core.hpp -- shapes of the box trees as plain __host__ __device__
+// functions: the levels of the packed 8-wide tree the kernels use, and the
+// binary radix hierarchy over sorted keys with its ropes, which the host-side
+// structural check (tests/bvh_host_check.hip) covers.
 #pragma once
 
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
 namespace d3d {
+
+// Packed tree over n sorted boxes: level 0 has n rows, level k + 1 one row per
+// 8 rows of level k, the top level at most 8.  Every level starts at a multiple
+// of 8 rows (nodes: rows in all).  An entry of a query's stack is
+// level << kNodeBits | index of the group of 8 rows: n < 2^30 leaves 27 bits
+// for the group and 10 levels.
+constexpr int kBvhMaxLevels = 10;
+constexpr int kNodeBits = 27;
+
+struct BvhLevels {
+    int64_t count[kBvhMaxLevels], off[kBvhMaxLevels];
+    int64_t nodes;
+    int top;
+};
+
+__host__ __device__ inline int64_t round8(int64_t n) { return (n + 7) / 8 * 8; }
+
+__host__ __device__ inline BvhLevels bvh_levels(int64_t n) {
+    BvhLevels lv;
+    lv.nodes = 0;
+    lv.top = -1;
+    for (int k = 0; k < kBvhMaxLevels; ++k) {
+        const bool more = k == 0 || lv.count[k - 1] > 8;
+        lv.count[k] = !more ? 0 : k == 0 ? n : (lv.count[k - 1] + 7) / 8;
+        lv.off[k] = lv.nodes;
+        lv.nodes += round8(lv.count[k]);
+        if (more) lv.top = k;
+    }
+    return lv;
+}
 
 __host__ __device__ inline int clz32(uint32_t v) { return v ? __builtin_clz(v) : 32; }
 

@@ -391,6 +391,10 @@ def bvh_query(bvh, queries, cap=None, counter=None, stream=None, sort=True):
     q = torch.as_tensor(queries, dtype=torch.float64)
     q = q.to(bvh.aabbs.device).reshape(-1, 3, 2).contiguous()
     m = q.shape[0]
+    if sort and m > 0:
+        pairs = _bvh_query_sorted(bvh, q, cap, counter, stream)
+        if pairs is not None:
+            return pairs
     if counter is None:
         counter = torch.zeros(1, dtype=torch.int64, device=q.device)
     if cap is None:
@@ -408,6 +412,47 @@ def bvh_query(bvh, queries, cap=None, counter=None, stream=None, sort=True):
         key = pairs[:, 0].to(torch.int64) * bvh.n + pairs[:, 1].to(torch.int64)
         pairs = pairs[torch.argsort(key)]
     return pairs
+
+
+# longest list of one query that is ordered by counting (quadratic in its
+# length) instead of a sort of all pairs
+SORTED_QUERY_MAX_LIST = 1024
+
+
+def _bvh_query_sorted(bvh, q, cap, counter, stream):
+    """The pairs of :func:`bvh_query` ordered by the library, or None when a
+    query's list is too long for that."""
+    import torch
+    m = q.shape[0]
+    # room for sixteen pairs per query (a scene's own boxes overlap several
+    # others each); a large batch, whose buffers would be large too, for four
+    cap = 4 * m + min(12 * m, 1 << 22) + 1024 if cap is None else max(int(cap), 1)
+    result = torch.empty(3, dtype=torch.int64, device=q.device)
+    while True:
+        pairs = torch.empty((cap, 2), dtype=torch.int32, device=q.device)
+        ws = torch.empty(int(lib().d3d_bvh_query_sorted_workspace_bytes(m, cap)), dtype=torch.uint8,
+                         device=q.device)
+        check(lib().d3d_bvh_query_sorted(ptr(bvh.buffer), bvh.n, ptr(bvh.aabbs), ptr(q), m,
+                                         ptr(pairs), cap, ptr(result), ptr(ws), ws.numel(),
+                                         stream_ptr(stream)), "d3d_bvh_query_sorted")
+        if stream is None:
+            k, longest, spilled = result.tolist()
+        else:
+            ws.record_stream(stream)
+            result.record_stream(stream)
+            with torch.cuda.stream(stream):
+                k, longest, spilled = result.tolist()
+        if spilled and longest > SORTED_QUERY_MAX_LIST:
+            return None
+        if k <= cap:
+            break
+        cap = k
+    if spilled:
+        check(lib().d3d_bvh_query_sorted_finish(m, ptr(pairs), cap, ptr(result), ptr(ws), ws.numel(),
+                                                stream_ptr(stream)), "d3d_bvh_query_sorted_finish")
+    if counter is not None:
+        counter[0] = k
+    return pairs[:k]
 
 
 class SceneView:

@@ -422,7 +422,7 @@ int d3d_tet_contact_forces(const double *T1, const double *e1, const int32_t *pa
                            double youngs_modulus1, double *out, void *stream);
 
 /*
- * Broad phase: linear BVH over n AABBs and overlap queries
+ * Broad phase: box tree over n AABBs and overlap queries
  * (aabb_tree.py:15-191 AabbTree, 381-403 query_overlap, 465-527
  * all_aabbs_overlap / aabb_overlap).
  *
@@ -439,6 +439,24 @@ int64_t d3d_bvh_bytes(int64_t n);
 int d3d_bvh_build(const double *aabbs, int64_t n, void *bvh, int64_t bvh_bytes, void *stream);
 int d3d_bvh_query(const void *bvh, int64_t n, const double *aabbs, const double *queries,
                   int64_t m, int32_t *pairs, int64_t cap, uint64_t *n_pairs, void *stream);
+
+/*
+ * d3d_bvh_query with the pairs in ascending order of (query, box).
+ * result: 3 device uint64: the number of pairs, the most pairs of one query,
+ * and the pairs that lists longer than 16 keep outside their queries' rows.
+ * When result[0] <= cap and result[2] == 0 the pairs are complete; when
+ * result[2] > 0 d3d_bvh_query_sorted_finish, with the same arguments, adds the
+ * long lists (quadratic in a list's length: past about a thousand pairs per
+ * query sort the output of d3d_bvh_query instead); when result[0] > cap call
+ * again with more room.  m and cap must be >= 1; the workspace
+ * (d3d_bvh_query_sorted_workspace_bytes(m, cap) bytes) is the caller's.
+ */
+int64_t d3d_bvh_query_sorted_workspace_bytes(int64_t m, int64_t cap);
+int d3d_bvh_query_sorted(const void *bvh, int64_t n, const double *aabbs, const double *queries,
+                         int64_t m, int32_t *pairs, int64_t cap, uint64_t *result, void *workspace,
+                         int64_t workspace_bytes, void *stream);
+int d3d_bvh_query_sorted_finish(int64_t m, int32_t *pairs, int64_t cap, const uint64_t *result,
+                                void *workspace, int64_t workspace_bytes, void *stream);
 
 /*
  * all_aabbs_overlap (aabb_tree.py:465-500) by brute force: every (i, j) with

@@ -37,3 +37,60 @@ def test_aabbs_of_mixed_hulls(box_scene, n):
     got = kernels.aabb_batch(box_scene.to_device(), ids).cpu().numpy()
     want = oracle.aabbs(box_scene, np.arange(box_scene.n_shapes, dtype=np.int32))
     assert np.array_equal(got, want[ids])
+
+
+def _boxes(rs, n, extent, wmax):
+    lo = rs.uniform(0.0, extent, (n, 3))
+    return np.stack([lo, lo + rs.uniform(0.01, wmax, (n, 3))], axis=2)
+
+
+def _overlaps(boxes, queries):
+    p, _ = oracle.all_aabbs_overlap(queries, boxes)
+    return p[np.lexsort((p[:, 1], p[:, 0]))]
+
+
+@pytest.mark.parametrize("n", (1, 7, 8, 9, 64, 65, 511, 513, 4095, 4097, 32769, 393215, 393217))
+def test_box_tree_levels(gpu, n):
+    """Trees around every level's edge and both sort tiles, with empty, NaN and
+    infinite boxes among them; again after a refit with new boxes."""
+    rs = np.random.RandomState(n)
+    extent = max(1.0, n ** (1.0 / 3.0))
+    boxes = _boxes(rs, n, extent, 0.8)
+    boxes[n // 2, 1, 1] = np.inf
+    boxes[n // 3, 0, 0] = np.nan
+    boxes[n // 5] = boxes[n // 5][:, ::-1]
+    queries = _boxes(rs, 67, extent, 1.5)
+    queries[3] = [[-np.inf, np.inf]] * 3 if n <= 513 else queries[3]
+    bvh = kernels.bvh_build(boxes)
+    assert np.array_equal(kernels.bvh_query(bvh, queries).cpu().numpy(), _overlaps(boxes, queries))
+    moved = boxes + rs.uniform(-1.0, 1.0, (n, 3, 1))
+    kernels.bvh_refit(bvh, moved)
+    assert np.array_equal(kernels.bvh_query(bvh, queries).cpu().numpy(), _overlaps(moved, queries))
+
+
+@pytest.mark.parametrize("m", (1, 3, 4, 5, 8191, 8192, 8203, 49151, 49152, 49183))
+def test_box_queries_by_lane_count(gpu, m):
+    """Every query width at its edges; lists shorter and longer than a query's
+    rows, sorted, unsorted and with too little room at first."""
+    rs = np.random.RandomState(m)
+    boxes = _boxes(rs, 600, 10.0, 0.5)
+    boxes[:40] = [[4.0, 4.5]] * 3  # lists of forty and more
+    queries = _boxes(rs, m, 10.0, 0.4)
+    queries[m // 2] = [[4.2, 4.3]] * 3
+    want = _overlaps(boxes, queries)
+    bvh = kernels.bvh_build(boxes)
+    assert np.array_equal(kernels.bvh_query(bvh, queries).cpu().numpy(), want)
+    assert np.array_equal(kernels.bvh_query(bvh, queries, cap=1).cpu().numpy(), want)
+    got = kernels.bvh_query(bvh, queries, sort=False).cpu().numpy()
+    assert np.array_equal(got[np.lexsort((got[:, 1], got[:, 0]))], want)
+
+
+@pytest.mark.parametrize("k", (15, 16, 17, 1023, 1024, 1025, 3000))
+def test_box_query_list_lengths(gpu, k):
+    """One query's list at the row limit and around the longest list that is
+    ordered by counting."""
+    boxes = np.zeros((k, 3, 2))
+    boxes[:, :, 1] = 1.0 + np.arange(k)[:, None]
+    queries = np.array([[[0.5, 0.6]] * 3, [[-2.0, -1.0]] * 3])
+    got = kernels.bvh_query(kernels.bvh_build(boxes), queries).cpu().numpy()
+    assert np.array_equal(got, np.stack([np.zeros(k, int), np.arange(k)], 1))
