@@ -328,20 +328,6 @@ __global__ __launch_bounds__(kBlock) void aabb_kernel(d3d_scene s, const int32_t
 
 using namespace d3d;
 
-static d3d_gjk_params default_params() {
-    d3d_gjk_params p;
-    p.tolerance = 1e-10;
-    p.max_distance_squared = 100000.0;
-    p.sanity_check = 1e-8;
-    p.max_iterations = 128;
-    p.hull_serial_max = 16;
-    for (int c = 0; c < D3D_NUM_CLASSES; ++c) p.lanes_per_pair[c] = 0;
-    p.blocks_per_cu = 0;
-    p.claim_factor = 0;
-    p.epa_blocks_per_cu = 0;
-    return p;
-}
-
 extern "C" int d3d_support_batch(const d3d_scene *scene, const int32_t *shape, const double *dirs,
                                  int64_t n, double *out, void *stream) {
     clear_error();

@@ -1,4 +1,5 @@
-// d3d_gjk_queue.hip -- batched GJK distance as a sorted, queue-fed pipeline.
+// d3d_gjk_queue.hip -- batched GJK distance and intersection as a sorted,
+// queue-fed pipeline (d3d_queue.hpp).
 //
 // 1. classify + counting sort (device): every pair gets a key
 //        work class (total hull vertices of the pair, 8 classes)
@@ -21,66 +22,9 @@
 #include <utility>
 #include <vector>
 
-#include "d3d_device.hpp"
-#include "d3d_runtime.hpp"
+#include "d3d_queue.hpp"
 
 namespace d3d {
-
-constexpr int kQBlock = 256;
-constexpr int kSizeClasses = 8;
-constexpr int kNumClasses = D3D_NUM_CLASSES;  // size class, + 8 when both are hulls
-static_assert(kNumClasses == 2 * kSizeClasses, "work classes: size x one or two hulls");
-constexpr int kNumTypes = 9;
-constexpr int kNumKeys = kNumClasses * kNumTypes * kNumTypes;
-constexpr int kBadInput = 0x200;
-
-// size class from the total hull vertex count of a pair
-__device__ __forceinline__ int work_class(int nverts) {
-    if (nverts == 0) return 0;
-    if (nverts <= 32) return 1;
-    if (nverts <= 128) return 2;
-    if (nverts <= 512) return 3;
-    if (nverts <= 1024) return 4;
-    if (nverts <= 2048) return 5;
-    if (nverts <= 4096) return 6;
-    return 7;
-}
-
-__device__ __forceinline__ int pair_key(const d3d_scene &s, int a, int b) {
-    if (a < 0 || b < 0 || (int64_t)a >= s.n_shapes || (int64_t)b >= s.n_shapes) return 0;
-    const int4 A = *reinterpret_cast<const int4 *>(s.shape_i32 + 4 * (int64_t)a);
-    const int4 B = *reinterpret_cast<const int4 *>(s.shape_i32 + 4 * (int64_t)b);
-    const int ta = (A.x >= 0 && A.x < kNumTypes) ? A.x : 0;
-    const int tb = (B.x >= 0 && B.x < kNumTypes) ? B.x : 0;
-    const int na = (ta == D3D_HULL) ? (A.y > 0 ? A.y : 0) : 0;
-    const int nb = (tb == D3D_HULL) ? (B.y > 0 ? B.y : 0) : 0;
-    const int cls = work_class(na + nb) + (na > 0 && nb > 0 ? kSizeClasses : 0);
-    return (cls * kNumTypes + ta) * kNumTypes + tb;
-}
-
-// Workspace layout (int32): hist[K] key_off[K] key_cur[K] cls_begin[C]
-// cls_count[C] cls_cursor[C] pad order[n]
-struct QueueWs {
-    int32_t *hist, *key_off, *key_cur, *cls_begin, *cls_count, *cls_cursor, *order;
-};
-
-__host__ __device__ constexpr int64_t ws_header_ints() {
-    return ((3 * kNumKeys + 3 * kNumClasses) + 63) / 64 * 64;
-}
-
-inline QueueWs ws_view(void *base, int64_t n) {
-    (void)n;
-    int32_t *p = (int32_t *)base;
-    QueueWs w;
-    w.hist = p;
-    w.key_off = p + kNumKeys;
-    w.key_cur = p + 2 * kNumKeys;
-    w.cls_begin = p + 3 * kNumKeys;
-    w.cls_count = w.cls_begin + kNumClasses;
-    w.cls_cursor = w.cls_count + kNumClasses;
-    w.order = p + ws_header_ints();
-    return w;
-}
 
 // Clears the header with a fill kernel (no memset node, so the sequence can
 // be captured in a graph and replayed).
@@ -169,59 +113,6 @@ __global__ __launch_bounds__(kQBlock) void queue_scatter_kernel(
 }
 
 // ------------------------------------------------------------- GJK state
-
-// Support points on A (P) and B (Q) of the simplex rows, in LDS: they are
-// touched only on append, compaction and at the end, so keeping them out of
-// VGPRs leaves the registers to the simplex solve.  Structure of arrays over
-// the block's threads: component c (slot * 6 + {Px,Py,Pz,Qx,Qy,Qz}) of thread
-// t at base[c * kQBlock + t], conflict-free.
-// P, Q rows of the simplex in LDS, structure of arrays with stride `st`
-// doubles: one slot per pair, shared by the G lanes of a group (all lanes
-// read it; the group's first lane, `wr`, writes it; LDS operations of a
-// wavefront complete in order, so the other lanes see the writes).
-struct PQ {
-    double *base;
-    int st;
-    bool wr;
-    __device__ __forceinline__ void put(int slot, v3 p, v3 q) const {
-        if (!wr) return;
-        double *b = base + slot * 6 * st;
-        b[0] = p.x;
-        b[st] = p.y;
-        b[2 * st] = p.z;
-        b[3 * st] = q.x;
-        b[4 * st] = q.y;
-        b[5 * st] = q.z;
-    }
-    __device__ __forceinline__ v3 P(int slot) const {
-        const double *b = base + slot * 6 * st;
-        return mk(b[0], b[st], b[2 * st]);
-    }
-    __device__ __forceinline__ v3 Q(int slot) const {
-        const double *b = base + slot * 6 * st;
-        return mk(b[3 * st], b[4 * st], b[5 * st]);
-    }
-    __device__ __forceinline__ void zero() const {
-        if (!wr) return;
-#pragma unroll
-        for (int c = 0; c < 24; ++c) base[c * st] = 0.0;
-    }
-    __device__ __forceinline__ void move(int from, int to) const {
-        if (from == to || !wr) return;
-        const double *a = base + from * 6 * st;
-        double *b = base + to * 6 * st;
-#pragma unroll
-        for (int c = 0; c < 6; ++c) b[c * st] = a[c * st];
-    }
-    // applies a compaction map (sources are >= destinations, so moving
-    // rows in increasing order reads every row before it is overwritten)
-    __device__ __forceinline__ void compact(const CompactMap &c) const {
-        if (!c.moved) return;
-        move(c.k0, 0);
-        if (c.m > 1) move(c.k1, 1);
-        if (c.m > 2) move(c.k2, 2);
-    }
-};
 
 struct GjkState {
     Simplex S;
@@ -412,372 +303,33 @@ __device__ __forceinline__ void gjk_write_bad(int64_t pid, const GjkOut &o) {
     epa_route(pid, false, o);
 }
 
-// ------------------------------------------------------- group supports
-
-__device__ __forceinline__ unsigned long long lanemask_lt(int lane) {
-    return lane == 0 ? 0ull : (~0ull >> (kWave - lane));
-}
-
-// ---------------------------------------------- LDS-resident hull vertices
-//
-// A wavefront's 12 KB LDS region holds the P/Q rows of its 64/G pair slots
-// (24 doubles each, interleaved) and, for hull classes with G >= 4, one vertex
-// cache per slot in the rest: the FP32 vertices of the pair's hulls in their
-// original order (A's at 0, B's after them; x, y and z arrays of
-// cache_verts<G>() entries), loaded once when the group takes the pair.  Every
-// support sweep of the pair then reads LDS instead of the pools.  Slot
-// strides are congruent to G modulo 64 words, so the 64/G groups sweeping at
-// the same time hit distinct banks.  Pairs whose hulls do not fit, or whose
-// vertices are not exact in FP32, sweep the pools as before.
-template <int G>
-__host__ __device__ constexpr int cache_stride_words() {
-    // (12288 bytes - P/Q rows) / slots, rounded down to G modulo 64 words
-    constexpr int room = (3072 - 48 * (kWave / G)) / (kWave / G);
-    return G >= kWave ? room : ((room - G) / 64) * 64 + G;
-}
-// With 8 to 32 lanes per pair the last kRecWords words of a slot hold the
-// pair's two collider records (the FP64 blocks of A and B, then their int32
-// parts), staged once when the group takes the pair, so the supports read
-// them from LDS instead of reloading them from memory at every iteration
-// (a wavefront-wide group loads them into scalar registers instead).
-constexpr int kRecWords = 2 * 16 * 2 + 2 * 4;
-template <int G>
-__host__ __device__ constexpr bool slot_recs() {
-    return G >= 8 && G < kWave;
-}
-// words of a slot for vertices or cluster records
-template <int G>
-__host__ __device__ constexpr int cache_words() {
-    return cache_stride_words<G>() - (slot_recs<G>() ? kRecWords : 0);
-}
-template <int G>
-__host__ __device__ constexpr int cache_verts() {
-    return cache_words<G>() / 3;
-}
-static_assert(cache_verts<4>() >= 32, "class 1 pairs fit a 4-lane slot");
-static_assert(cache_verts<64>() >= 1000, "one slot per wavefront holds 1000 vertices");
-static_assert(cache_words<8>() % 2 == 0 && cache_stride_words<8>() % 2 == 0 &&
-                  cache_words<16>() % 2 == 0 && cache_stride_words<16>() % 2 == 0,
-              "slot records are 8-byte aligned");
-
-// Collider record k (0: A, 1: B) of the pair in a slot (see slot_recs).
-__device__ __forceinline__ Shape slot_shape(const float *recs, int k) {
-    const double *f = reinterpret_cast<const double *>(recs) + 16 * k;
-    const int32_t *i = reinterpret_cast<const int32_t *>(recs + 64) + 4 * k;
-    Shape h;
-#pragma unroll
-    for (int j = 0; j < 9; ++j) h.R[j] = f[j];
-#pragma unroll
-    for (int j = 0; j < 3; ++j) {
-        h.t[j] = f[9 + j];
-        h.p[j] = f[12 + j];
+// GJK distance as a queue Mode.
+struct DistanceMode {
+    using State = GjkState;
+    using Out = GjkOut;
+    static __device__ __forceinline__ void clear(State &g, const PQ &pq) { gjk_init(g, pq); }
+    static __device__ __forceinline__ bool start(State &g, const PQ &pq, int, int,
+                                                 const d3d_gjk_params &, const Out &) {
+        gjk_init(g, pq);
+        return true;
     }
-    h.margin = f[15];
-    h.type = i[0];
-    h.nv = i[1];
-    h.voff = i[2];
-    h.voff64 = i[3];
-    return h;
-}
-
-// The collider record k of a pair: from the slot when it holds them, else
-// from the scene by index (kUniform: the same record for the whole
-// wavefront, so a wavefront-wide group loads it into scalar registers).
-template <int G, bool kUniform>
-__device__ __forceinline__ Shape pair_shape(const d3d_scene &s, const float *recs, int k, int idx) {
-    if constexpr (slot_recs<G>()) {
-        (void)s;
-        (void)idx;
-        return slot_shape(recs, k);
-    } else {
-        (void)recs;
-        (void)k;
-        return load_shape(s, (kUniform && G == kWave) ? wave_uniform(idx) : opaque(idx));
+    static __device__ __forceinline__ bool more(State &g, const d3d_gjk_params &prm) {
+        if (g.it < prm.max_iterations) return true;
+        g.state = D3D_ITER_CAP;
+        return false;
     }
-}
-
-// Copies the FP32 vertices of hull record h (validated) into the cache at
-// `at`, in original order (vorig), by the G lanes of a group.
-template <int G>
-__device__ __forceinline__ void cache_fill(const d3d_scene &s, const Shape &h, float *cache,
-                                           int at, int sub) {
-    constexpr int C = cache_verts<G>();
-    fill_orig<G>(s, h.voff, h.nv, cache, cache + C, cache + 2 * C, at, sub);
-}
-
-// Supports of records ia along d and ib along -d (see support_pair) for a
-// pair whose hull vertices are in the group's cache (A's first, nA of them).
-// Two hulls: the lower half of the group sweeps A while the upper half sweeps
-// B; one hull: the whole group sweeps it.  Same results as support_pair.
-template <int G>
-__device__ __forceinline__ SupportPair support_pair_cached(const d3d_scene &s, int ia, int ib, v3 d,
-                                                           int sub, const float *cache, int nA,
-                                                           bool two) {
-    constexpr int C = cache_verts<G>();
-    const float *cx = cache, *cy = cache + C, *cz = cache + 2 * C;
-    const float *recs = cache + cache_words<G>();
-    if (two) {
-        constexpr int H = G / 2;
-        const bool upper = sub >= H;
-        const Shape h = pair_shape<G, false>(s, recs, upper ? 1 : 0, upper ? ib : ia);
-        const v3 dir = vsel(upper, -d, d);
-        const int off = upper ? nA : 0;
-        const int j = lds_orig_argmax<H>(cx, cy, cz, off, h.nv, h.p[0], to_local(h, dir), sub & (H - 1));
-        const v3 v = mk((double)cx[off + j], (double)cy[off + j], (double)cz[off + j]);
-        const v3 out = apply_margin(h, to_world(h, v), dir);
-        SupportPair r;
-        halves<H>(out.x, r.a.x, r.b.x);
-        halves<H>(out.y, r.a.y, r.b.y);
-        halves<H>(out.z, r.a.z, r.b.z);
-        return r;
+    static __device__ __forceinline__ bool step(State &g, const PQ &pq, v3 p, v3 q,
+                                                const d3d_gjk_params &prm, const Out &) {
+        return gjk_distance_step(g, pq, p, q, prm.max_distance_squared,
+                                 prm.tolerance * prm.tolerance);
     }
-    v3 a = mk(0.0, 0.0, 0.0), b = a;
-#pragma unroll 1
-    for (int k = 0; k < 2; ++k) {
-        const Shape h = pair_shape<G, false>(s, recs, k, k == 0 ? ia : ib);
-        const v3 dir = vsel(k == 0, d, -d);
-        v3 out;
-        if (h.type == D3D_HULL) {
-            const int j = lds_orig_argmax<G>(cx, cy, cz, 0, h.nv, h.p[0], to_local(h, dir), sub);
-            out = to_world(h, mk((double)cx[j], (double)cy[j], (double)cz[j]));
-        } else {
-            out = support_analytic(h, dir);
-        }
-        out = apply_margin(h, out, dir);
-        a = vsel(k == 0, out, a);
-        b = vsel(k == 0, b, out);
+    static __device__ __forceinline__ void write(const State &g, const PQ &pq, int64_t pid,
+                                                 const d3d_gjk_params &prm, const Out &o) {
+        gjk_write(g, pq, pid, prm.sanity_check, o);
     }
-    return SupportPair{a, b};
-}
+    static __device__ __forceinline__ void bad(int64_t pid, const Out &o) { gjk_write_bad(pid, o); }
+};
 
-// Copies the cluster records of hull record h (validated, clustered) into
-// the slot at record `at`, by the G lanes of a group.
-template <int G>
-__device__ __forceinline__ void bounds_fill(const d3d_scene &s, const Shape &h, float4 *slot, int at,
-                                            int sub) {
-    const float4 *__restrict__ cl = reinterpret_cast<const float4 *>(s.clusters) + (int64_t)h.p[1];
-    const int nc = (int)h.p[2];
-#pragma unroll 4
-    for (int k = sub; k < nc; k += G) slot[at + k] = cl[k];
-}
-
-// Supports of records ia along d and ib along -d (see support_pair) for a pair
-// whose clustered hulls have their cluster records in the group's slot (A's
-// first, ncA of them): the sweeps read the bounds from LDS and the vertices
-// from the pools.  Same results as support_pair.
-template <int G>
-__device__ __forceinline__ SupportPair support_pair_bounds(const d3d_scene &s, int ia, int ib, v3 d,
-                                                           int sub, const float4 *slot, int ncA,
-                                                           int nrec) {
-    v3 a = mk(0.0, 0.0, 0.0), b = a;
-    if (G == kWave) d = mk(wave_uniform(d.x), wave_uniform(d.y), wave_uniform(d.z));
-    const float *recs = reinterpret_cast<const float *>(slot) + cache_words<G>();
-#pragma unroll 1
-    for (int k = 0; k < 2; ++k) {
-        const Shape h = pair_shape<G, true>(s, recs, k, k == 0 ? ia : ib);
-        const v3 dir = vsel(k == 0, d, -d);
-        v3 out;
-        if (h.type == D3D_HULL) {
-            const v3 l = to_local(h, dir);
-            const HullRef H = hull_ref(h);
-            // the slot's words past the cluster records hold the survivor list
-            int *list = const_cast<int *>(reinterpret_cast<const int *>(slot + nrec));
-            const int hi = H.nc > 0 ? hull_argmax<G, true>(s, H, l, sub, slot + (k == 0 ? 0 : ncA),
-                                                           list, cache_words<G>() - 4 * nrec)
-                                    : hull_argmax<G>(s, H, l, sub);
-            out = to_world(h, hull_vertex(s, h.voff, h.voff64, hi));
-        } else {
-            out = support_analytic(h, dir);
-        }
-        out = apply_margin(h, out, dir);
-        a = vsel(k == 0, out, a);
-        b = vsel(k == 0, b, out);
-    }
-    return SupportPair{a, b};
-}
-
-// One work class, G lanes per pair, by one wavefront: groups of G lanes take
-// pairs of the class (chunked claims from the class cursor) until the class is
-// exhausted and every group of the wavefront has finished its pair.  The
-// wavefront's P/Q slots are `pq_wave` (24 x 64 doubles, slot stride 64 / G);
-// with kCache (hull classes, G >= 4) the rest of the region holds each slot's
-// vertex cache.
-template <int G, bool kHull, bool kCache = (kHull && G >= 4)>
-__device__ __forceinline__ void run_class(const d3d_scene &s, const int32_t *__restrict__ pa,
-                                          const int32_t *__restrict__ pb,
-                                          const int32_t *__restrict__ order, int begin, int count,
-                                          int32_t *__restrict__ cursor, const d3d_gjk_params &prm,
-                                          const GjkOut &o, double *pq_wave, int chunk, int rot) {
-    const int lane = lane_id();
-    const int sub = lane & (G - 1);
-    const int leader = lane - sub;
-    const double tol2 = prm.tolerance * prm.tolerance;
-    const PQ pq{pq_wave + lane / G, kWave / G, sub == 0};
-    float *const cache = reinterpret_cast<float *>(pq_wave + 24 * (kWave / G)) +
-                         (lane / G) * cache_stride_words<G>();
-    GjkState g;
-    gjk_init(g, pq);
-    int ia = 0, ib = 0;
-    int pid = 0;
-    // pairs with their hull vertices in the group's cache: hull vertices of
-    // A (the offset of B's), both records hulls
-    bool cached = false, two = false;
-    int nA = 0;
-    // otherwise, pairs with their hulls' cluster records in the slot (ncA: A's
-    // record count, the offset of B's)
-    bool bounded = false;
-    int ncA = 0, nrec = 0;
-    // analytic classes: the two record types, read once per pair
-    int ta = 0, tb = 0;
-    bool have = false, exhausted = false;
-    // The first chunk of every wavefront is fixed by its rank (wavefront index
-    // minus `rot`, modulo the wavefront count): no atomic, so thousands of
-    // wavefronts do not queue on one cursor when a launch starts, and the
-    // rotation hands each class's fixed chunks to the wavefronts the earlier
-    // classes left without one.  Later chunks come from the cursor, past all
-    // fixed chunks; when the fixed chunks cover the class there are none.
-    const int n_waves = (int)gridDim.x * (kQBlock / kWave);
-    const int wv = (int)blockIdx.x * (kQBlock / kWave) + (int)threadIdx.x / kWave;
-    const int64_t r = (wv - rot + n_waves) % n_waves;
-    const int64_t fixed_end = (int64_t)n_waves * chunk;
-    const bool dynamic = fixed_end < count;
-    int cb = (int)min(r * chunk, (int64_t)count), ce = cb + chunk;
-    // the wavefront's unclaimed items are [cb, ce) of the class
-    while (true) {
-        const bool need = !have && !exhausted;
-        const unsigned long long m = __ballot(need && sub == 0);
-        if (m != 0ull) {
-            // groups take items from the wavefront's chunk of the class range;
-            // one atomic fetches the next chunk when it runs out.  Groups
-            // ranked past the items at hand wait for the next round.
-            const int c = __popcll(m);
-            const int rank = __popcll(m & lanemask_lt(leader));
-            const int avail = ce - cb;
-            int nb = 0;
-            if (avail < c) {
-                const int first = __ffsll((long long)m) - 1;
-                if (dynamic) {
-                    if (lane == first) nb = (int)fixed_end + atomicAdd(cursor, chunk);
-                    nb = readlane_i32(nb, first);
-                } else {
-                    nb = count;  // nothing past the fixed chunks
-                }
-            }
-            const int base = rank < avail ? cb : nb - avail;
-            const bool served = rank < avail + (avail < c ? chunk : 0);
-            if (avail < c) {
-                const int taken = c - avail < chunk ? c - avail : chunk;
-                cb = nb + taken;
-                ce = nb + chunk;
-            } else {
-                cb += c;
-            }
-            if (need && served) {
-                const int idx = base + rank;
-                if (idx < count) {
-                    pid = order[begin + idx];
-                    ia = pa[pid];
-                    ib = pb[pid];
-                    Shape A, B;
-                    const bool okA = load_checked(s, ia, A);
-                    const bool okB = load_checked(s, ib, B);
-                    const bool ok =
-                        okA && okB && (kHull || (A.type != D3D_HULL && B.type != D3D_HULL));
-                    gjk_init(g, pq);
-                    if (ok) {
-                        have = true;
-                        ta = A.type;
-                        tb = B.type;
-                        if constexpr (kCache) {
-                            const bool ha = A.type == D3D_HULL, hb = B.type == D3D_HULL;
-                            nA = ha ? A.nv : 0;
-                            const int nB = hb ? B.nv : 0;
-                            cached = nA + nB <= cache_verts<G>() && (!ha || A.voff64 < 0) &&
-                                     (!hb || B.voff64 < 0);
-                            two = ha && hb;
-                            ncA = ha ? (int)A.p[2] : 0;
-                            const int ncB = hb ? (int)B.p[2] : 0;
-                            bounded = !cached && ncA + ncB > 0 &&
-                                      4 * (ncA + ncB) <= cache_words<G>();
-                            nrec = ncA + ncB;
-                            if (cached) {
-                                if (ha) cache_fill<G>(s, A, cache, 0, sub);
-                                if (hb) cache_fill<G>(s, B, cache, nA, sub);
-                            } else if (bounded) {
-                                float4 *slot = reinterpret_cast<float4 *>(cache);
-                                if (ncA > 0) bounds_fill<G>(s, A, slot, 0, sub);
-                                if (ncB > 0) bounds_fill<G>(s, B, slot, ncA, sub);
-                            }
-                            if constexpr (slot_recs<G>()) {
-                                double *rf = reinterpret_cast<double *>(cache + cache_words<G>());
-                                int32_t *ri = reinterpret_cast<int32_t *>(rf + 32);
-                                for (int k = sub; k < 40; k += G) {
-                                    if (k < 32)
-                                        rf[k] = s.shape_f64[16 * (int64_t)(k < 16 ? ia : ib) + (k & 15)];
-                                    else
-                                        ri[k - 32] = s.shape_i32[4 * (int64_t)(k < 36 ? ia : ib) + (k & 3)];
-                                }
-                            }
-                            // the group's lanes read what the others wrote
-                            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-                            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-                        }
-                    } else if (sub == 0) {
-                        gjk_write_bad(pid, o);
-                    }
-                } else {
-                    exhausted = true;
-                }
-            }
-            // the cursor only grows: once any group sees an item past the end
-            // the class is empty for every group of the wavefront
-            if (__ballot(exhausted) != 0ull) exhausted = true;
-        }
-        if (__ballot(have) == 0ull) {
-            if (__ballot(!exhausted) == 0ull) break;
-            continue;
-        }
-        if (have) {
-            bool running = true;
-            if (g.it >= prm.max_iterations) {
-                g.state = D3D_ITER_CAP;
-                running = false;
-            } else {
-                // the records were validated when the pair was taken
-                SupportPair w;
-                // a wavefront in its support sweep (memory rounds) issues ahead of
-                // those in their FP64 simplex step, so its loads go out sooner;
-                // priority only orders issue between the SIMD's wavefronts
-                __builtin_amdgcn_s_setprio(2);
-                if constexpr (kCache) {
-                    if (cached)
-                        w = support_pair_cached<G>(s, ia, ib, g.d, sub, cache, nA, two);
-                    else if (bounded)
-                        w = support_pair_bounds<G>(s, ia, ib, g.d, sub,
-                                                   reinterpret_cast<const float4 *>(cache), ncA, nrec);
-                    else
-                        w = support_pair<G, kHull>(s, ia, ib, g.d, sub);
-                } else if constexpr (!kHull) {
-                    w = support_pair_analytic(s, ia, ib, ta, tb, g.d);
-                } else {
-                    w = support_pair<G, kHull>(s, ia, ib, g.d, sub);
-                }
-                __builtin_amdgcn_s_setprio(0);
-                running = gjk_distance_step(g, pq, w.a, w.b, prm.max_distance_squared, tol2);
-            }
-            if (!running) {
-                if (sub == 0) gjk_write(g, pq, pid, prm.sanity_check, o);
-                have = false;
-            }
-        }
-    }
-}
-
-// All work classes in one persistent launch: every wavefront walks the classes
-// from the largest hulls to the analytic pairs (size classes 7 .. 0, the pairs
-// of two hulls before those of one at each size), switching its lanes per pair
-// at each class, so classes overlap without a launch per class.
-// lanes_per_pair holds resolved values (1..64, class 0: 1, 2 or 4).
 // Occupancy 3 (<= 168 VGPRs): measured faster than occupancy 2 without the
 // register cap, at the cost of a few spilled registers.
 __global__ __launch_bounds__(kQBlock) __attribute__((amdgpu_waves_per_eu(3))) void gjk_all_kernel(
@@ -786,40 +338,99 @@ __global__ __launch_bounds__(kQBlock) __attribute__((amdgpu_waves_per_eu(3))) vo
     const int32_t *__restrict__ cls_count, int32_t *__restrict__ cls_cursor, d3d_gjk_params prm,
     GjkOut o) {
     __shared__ double pq_lds[24 * kQBlock];
-    double *pq_wave = pq_lds + 24 * kWave * (threadIdx.x / kWave);
-    const int n_waves = (int)gridDim.x * (kQBlock / kWave);
-    int rot = 0;  // wavefronts given a fixed chunk by the classes walked so far
-    for (int step = 0; step < kNumClasses; ++step) {
-        const int cls = (step & 1) ? kSizeClasses - 1 - step / 2 : kNumClasses - 1 - step / 2;
-        const int count = cls_count[cls];
-        if (count == 0) continue;
-        const int begin = cls_begin[cls];
-        int32_t *cur = cls_cursor + cls;
-        const int G = prm.lanes_per_pair[cls];
-        // items per claim: claim_factor * (64 / G), or the class's fair share per
-        // wavefront when that is smaller, so a small batch spreads its pairs
-        // over all wavefronts instead of a few wavefronts holding all of them
-        const int full = prm.claim_factor * (kWave / G);
-        const int fair = (count + n_waves - 1) / n_waves;
-        const int chunk = fair < full ? fair : full;
-        if (cls == 0) {
-            if (G <= 1) run_class<1, false>(s, pa, pb, order, begin, count, cur, prm, o, pq_wave, chunk, rot);
-            else if (G == 2) run_class<2, false>(s, pa, pb, order, begin, count, cur, prm, o, pq_wave, chunk, rot);
-            else run_class<4, false>(s, pa, pb, order, begin, count, cur, prm, o, pq_wave, chunk, rot);
-        } else {
-            switch (G) {
-            case 1: run_class<1, true>(s, pa, pb, order, begin, count, cur, prm, o, pq_wave, chunk, rot); break;
-            case 2: run_class<2, true>(s, pa, pb, order, begin, count, cur, prm, o, pq_wave, chunk, rot); break;
-            case 4: run_class<4, true>(s, pa, pb, order, begin, count, cur, prm, o, pq_wave, chunk, rot); break;
-            case 8: run_class<8, true>(s, pa, pb, order, begin, count, cur, prm, o, pq_wave, chunk, rot); break;
-            case 16: run_class<16, true>(s, pa, pb, order, begin, count, cur, prm, o, pq_wave, chunk, rot); break;
-            case 32: run_class<32, true>(s, pa, pb, order, begin, count, cur, prm, o, pq_wave, chunk, rot); break;
-            default: run_class<64, true>(s, pa, pb, order, begin, count, cur, prm, o, pq_wave, chunk, rot); break;
-            }
-        }
-        const int used = (count + chunk - 1) / chunk;
-        rot = (int)(((int64_t)rot + (used < n_waves ? used : n_waves)) % n_waves);
+    run_all<DistanceMode>(s, pa, pb, order, cls_begin, cls_count, cls_cursor, prm, o, pq_lds);
+}
+
+// ------------------------------------------------------- GJK intersection
+
+// The simplex of the intersection test holds Y alone: its rows go to the P half
+// of the pair's LDS rows.
+struct HitState {
+    v3 d;
+    double prev;
+    int it, state, n;
+};
+
+struct HitOut {
+    uint8_t *hit;
+    int32_t *status;
+};
+
+// gjk_intersection_jolt (_gjk_jolt.py:29-80) and _intersection_loop (:83-135)
+// as a queue Mode.
+struct IntersectMode {
+    using State = HitState;
+    using Out = HitOut;
+    static __device__ __forceinline__ void clear(State &g, const PQ &) {
+        g.d = mk(1.0, 0.0, 0.0);
+        g.prev = kMaxFloat;
+        g.it = 0;
+        g.state = -1;
+        g.n = 0;
     }
+    static __device__ __forceinline__ bool start(State &g, const PQ &pq, int, int,
+                                                 const d3d_gjk_params &, const Out &) {
+        clear(g, pq);
+        return true;
+    }
+    static __device__ __forceinline__ bool more(State &g, const d3d_gjk_params &prm) {
+        if (g.it < prm.max_iterations) return true;
+        g.state = D3D_ITER_CAP;
+        return false;
+    }
+    static __device__ __forceinline__ bool step(State &g, const PQ &pq, v3 p, v3 q,
+                                                const d3d_gjk_params &prm, const Out &) {
+        ++g.it;
+        const v3 w = p - q;
+        g.state = D3D_SEPARATED;
+        if (dot(g.d, w) < -kEps) return false;
+        // rows past n are not read before they are appended
+        Simplex S;
+        S.n = g.n;
+        S.Y0 = pq.P(0);
+        S.Y1 = pq.P(1);
+        S.Y2 = pq.P(2);
+        S.Y3 = w;
+        pq.put_p(S.n < 3 ? S.n : 3, w);
+        simplex_append(S, w);
+        v3 v;
+        double vv;
+        int set;
+        if (!closest_to_origin(S, g.prev, v, vv, set)) return false;
+        if (set == 15 || vv <= prm.tolerance * prm.tolerance || vv <= kEps * max_y_len_sq(S)) {
+            g.state = D3D_INTERSECT;
+            return false;
+        }
+        g.d = -v;
+        if (g.prev - vv <= kEps * g.prev) return false;
+        g.prev = vv;
+        const CompactMap cm = compact_map(S.n, set);
+        pq.compact<3>(cm);
+        g.n = cm.m;
+        return true;
+    }
+    static __device__ __forceinline__ void write(const State &g, const PQ &, int64_t pid,
+                                                 const d3d_gjk_params &, const Out &o) {
+        o.hit[pid] = g.state == D3D_INTERSECT ? 1 : 0;
+        if (o.status) o.status[pid] = g.state;
+    }
+    static __device__ __forceinline__ void bad(int64_t pid, const Out &o) {
+        o.hit[pid] = 0;
+        if (o.status) o.status[pid] = kBadInput;
+    }
+};
+
+// Bound like gjk_all_kernel (latency of the hull sweeps and of the FP64 chains),
+// with about a quarter of its rounds.  262,144 mixed pairs: 401 us with the
+// sort, against 740 us one lane per pair in list order, where a wavefront sweeps
+// the hulls of its lanes one after the other in every round.
+__global__ __launch_bounds__(kQBlock) __attribute__((amdgpu_waves_per_eu(3))) void
+gjk_intersect_all_kernel(d3d_scene s, const int32_t *__restrict__ pa, const int32_t *__restrict__ pb,
+                         const int32_t *__restrict__ order, const int32_t *__restrict__ cls_begin,
+                         const int32_t *__restrict__ cls_count, int32_t *__restrict__ cls_cursor,
+                         d3d_gjk_params prm, HitOut o) {
+    __shared__ double pq_lds[24 * kQBlock];
+    run_all<IntersectMode>(s, pa, pb, order, cls_begin, cls_count, cls_cursor, prm, o, pq_lds);
 }
 
 // ---------------------------------------------------------------- host
@@ -910,15 +521,10 @@ static bool stage_events(std::array<hipEvent_t, 4> &ev) {
     return true;
 }
 
-static int launch_all(const d3d_scene &s, const int32_t *pa, const int32_t *pb, int64_t n,
-                      const d3d_gjk_params &prm, const GjkOut &o, void *ws, hipStream_t stream,
-                      const EpaHook *epa) {
-    const QueueWs w = ws_view(ws, n);
-    const int hdr = (int)ws_header_ints();
-    std::array<hipEvent_t, 4> ev;
-    const bool timed = stage_events(ev);
-    if (timed) D3D_CHECK_HIP(hipEventRecord(ev[0], stream));
-    hipLaunchKernelGGL(queue_clear_kernel, dim3(4), dim3(kQBlock), 0, stream, (int32_t *)ws, hdr);
+int queue_sort(const d3d_scene &s, const int32_t *pa, const int32_t *pb, int64_t n, const QueueWs &w,
+               hipStream_t stream) {
+    hipLaunchKernelGGL(queue_clear_kernel, dim3(4), dim3(kQBlock), 0, stream, w.hist,
+                       (int)ws_header_ints());
     D3D_CHECK_LAUNCH("queue_clear_kernel");
     int64_t g = (n + kQBlock - 1) / kQBlock;
     if (g > 2048) g = 2048;
@@ -931,8 +537,10 @@ static int launch_all(const d3d_scene &s, const int32_t *pa, const int32_t *pb, 
     hipLaunchKernelGGL(queue_scatter_kernel, dim3((unsigned)g), dim3(kQBlock), 0, stream, s, pa, pb,
                        n, w.key_off, w.key_cur, w.order);
     D3D_CHECK_LAUNCH("queue_scatter_kernel");
-    // one persistent launch for every class; lanes and launch shape resolved
-    // on the host
+    return D3D_OK;
+}
+
+d3d_gjk_params queue_params(const d3d_gjk_params &prm) {
     d3d_gjk_params rp = prm;
     for (int c = 0; c < kNumClasses; ++c) {
         int G = prm.lanes_per_pair[c] > 0 ? prm.lanes_per_pair[c] : kDefaultLanes[c];
@@ -942,14 +550,29 @@ static int launch_all(const d3d_scene &s, const int32_t *pa, const int32_t *pb, 
     rp.blocks_per_cu = prm.blocks_per_cu > 0 ? prm.blocks_per_cu : 3;
     rp.claim_factor = prm.claim_factor > 0 ? prm.claim_factor : 2;
     rp.epa_blocks_per_cu = prm.epa_blocks_per_cu > 0 ? prm.epa_blocks_per_cu : 8;
+    return rp;
+}
+
+// resident at occupancy 3 (4 wavefronts per block) by default
+unsigned queue_grid(const d3d_gjk_params &resolved) {
+    return (unsigned)(cu_count() * resolved.blocks_per_cu);
+}
+
+static int launch_all(const d3d_scene &s, const int32_t *pa, const int32_t *pb, int64_t n,
+                      const d3d_gjk_params &prm, const GjkOut &o, void *ws, hipStream_t stream,
+                      const EpaHook *epa) {
+    const QueueWs w = ws_view(ws, n);
+    std::array<hipEvent_t, 4> ev;
+    const bool timed = stage_events(ev);
+    if (timed) D3D_CHECK_HIP(hipEventRecord(ev[0], stream));
+    if (int rc = queue_sort(s, pa, pb, n, w, stream)) return rc;
+    const d3d_gjk_params rp = queue_params(prm);
     if (epa) {
         hipLaunchKernelGGL(zero_u64_kernel, dim3(1), dim3(1), 0, stream, epa->count);
         D3D_CHECK_LAUNCH("zero_u64_kernel");
     }
-    // resident at occupancy 3 (4 wavefronts per block) by default
-    const int64_t grid = (int64_t)cu_count() * rp.blocks_per_cu;
     if (timed) D3D_CHECK_HIP(hipEventRecord(ev[1], stream));
-    hipLaunchKernelGGL(gjk_all_kernel, dim3((unsigned)grid), dim3(kQBlock), 0, stream, s, pa, pb,
+    hipLaunchKernelGGL(gjk_all_kernel, dim3(queue_grid(rp)), dim3(kQBlock), 0, stream, s, pa, pb,
                        w.order, w.cls_begin, w.cls_count, w.cls_cursor, rp, o);
     D3D_CHECK_LAUNCH("gjk_all_kernel");
     if (timed) D3D_CHECK_HIP(hipEventRecord(ev[2], stream));
@@ -1075,13 +698,7 @@ static int gjk_distance_impl(const d3d_scene *scene, const int32_t *pair_a, cons
     if (params) {
         prm = *params;
     } else {
-        prm.tolerance = 1e-10;
-        prm.max_distance_squared = 100000.0;
-        prm.sanity_check = 1e-8;
-        prm.max_iterations = 128;
-        prm.hull_serial_max = 16;
-        for (int c = 0; c < kNumClasses; ++c) prm.lanes_per_pair[c] = 0;
-        prm.blocks_per_cu = prm.claim_factor = prm.epa_blocks_per_cu = 0;
+        prm = default_params();
     }
     D3D_CHECK_ARG(prm.max_iterations > 0, "max_iterations must be > 0");
     D3D_CHECK_ARG(prm.blocks_per_cu >= 0 && prm.blocks_per_cu <= 3, "blocks_per_cu must be in [0, 3]");
@@ -1133,6 +750,41 @@ extern "C" int d3d_gjk_distance_batch_ws(const d3d_scene *scene, const int32_t *
     D3D_CHECK_ARG(workspace != nullptr, "workspace is NULL");
     return gjk_distance_impl(scene, pair_a, pair_b, n, params, dist, cp_a, cp_b, status, iterations,
                              simplex, n_points, workspace, workspace_bytes, nullptr, stream);
+}
+
+// Pairs below which the sort's launches cost more than they save: with hulls in
+// the scene 16 mixed pairs take 33 us in the lane-per-pair kernel and 51 us
+// here, 64 pairs 91 and 51 us, 262,144 pairs 740 and 401 us.  A scene without
+// hulls has nothing to sort for (262,144 pairs of boxes 49 and 75 us).
+constexpr int64_t kIntersectQueueMin = 32;
+
+extern "C" int d3d_gjk_intersection_batch_ws(const d3d_scene *scene, const int32_t *pair_a,
+                                             const int32_t *pair_b, int64_t n, double tolerance,
+                                             int32_t max_iterations, uint8_t *hit, int32_t *status,
+                                             void *workspace, int64_t workspace_bytes,
+                                             void *stream) {
+    clear_error();
+    if (int rc = check_scene(scene)) return rc;
+    D3D_CHECK_ARG(n >= 0, "n must be >= 0");
+    if (n == 0) return D3D_OK;
+    D3D_CHECK_ARG(n < (int64_t)0x7fffffff, "n must fit in int32");
+    D3D_CHECK_ARG(pair_a && pair_b && hit && workspace, "NULL buffer");
+    D3D_CHECK_ARG(max_iterations > 0, "max_iterations must be > 0");
+    D3D_CHECK_ARG(workspace_bytes >= d3d_gjk_workspace_bytes(n), "workspace too small");
+    if (n < kIntersectQueueMin || scene->n_vertices == 0)
+        return d3d_gjk_intersection_batch(scene, pair_a, pair_b, n, tolerance, max_iterations, hit,
+                                          status, stream);
+    d3d_gjk_params prm = default_params();
+    prm.tolerance = tolerance;
+    prm.max_iterations = max_iterations;
+    const d3d_gjk_params rp = queue_params(prm);
+    const QueueWs w = ws_view(workspace, n);
+    if (int rc = queue_sort(*scene, pair_a, pair_b, n, w, (hipStream_t)stream)) return rc;
+    hipLaunchKernelGGL(gjk_intersect_all_kernel, dim3(queue_grid(rp)), dim3(kQBlock), 0,
+                       (hipStream_t)stream, *scene, pair_a, pair_b, w.order, w.cls_begin, w.cls_count,
+                       w.cls_cursor, rp, HitOut{hit, status});
+    D3D_CHECK_LAUNCH("gjk_intersect_all_kernel");
+    return D3D_OK;
 }
 
 // Workspace of the fused pipeline: GJK queue | simplex (n*36 f64) |

@@ -73,6 +73,21 @@ inline int check_scene(const d3d_scene *s) {
     return D3D_OK;
 }
 
+// every parameter's default (what NULL params stand for)
+inline d3d_gjk_params default_params() {
+    d3d_gjk_params p;
+    p.tolerance = 1e-10;
+    p.max_distance_squared = 100000.0;
+    p.sanity_check = 1e-8;
+    p.max_iterations = 128;
+    p.hull_serial_max = 16;
+    for (int c = 0; c < D3D_NUM_CLASSES; ++c) p.lanes_per_pair[c] = 0;
+    p.blocks_per_cu = 0;
+    p.claim_factor = 0;
+    p.epa_blocks_per_cu = 0;
+    return p;
+}
+
 inline unsigned grid_for(int64_t n, int block) { return (unsigned)((n + block - 1) / block); }
 
 // EPA launcher shared by d3d_epa_batch and the fused GJK+EPA pipeline: with

@@ -20,6 +20,15 @@ def _dev_f64(x, device):
                            dtype=torch.float64).to(device).contiguous()
 
 
+def _workspace(n_bytes, device, stream):
+    """A scratch tensor of one call, safe to drop when it runs on ``stream``."""
+    import torch
+    ws = torch.empty(max(int(n_bytes), 1), dtype=torch.uint8, device=device)
+    if stream is not None:
+        ws.record_stream(stream)
+    return ws
+
+
 def support_batch(scene, shape_ids, dirs, stream=None):
     """Support points of ``scene`` colliders ``shape_ids`` along ``dirs``
     (n, 3) -> (n, 3) float64 tensor."""
@@ -124,9 +133,10 @@ def gjk_intersection_batch(scene, pair_a, pair_b, tolerance=1e-10, max_iteration
         raise ValueError("pair_a and pair_b differ in length")
     hit = torch.empty(n, dtype=torch.uint8, device=scene.device)
     status = torch.empty(n, dtype=torch.int32, device=scene.device) if want_status else None
-    check(lib().d3d_gjk_intersection_batch(
+    ws = _workspace(gjk_workspace_bytes(n), scene.device, stream)
+    check(lib().d3d_gjk_intersection_batch_ws(
         scene.c, ptr(a), ptr(b), n, float(tolerance), int(max_iterations), ptr(hit),
-        ptr(status), stream_ptr(stream)), "d3d_gjk_intersection_batch")
+        ptr(status), ptr(ws), ws.numel(), stream_ptr(stream)), "d3d_gjk_intersection_batch_ws")
     return hit, status
 
 
@@ -430,15 +440,13 @@ def _bvh_query_sorted(bvh, q, cap, counter, stream):
     result = torch.empty(3, dtype=torch.int64, device=q.device)
     while True:
         pairs = torch.empty((cap, 2), dtype=torch.int32, device=q.device)
-        ws = torch.empty(int(lib().d3d_bvh_query_sorted_workspace_bytes(m, cap)), dtype=torch.uint8,
-                         device=q.device)
+        ws = _workspace(lib().d3d_bvh_query_sorted_workspace_bytes(m, cap), q.device, stream)
         check(lib().d3d_bvh_query_sorted(ptr(bvh.buffer), bvh.n, ptr(bvh.aabbs), ptr(q), m,
                                          ptr(pairs), cap, ptr(result), ptr(ws), ws.numel(),
                                          stream_ptr(stream)), "d3d_bvh_query_sorted")
         if stream is None:
             k, longest, spilled = result.tolist()
         else:
-            ws.record_stream(stream)
             result.record_stream(stream)
             with torch.cuda.stream(stream):
                 k, longest, spilled = result.tolist()

@@ -249,6 +249,16 @@ int d3d_gjk_intersection_batch(const d3d_scene *scene, const int32_t *pair_a,
                                void *stream);
 
 /*
+ * d3d_gjk_intersection_batch through the sorted pair queue of the distance
+ * pipeline (same results): faster for all but the smallest batches, with a
+ * caller-owned workspace of d3d_gjk_workspace_bytes(n) bytes.
+ */
+int d3d_gjk_intersection_batch_ws(const d3d_scene *scene, const int32_t *pair_a,
+                                  const int32_t *pair_b, int64_t n, double tolerance,
+                                  int32_t max_iterations, uint8_t *hit, int32_t *status,
+                                  void *workspace, int64_t workspace_bytes, void *stream);
+
+/*
  * Batched EPA penetration depth, epa.epa (epa.py:9-78), seeded from the GJK
  * simplices of d3d_gjk_distance_batch (simplex (n,3,4,3) f64 = Y, P, Q rows,
  * n_points (n) int32) of intersecting pairs.  One wavefront per pair, polytope

@@ -4,8 +4,9 @@ against the oracle.  Every compared value is exact (a selection, a comparison
 or the oracle's own operations in its order), so equality is bitwise."""
 import numpy as np
 import pytest
+import torch
 
-from distance3d_amd import kernels
+from distance3d_amd import kernels, workloads
 from distance3d_amd.scene import SceneBuilder
 from oracle import oracle
 from tests import geometry_brute as gb
@@ -94,3 +95,34 @@ def test_box_query_list_lengths(gpu, k):
     queries = np.array([[[0.5, 0.6]] * 3, [[-2.0, -1.0]] * 3])
     got = kernels.bvh_query(kernels.bvh_build(boxes), queries).cpu().numpy()
     assert np.array_equal(got, np.stack([np.zeros(k, int), np.arange(k)], 1))
+
+
+@pytest.mark.parametrize("n", (1, 31, 32, 33, 300, 5000))
+@pytest.mark.parametrize("kind", ("mixed", "near", "analytic"))
+def test_intersection_by_batch_size(gpu, kind, n):
+    """Both intersection kernels at the line between them, over every work
+    class, an invalid pair, a collider against itself and an iteration cap: hits
+    against the oracle, statuses against the lane-per-pair kernel's."""
+    if kind == "analytic":
+        host = workloads.broad_phase_scene(n_boxes=600, n_capsules=100, extent=4.0).scene
+    else:
+        host = workloads.mixed_pairs(seed=5, n_pairs=350).scene
+        if kind == "near":
+            host.shape_f64[:, 9:12] *= 0.4
+    rs = np.random.RandomState(n)
+    a, b = rs.randint(0, host.n_shapes, (2, n)).astype(np.int32)
+    dev = host.to_device()
+    for cap in (128, 2):
+        hit, status = kernels.gjk_intersection_batch(dev, a, b, max_iterations=cap, want_status=True)
+        want = oracle.gjk_intersection(host, a, b, max_iterations=cap)[0]  # -1 at the cap
+        assert np.array_equal(hit.cpu().numpy(), want == 1)
+        assert np.array_equal(status.cpu().numpy() == 4, want == -1)
+        da, db = (torch.as_tensor(x, device="cuda") for x in (a, b))
+        lane_hit, lane_status = torch.empty_like(hit), torch.empty_like(status)
+        kernels.check(kernels.lib().d3d_gjk_intersection_batch(
+            dev.c, kernels.ptr(da), kernels.ptr(db), n, 1e-10, cap, kernels.ptr(lane_hit),
+            kernels.ptr(lane_status), kernels.stream_ptr()), "d3d_gjk_intersection_batch")
+        assert torch.equal(hit, lane_hit) and torch.equal(status, lane_status)
+    a[-1] = host.n_shapes
+    hit, status = kernels.gjk_intersection_batch(dev, a, b, want_status=True)
+    assert int(hit[-1]) == 0 and int(status[-1]) == 0x200
