@@ -112,6 +112,81 @@ __global__ __launch_bounds__(kQBlock) void queue_scatter_kernel(
     }
 }
 
+// the EPA list counter and the EPA claim cursor
+__global__ void zero_u64_kernel(unsigned long long *c) {
+    c[0] = 0ull;
+    c[1] = 0ull;
+}
+
+// The whole sort of a small batch by one block: counts, scan and ranks in LDS,
+// with the class cursors and the optional EPA counters cleared on the way.
+// A whole GJK + EPA call with the four-launch sort and with this one: 1 pair 51
+// and 42 us, 64 mixed pairs 294 and 282 us, 2,048 hull pairs 142 and 135 us,
+// 4,096 mixed pairs 739 and 728 us; from 8,192 pairs on one block's chain of
+// loads is the longer one (hull pairs 176 and 181 us, 16,384 pairs 221 and 240).
+constexpr int kSmallSort = 4096;
+constexpr int kSmallBlock = 1024;
+
+__global__ __launch_bounds__(kSmallBlock) void queue_small_kernel(
+    d3d_scene s, const int32_t *__restrict__ pa, const int32_t *__restrict__ pb, int n, QueueWs w,
+    unsigned long long *__restrict__ epa_count) {
+    __shared__ int32_t h[kNumKeys];
+    __shared__ uint16_t key[kSmallSort], rank[kSmallSort];
+    __shared__ int32_t wsum[kSmallBlock / kWave];
+    const int t = threadIdx.x, lane = t & (kWave - 1), wave = t / kWave;
+    for (int k = t; k < kNumKeys; k += kSmallBlock) h[k] = 0;
+    if (t < kNumClasses) w.cls_cursor[t] = 0;
+    if (epa_count && t < 2) epa_count[t] = 0ull;
+    __syncthreads();
+    // the keys of four pairs at a time, so that their loads go out together
+    for (int b = 0; b < n; b += 4 * kSmallBlock) {
+        int a4[4], b4[4], k4[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int i = b + j * kSmallBlock + t;
+            a4[j] = i < n ? pa[i] : -1;
+            b4[j] = i < n ? pb[i] : -1;
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) k4[j] = pair_key(s, a4[j], b4[j]);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int i = b + j * kSmallBlock + t;
+            if (i < n) {
+                key[i] = (uint16_t)k4[j];
+                rank[i] = (uint16_t)atomicAdd(&h[k4[j]], 1);
+            }
+        }
+    }
+    __syncthreads();
+    // exclusive scan of the counts, two keys per thread
+    static_assert(kNumKeys <= 2 * kSmallBlock && kNumKeys % 2 == 0, "two keys per thread");
+    const bool in = 2 * t < kNumKeys;
+    const int c0 = in ? h[2 * t] : 0, c1 = in ? h[2 * t + 1] : 0;
+    int incl = c0 + c1;
+#pragma unroll
+    for (int off = 1; off < kWave; off <<= 1) {
+        const int v = __shfl_up(incl, off);
+        if (lane >= off) incl += v;
+    }
+    if (lane == kWave - 1) wsum[wave] = incl;
+    __syncthreads();
+    int first = incl - c0 - c1;
+    for (int k = 0; k < wave; ++k) first += wsum[k];
+    if (in) {
+        h[2 * t] = first;
+        h[2 * t + 1] = first + c0;
+    }
+    __syncthreads();
+    if (t < kNumClasses) {
+        constexpr int per = kNumTypes * kNumTypes;
+        const int b = h[t * per], e = t + 1 < kNumClasses ? h[(t + 1) * per] : n;
+        w.cls_begin[t] = b;
+        w.cls_count[t] = e - b;
+    }
+    for (int i = t; i < n; i += kSmallBlock) w.order[h[key[i]] + rank[i]] = i;
+}
+
 // ------------------------------------------------------------- GJK state
 
 struct GjkState {
@@ -490,12 +565,6 @@ struct EpaHook {
     int32_t *status;
 };
 
-// the EPA list counter and the EPA claim cursor
-__global__ void zero_u64_kernel(unsigned long long *c) {
-    c[0] = 0ull;
-    c[1] = 0ull;
-}
-
 // ---------------------------------------------------------- stage timing
 
 // Events of the calls recorded while stage timing is enabled: before the sort,
@@ -522,7 +591,17 @@ static bool stage_events(std::array<hipEvent_t, 4> &ev) {
 }
 
 int queue_sort(const d3d_scene &s, const int32_t *pa, const int32_t *pb, int64_t n, const QueueWs &w,
-               hipStream_t stream) {
+               hipStream_t stream, unsigned long long *epa_count) {
+    if (n <= kSmallSort) {
+        hipLaunchKernelGGL(queue_small_kernel, dim3(1), dim3(kSmallBlock), 0, stream, s, pa, pb, (int)n,
+                           w, epa_count);
+        D3D_CHECK_LAUNCH("queue_small_kernel");
+        return D3D_OK;
+    }
+    if (epa_count) {
+        hipLaunchKernelGGL(zero_u64_kernel, dim3(1), dim3(1), 0, stream, epa_count);
+        D3D_CHECK_LAUNCH("zero_u64_kernel");
+    }
     hipLaunchKernelGGL(queue_clear_kernel, dim3(4), dim3(kQBlock), 0, stream, w.hist,
                        (int)ws_header_ints());
     D3D_CHECK_LAUNCH("queue_clear_kernel");
@@ -565,12 +644,8 @@ static int launch_all(const d3d_scene &s, const int32_t *pa, const int32_t *pb, 
     std::array<hipEvent_t, 4> ev;
     const bool timed = stage_events(ev);
     if (timed) D3D_CHECK_HIP(hipEventRecord(ev[0], stream));
-    if (int rc = queue_sort(s, pa, pb, n, w, stream)) return rc;
+    if (int rc = queue_sort(s, pa, pb, n, w, stream, epa ? epa->count : nullptr)) return rc;
     const d3d_gjk_params rp = queue_params(prm);
-    if (epa) {
-        hipLaunchKernelGGL(zero_u64_kernel, dim3(1), dim3(1), 0, stream, epa->count);
-        D3D_CHECK_LAUNCH("zero_u64_kernel");
-    }
     if (timed) D3D_CHECK_HIP(hipEventRecord(ev[1], stream));
     hipLaunchKernelGGL(gjk_all_kernel, dim3(queue_grid(rp)), dim3(kQBlock), 0, stream, s, pa, pb,
                        w.order, w.cls_begin, w.cls_count, w.cls_cursor, rp, o);
@@ -597,11 +672,13 @@ __global__ __launch_bounds__(kQBlock) void instance_kernel(
     d3d_scene s, const int32_t *__restrict__ a, const int32_t *__restrict__ b,
     const double *__restrict__ pose_a, const double *__restrict__ pose_b,
     const int32_t *__restrict__ pidx_a, const int32_t *__restrict__ pidx_b, int64_t n_poses,
-    int64_t n, double *__restrict__ f64, int32_t *__restrict__ i32) {
+    int64_t n, double *__restrict__ f64, int32_t *__restrict__ i32, int32_t *__restrict__ inst_a,
+    int32_t *__restrict__ inst_b) {
     const int64_t t = (int64_t)blockIdx.x * kQBlock + threadIdx.x;
     if (t >= 2 * n) return;
     const int64_t pair = t >> 1;
     const int side = (int)(t & 1);
+    if (inst_a && inst_b) (side ? inst_b : inst_a)[pair] = (int32_t)t;
     const int k = side ? b[pair] : a[pair];
     const double *pose = side ? pose_b : pose_a;
     const int32_t *pidx = side ? pidx_b : pidx_a;
@@ -626,15 +703,6 @@ __global__ __launch_bounds__(kQBlock) void instance_kernel(
     const int32_t *si = s.shape_i32 + 4 * (int64_t)k;
 #pragma unroll
     for (int j = 0; j < 4; ++j) di[j] = si[j];
-}
-
-__global__ __launch_bounds__(kQBlock) void iota_pairs_kernel(int32_t *__restrict__ a,
-                                                             int32_t *__restrict__ b, int64_t n) {
-    const int64_t i = (int64_t)blockIdx.x * kQBlock + threadIdx.x;
-    if (i < n) {
-        a[i] = (int32_t)(2 * i);
-        b[i] = (int32_t)(2 * i + 1);
-    }
 }
 
 }  // namespace d3d
@@ -779,7 +847,7 @@ extern "C" int d3d_gjk_intersection_batch_ws(const d3d_scene *scene, const int32
     prm.max_iterations = max_iterations;
     const d3d_gjk_params rp = queue_params(prm);
     const QueueWs w = ws_view(workspace, n);
-    if (int rc = queue_sort(*scene, pair_a, pair_b, n, w, (hipStream_t)stream)) return rc;
+    if (int rc = queue_sort(*scene, pair_a, pair_b, n, w, (hipStream_t)stream, nullptr)) return rc;
     hipLaunchKernelGGL(gjk_intersect_all_kernel, dim3(queue_grid(rp)), dim3(kQBlock), 0,
                        (hipStream_t)stream, *scene, pair_a, pair_b, w.order, w.cls_begin, w.cls_count,
                        w.cls_cursor, rp, HitOut{hit, status});
@@ -845,13 +913,8 @@ extern "C" int d3d_instance_pairs(const d3d_scene *scene, const int32_t *pair_a,
     D3D_CHECK_ARG(!(pose_idx_a || pose_idx_b) || n_poses > 0, "pose indices need n_poses > 0");
     hipLaunchKernelGGL(instance_kernel, dim3(grid_for(2 * n, kQBlock)), dim3(kQBlock), 0, st, *scene,
                        pair_a, pair_b, pose_a, pose_b, pose_idx_a, pose_idx_b, n_poses, n, inst_f64,
-                       inst_i32);
+                       inst_i32, inst_a, inst_b);
     D3D_CHECK_LAUNCH("instance_kernel");
-    if (inst_a && inst_b) {
-        hipLaunchKernelGGL(iota_pairs_kernel, dim3(grid_for(n, kQBlock)), dim3(kQBlock), 0, st, inst_a,
-                           inst_b, n);
-        D3D_CHECK_LAUNCH("iota_pairs_kernel");
-    }
     return D3D_OK;
 }
 

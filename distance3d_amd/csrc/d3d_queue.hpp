@@ -546,9 +546,10 @@ __device__ __forceinline__ void run_all(const d3d_scene &s, const int32_t *__res
 }
 
 // Sorts the pairs of a batch into `w` (work class, type of A, type of B) on
-// `stream`: w.order, the class ranges and cleared class cursors.
+// `stream`: w.order, the class ranges and cleared class cursors; epa_count
+// (optional, two counters) is cleared too.
 int queue_sort(const d3d_scene &s, const int32_t *pa, const int32_t *pb, int64_t n, const QueueWs &w,
-               hipStream_t stream);
+               hipStream_t stream, unsigned long long *epa_count = nullptr);
 
 // prm with the lanes per class and the launch shape resolved; the grid of a
 // persistent launch (kQBlock threads per block).

@@ -126,3 +126,23 @@ def test_intersection_by_batch_size(gpu, kind, n):
     a[-1] = host.n_shapes
     hit, status = kernels.gjk_intersection_batch(dev, a, b, want_status=True)
     assert int(hit[-1]) == 0 and int(status[-1]) == 0x200
+
+
+@pytest.mark.parametrize("n", (1, 1023, 1025, 4095, 4096, 4097))
+def test_pair_sort_by_batch_size(gpu, n):
+    """GJK distance and intersection on both sides of the one-block sort, with
+    invalid pairs: every pair is taken exactly once."""
+    host = workloads.mixed_pairs(seed=9, n_pairs=200).scene
+    rs = np.random.RandomState(n)
+    a, b = rs.randint(0, host.n_shapes, (2, n)).astype(np.int32)
+    bad = rs.rand(n) < 0.01
+    a[bad] = host.n_shapes + 3
+    dev = host.to_device()
+    out = kernels.gjk_distance_batch(dev, a, b)
+    hit, _ = kernels.gjk_intersection_batch(dev, a, b)
+    ok = ~bad
+    want = oracle.gjk_distance(host, a[ok], b[ok])
+    assert np.array_equal(out.dist.cpu().numpy()[ok], want["dist"])
+    assert np.array_equal(out.status.cpu().numpy()[bad], np.full(bad.sum(), 0x200))
+    assert np.array_equal(hit.cpu().numpy()[ok], oracle.gjk_intersection(host, a[ok], b[ok])[0])
+    assert not hit.cpu().numpy()[bad].any()
