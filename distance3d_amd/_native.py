@@ -214,9 +214,11 @@ def gjk_params(tolerance=1e-10, max_distance_squared=100000.0, sanity_check=1e-8
     p.sanity_check = float(sanity_check)
     p.max_iterations = int(max_iterations)
     p.hull_serial_max = int(hull_serial_max)
-    lanes = expand_lanes(DEFAULT_LANES if lanes_per_pair is None else lanes_per_pair)
-    for c, g in enumerate(lanes):
-        p.lanes_per_pair[c] = int(g)
+    # without a table of the caller's the entries stay 0: the library's own table
+    # (DEFAULT_LANES), widened where a batch leaves the chip idle
+    if lanes_per_pair is not None:
+        for c, g in enumerate(expand_lanes(lanes_per_pair)):
+            p.lanes_per_pair[c] = int(g)
     launch = launch or {}
     unknown = set(launch) - {"blocks_per_cu", "claim_factor", "epa_blocks_per_cu"}
     if unknown:

@@ -622,7 +622,7 @@ int queue_sort(const d3d_scene &s, const int32_t *pa, const int32_t *pb, int64_t
 d3d_gjk_params queue_params(const d3d_gjk_params &prm) {
     d3d_gjk_params rp = prm;
     for (int c = 0; c < kNumClasses; ++c) {
-        int G = prm.lanes_per_pair[c] > 0 ? prm.lanes_per_pair[c] : kDefaultLanes[c];
+        int G = prm.lanes_per_pair[c] > 0 ? prm.lanes_per_pair[c] : -kDefaultLanes[c];
         if (c == 0 && G > 4) G = 4;
         rp.lanes_per_pair[c] = G;
     }

@@ -500,7 +500,7 @@ __device__ __forceinline__ void run_class(const d3d_scene &s, const int32_t *__r
 // from the largest hulls to the analytic pairs (size classes 7 .. 0, the pairs
 // of two hulls before those of one at each size), switching its lanes per pair
 // at each class, so classes overlap without a launch per class.
-// lanes_per_pair holds resolved values (1..64, class 0: 1, 2 or 4).
+// lanes_per_pair holds resolved values (see queue_params; class 0: 1, 2 or 4).
 template <class M>
 __device__ __forceinline__ void run_all(const d3d_scene &s, const int32_t *__restrict__ pa,
                                         const int32_t *__restrict__ pb,
@@ -511,6 +511,19 @@ __device__ __forceinline__ void run_all(const d3d_scene &s, const int32_t *__res
                                         const typename M::Out &o, double *pq_lds) {
     double *pq_wave = pq_lds + 24 * kWave * (threadIdx.x / kWave);
     const int n_waves = (int)gridDim.x * (kQBlock / kWave);
+    // A batch that leaves wavefronts idle widens the groups of the classes whose
+    // lanes are the table's (negative entries): all by the largest factor that
+    // still gives every pair a group at once.  More lanes shorten a pair's hull
+    // sweeps and its longest chain; once the chip is full they only add FP64 work,
+    // which every lane of a group repeats.  Distance batches with the table's lanes
+    // and widened: 300 mixed pairs 401 and 281 us, 4,096 mixed 477 and 413, 16,384
+    // mixed 691 and 659; overlapping hulls of 64 to 256 vertices, 64 pairs 155 and
+    // 72 us, 2,048 pairs 158 and 82, 8,192 pairs 205 and 190.  Stopping at half the
+    // chip leaves 2,048 of those pairs at 140 us.
+    int64_t lanes = 0;
+    for (int c = 0; c < kNumClasses; ++c) lanes += (int64_t)cls_count[c] * abs(prm.lanes_per_pair[c]);
+    int widen = 1;
+    while (widen < kWave && 2 * widen * lanes <= (int64_t)n_waves * kWave) widen *= 2;
     int rot = 0;  // wavefronts given a fixed chunk by the classes walked so far
     for (int step = 0; step < kNumClasses; ++step) {
         const int cls = (step & 1) ? kSizeClasses - 1 - step / 2 : kNumClasses - 1 - step / 2;
@@ -518,7 +531,15 @@ __device__ __forceinline__ void run_all(const d3d_scene &s, const int32_t *__res
         if (count == 0) continue;
         const int begin = cls_begin[cls];
         int32_t *cur = cls_cursor + cls;
-        const int G = prm.lanes_per_pair[cls];
+        const int table = prm.lanes_per_pair[cls];
+        int G = abs(table);
+        if (table < 0 && cls != 0) {
+            // pairs of at most 128 vertices have no use for the widths between: two
+            // 32-vertex hulls, 4,096 pairs 72 us with 16 lanes and 73 with 32, 2,048
+            // pairs 66 with 16, 67 with 32 and 62 with 64
+            const int wide = min(G * widen, kWave);
+            G = (cls & (kSizeClasses - 1)) <= 2 && wide < kWave ? G : wide;
+        }
         // items per claim: claim_factor * (64 / G), or the class's fair share per
         // wavefront when that is smaller, so a small batch spreads its pairs
         // over all wavefronts instead of a few wavefronts holding all of them
@@ -551,7 +572,8 @@ __device__ __forceinline__ void run_all(const d3d_scene &s, const int32_t *__res
 int queue_sort(const d3d_scene &s, const int32_t *pa, const int32_t *pb, int64_t n, const QueueWs &w,
                hipStream_t stream, unsigned long long *epa_count = nullptr);
 
-// prm with the lanes per class and the launch shape resolved; the grid of a
+// prm with the lanes per class (negative: the table's, which the kernel may
+// widen; positive: the caller's) and the launch shape resolved; the grid of a
 // persistent launch (kQBlock threads per block).
 d3d_gjk_params queue_params(const d3d_gjk_params &prm);
 unsigned queue_grid(const d3d_gjk_params &resolved);
