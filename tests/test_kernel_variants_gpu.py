@@ -146,3 +146,29 @@ def test_pair_sort_by_batch_size(gpu, n):
     assert np.array_equal(out.status.cpu().numpy()[bad], np.full(bad.sum(), 0x200))
     assert np.array_equal(hit.cpu().numpy()[ok], oracle.gjk_intersection(host, a[ok], b[ok])[0])
     assert not hit.cpu().numpy()[bad].any()
+
+
+@pytest.mark.parametrize("m", (1, 63, 64, 65, 200, 131072 + 65))
+def test_tet_pairs_by_batch_size(gpu, m):
+    """Pairs that wait to be clipped: a single tile, several tiles per block, a
+    last partial queue; coinciding tetrahedra and pairs the plane misses among
+    them, with and without planes and polygons."""
+    rs = np.random.RandomState(m)
+    n = 50
+    bodies = []
+    for _ in range(2):
+        T = rs.uniform(-0.6, 0.6, (n, 1, 3)) + 0.5 * rs.randn(n, 4, 3)
+        e = rs.uniform(0.0, 1.0, (n, 4))
+        bodies.append([T, e])
+    bodies[1][0][:10], bodies[1][1][:10] = bodies[0][0][:10], bodies[0][1][:10]
+    X = [oracle.tet_mesh_prep(T)[1] for T, _ in bodies]
+    pairs = rs.randint(0, n, (m, 2)).astype(np.int32)
+    pairs[::7, 1] = pairs[::7, 0]
+    (T1, e1), (T2, e2) = bodies
+    used, inverse = np.unique(pairs, axis=0, return_inverse=True)
+    want = [x[inverse.reshape(-1)] for x in oracle.tet_pairs(T1, e1, X[0], T2, e2, X[1], used)]
+    for geometry in (True, False):
+        got = kernels.tet_pairs_batch(T1, e1, X[0], T2, e2, X[1], pairs, geometry=geometry)
+        for g, w in zip(got, want):
+            if g is not None:
+                assert np.array_equal(g.cpu().numpy(), w, equal_nan=True)
