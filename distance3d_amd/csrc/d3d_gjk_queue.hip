@@ -393,6 +393,7 @@ struct DistanceMode {
         g.state = D3D_ITER_CAP;
         return false;
     }
+    template <int G>
     static __device__ __forceinline__ bool step(State &g, const PQ &pq, v3 p, v3 q,
                                                 const d3d_gjk_params &prm, const Out &) {
         return gjk_distance_step(g, pq, p, q, prm.max_distance_squared,
@@ -453,6 +454,7 @@ struct IntersectMode {
         g.state = D3D_ITER_CAP;
         return false;
     }
+    template <int G>
     static __device__ __forceinline__ bool step(State &g, const PQ &pq, v3 p, v3 q,
                                                 const d3d_gjk_params &prm, const Out &) {
         ++g.it;

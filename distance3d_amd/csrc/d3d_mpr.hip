@@ -9,8 +9,10 @@
 // sweeps large hulls with the whole wavefront).  The portal (4 rows of the
 // Minkowski point and both support points) stays in registers: rows are only
 // addressed with compile-time indices, runtime row choices become selects.
-#include "d3d_device.hpp"
-#include "d3d_runtime.hpp"
+//
+// Batches with hulls go through the sorted pair queue instead (MprMode): the
+// same state machine with the support points of the portal rows in LDS.
+#include "d3d_queue.hpp"
 
 namespace d3d {
 
@@ -312,6 +314,224 @@ __global__ __launch_bounds__(kMprBlock) void mpr_kernel(
     }
 }
 
+// ------------------------------------------------------ the queued machine
+
+// The portal's support points are the pair's LDS rows (a: P, b: Q); its points
+// v are their differences, except v0, which may have been moved off zero.
+struct MprState {
+    v3 d, v0;
+    int phase, it, status, found;
+};
+
+// what the result comes from
+enum : int { kMprNone = 0, kMprTouch = 1, kMprSegment = 2, kMprPortal = 3 };
+
+struct MprOut {
+    const double *centers;
+    double tol;
+    int max_iter, penetration;
+    int32_t *status;
+    double *out;
+};
+
+__device__ __forceinline__ v3 mpr_row(const PQ &pq, int r) { return pq.P(r) - pq.Q(r); }
+
+__device__ __forceinline__ v3 portal_dir(v3 v1, v3 v2, v3 v3_) {
+    return norm_vector(cross(v2 - v1, v3_ - v1));
+}
+
+__device__ __forceinline__ bool portal_reach_tol(v3 v1, v3 v2, v3 v3_, v3 v4, v3 d, double tol) {
+    const double p = dot(v4, d);
+    double m = p - dot(v1, d);
+    const double t2 = p - dot(v2, d);
+    if (t2 < m) m = t2;
+    const double t3 = p - dot(v3_, d);
+    if (t3 < m) m = t3;
+    return m < tol + kEps;
+}
+
+struct MprMode {
+    using State = MprState;
+    using Out = MprOut;
+    static __device__ __forceinline__ void clear(State &g, const PQ &) {
+        g.d = g.v0 = mk(0.0, 0.0, 0.0);
+        g.phase = kMprDone;
+        g.it = g.status = 0;
+        g.found = kMprNone;
+    }
+    // _find_origin_ray (mpr.py:163-177)
+    static __device__ __forceinline__ bool start(State &g, const PQ &pq, int ia, int ib,
+                                                 const d3d_gjk_params &, const Out &o) {
+        const double *ca = o.centers + 3 * (int64_t)ia, *cb = o.centers + 3 * (int64_t)ib;
+        const v3 a = mk(ca[0], ca[1], ca[2]), b = mk(cb[0], cb[1], cb[2]);
+        pq.put(0, a, b);
+        g.v0 = a - b;
+        if (g.v0.x == 0.0 && g.v0.y == 0.0 && g.v0.z == 0.0) g.v0.x += kEps * 10.0;
+        g.d = norm_vector(-g.v0);
+        g.phase = kMprV1;
+        g.it = g.status = 0;
+        g.found = kMprNone;
+        return true;
+    }
+    static __device__ __forceinline__ bool more(State &, const d3d_gjk_params &) { return true; }
+
+    // a refinement round along the portal v1 v2 v3, or what follows the last one
+    static __device__ __forceinline__ bool refine_round(State &g, const Out &o, v3 v1, v3 v2, v3 v3_) {
+        g.d = portal_dir(v1, v2, v3_);
+        if (mpr_encapsulates(v1, g.d)) {
+            g.it = 0;
+            if (o.penetration) {
+                g.phase = kMprPen;
+                return true;
+            }
+            g.status = 1;
+            return false;
+        }
+        if (g.it >= o.max_iter) {
+            // the reference refines without bound; here it gives up
+            g.status = kMprRefineCap;
+            return false;
+        }
+        g.phase = kMprRefine;
+        return true;
+    }
+
+    template <int G>
+    static __device__ __forceinline__ bool step(State &g, const PQ &pq, v3 p, v3 q,
+                                                const d3d_gjk_params &, const Out &o) {
+        const v3 w = p - q;
+        if (g.phase == kMprV1) {
+            pq.put(1, p, q);
+            const bool v1_zero = w.x == 0.0 && w.y == 0.0 && w.z == 0.0;
+            if (!v1_zero && dot(w, g.d) < kEps) return false;  // origin outside
+            g.d = cross(g.v0, w);
+            if (dot(g.d, g.d) < kEps) {
+                g.status = 1;
+                g.found = v1_zero ? kMprTouch : kMprSegment;
+                return false;
+            }
+            g.d = norm_vector(g.d);
+            g.phase = kMprV2;
+            return true;
+        }
+        const v3 r1 = mpr_row(pq, 1);
+        if (g.phase == kMprV2) {
+            if (dot(w, g.d) < kEps) return false;
+            // _search_direction_perpendicular_to_plane_containing_v012 (mpr.py:208-214)
+            g.d = norm_vector(cross(r1 - g.v0, w - g.v0));
+            const bool swap = dot(g.d, g.v0) > 0.0;
+            if (swap) g.d = g.d * -1.0;
+            // rows 1 and 2, exchanged when the direction points away
+            if (swap) pq.move(1, 2);
+            pq.put(swap ? 1 : 2, p, q);
+            g.it = 0;
+            g.phase = kMprV3;
+            return true;
+        }
+        const v3 r2 = mpr_row(pq, 2);
+        v3 v1 = r1, v2 = r2, v3_ = w;
+        if (g.phase == kMprV3) {
+            if (dot(w, g.d) < kEps) return false;
+            // _iterate_discover_portal (mpr.py:217-235): the new row is row 3 and,
+            // where the portal misses the origin ray, takes row 2's or row 1's place
+            pq.put(3, p, q);
+            const bool c2 = dot(cross(v1, w), g.v0) < kEps;
+            const bool c1 = !c2 && dot(cross(w, v2), g.v0) < kEps;
+            if (c1 || c2) {
+                pq.put(c2 ? 2 : 1, p, q);
+                v1 = vsel(c1, w, v1);
+                v2 = vsel(c2, w, v2);
+                g.d = norm_vector(cross(v1 - g.v0, v2 - g.v0));
+            }
+            ++g.it;
+            if ((c1 || c2) && g.it < o.max_iter) return true;
+            g.it = 0;
+            return refine_round(g, o, v1, v2, v3_);
+        }
+        v3_ = mpr_row(pq, 3);
+        const bool reached = portal_reach_tol(v1, v2, v3_, w, g.d, o.tol);
+        if (g.phase == kMprRefine) {
+            if (!mpr_encapsulates(w, g.d) || reached) return false;  // separated
+        } else if (reached || g.it > o.max_iter) {
+            g.status = 1;
+            g.found = kMprPortal;
+            return false;
+        }
+        // _expand_portal (mpr.py:314-329)
+        const v3 x = cross(w, g.v0);
+        const int r = dot(v1, x) > 0.0 ? (dot(v2, x) > 0.0 ? 1 : 3) : (dot(v3_, x) > 0.0 ? 2 : 1);
+        pq.put(r, p, q);
+        v1 = vsel(r == 1, w, v1);
+        v2 = vsel(r == 2, w, v2);
+        v3_ = vsel(r == 3, w, v3_);
+        ++g.it;
+        if (g.phase == kMprRefine) return refine_round(g, o, v1, v2, v3_);
+        g.d = portal_dir(v1, v2, v3_);
+        return true;
+    }
+
+    static __device__ __forceinline__ void write(const State &g, const PQ &pq, int64_t pid,
+                                                 const d3d_gjk_params &, const Out &o) {
+        o.status[pid] = g.status;
+        if (!o.out) return;
+        double *r = o.out + 7 * pid;
+        if (g.found == kMprNone) {
+#pragma unroll
+            for (int k = 0; k < 7; ++k) r[k] = NAN;
+            return;
+        }
+        double depth = 0.0;
+        v3 dir = mk(0.0, 0.0, 0.0), pos;
+        if (g.found == kMprPortal) {
+            // _penetration_info (mpr.py:349-358)
+            MprPortal P;
+            P.v[0] = g.v0;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                P.a[k] = pq.P(k);
+                P.b[k] = pq.Q(k);
+                if (k > 0) P.v[k] = P.a[k] - P.b[k];
+            }
+            v3 cp;
+            depth = origin_to_triangle(P.v[1], P.v[2], P.v[3], cp);
+            dir = norm_vector(vsel(fabs(depth) < kEps, mk(0.0, 0.0, 0.0), cp));
+            pos = mpr_contact(P, mpr_portal_dir(P));
+        } else {
+            pos = (pq.P(1) + pq.Q(1)) * 0.5;
+            if (g.found == kMprSegment) {
+                // _find_penetration_segment (mpr.py:370-378)
+                const v3 v1 = mpr_row(pq, 1);
+                dir = norm_vector(v1);
+                depth = vnorm(v1);
+            }
+        }
+        r[0] = depth;
+        r[1] = dir.x; r[2] = dir.y; r[3] = dir.z;
+        r[4] = pos.x; r[5] = pos.y; r[6] = pos.z;
+    }
+    static __device__ __forceinline__ void bad(int64_t pid, const Out &o) {
+        o.status[pid] = kMprBadInput;
+        if (!o.out) return;
+#pragma unroll
+        for (int k = 0; k < 7; ++k) o.out[7 * pid + k] = NAN;
+    }
+};
+
+// Bound like the other queue kernels: latency of the hull sweeps and of the FP64
+// chains.  Occupancy 2 keeps the portal machine free of spills: 262,144 mixed
+// pairs 672 us, 734 us at occupancy 3 with 196 spilled VGPRs, and 1,068 us one
+// lane per pair in list order (mpr_kernel); 262,144 pairs of 32-vertex hulls 497,
+// 515 and 1,077 us.
+constexpr int kMprBlocksPerCu = 2;
+__global__ __launch_bounds__(kQBlock) __attribute__((amdgpu_waves_per_eu(2))) void mpr_all_kernel(
+    d3d_scene s, const int32_t *__restrict__ pa, const int32_t *__restrict__ pb,
+    const int32_t *__restrict__ order, const int32_t *__restrict__ cls_begin,
+    const int32_t *__restrict__ cls_count, int32_t *__restrict__ cls_cursor, d3d_gjk_params prm,
+    MprOut o) {
+    __shared__ double pq_lds[24 * kQBlock];
+    run_all<MprMode>(s, pa, pb, order, cls_begin, cls_count, cls_cursor, prm, o, pq_lds);
+}
+
 }  // namespace d3d
 
 using namespace d3d;
@@ -331,5 +551,39 @@ extern "C" int d3d_mpr_batch(const d3d_scene *scene, const int32_t *pair_a, cons
                        (hipStream_t)stream, *scene, pair_a, pair_b, centers, n, tolerance,
                        max_iterations, penetration, kMprSerialMax, status, out);
     D3D_CHECK_LAUNCH("mpr_kernel");
+    return D3D_OK;
+}
+
+// Pairs below which the sort costs more than it saves: lane per pair and queue
+// take 13.7 and 19.0 us for 8 mixed pairs, 19.7 and 21.1 for 16, 35.8 and 23.7
+// for 32.  A scene without hulls has nothing to sort for (262,144 pairs of boxes
+// 56 and 77 us).
+constexpr int64_t kMprQueueMin = 32;
+
+extern "C" int d3d_mpr_batch_ws(const d3d_scene *scene, const int32_t *pair_a, const int32_t *pair_b,
+                                const double *centers, int64_t n, double tolerance,
+                                int32_t max_iterations, int32_t penetration, int32_t *status,
+                                double *out, void *workspace, int64_t workspace_bytes,
+                                void *stream) {
+    clear_error();
+    if (int rc = check_scene(scene)) return rc;
+    D3D_CHECK_ARG(n >= 0, "n must be >= 0");
+    if (n == 0) return D3D_OK;
+    D3D_CHECK_ARG(pair_a && pair_b && centers && status && workspace, "NULL buffer");
+    D3D_CHECK_ARG(penetration == 0 || out, "out is NULL but penetration was requested");
+    D3D_CHECK_ARG(max_iterations > 0, "max_iterations must be > 0");
+    D3D_CHECK_ARG(workspace_bytes >= d3d_gjk_workspace_bytes(n), "workspace too small");
+    if (n < kMprQueueMin || n >= (int64_t)0x7fffffff || scene->n_vertices == 0)
+        return d3d_mpr_batch(scene, pair_a, pair_b, centers, n, tolerance, max_iterations, penetration,
+                             status, out, stream);
+    d3d_gjk_params prm = default_params();
+    prm.blocks_per_cu = kMprBlocksPerCu;
+    const d3d_gjk_params rp = queue_params(prm);
+    const QueueWs w = ws_view(workspace, n);
+    if (int rc = queue_sort(*scene, pair_a, pair_b, n, w, (hipStream_t)stream)) return rc;
+    hipLaunchKernelGGL(mpr_all_kernel, dim3(queue_grid(rp)), dim3(kQBlock), 0, (hipStream_t)stream,
+                       *scene, pair_a, pair_b, w.order, w.cls_begin, w.cls_count, w.cls_cursor, rp,
+                       MprOut{centers, tolerance, max_iterations, penetration, status, out});
+    D3D_CHECK_LAUNCH("mpr_all_kernel");
     return D3D_OK;
 }

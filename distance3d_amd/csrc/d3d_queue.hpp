@@ -6,7 +6,7 @@
 //   start(...)      a new pair (its collider indices are validated); false when
 //                   it needs no round
 //   more(...)       false ends the pair before the next support (round cap)
-//   step(...)       one round with the supports on A along d and on B along -d;
+//   step<G>(...)    one round with the supports on A along d and on B along -d;
 //                   false once the pair has terminated
 //   write / bad     the pair's outputs, by one lane; those of an invalid pair
 // A pair's rows of support points live in LDS (PQ).
@@ -486,7 +486,7 @@ __device__ __forceinline__ void run_class(const d3d_scene &s, const int32_t *__r
                     w = support_pair<G, kHull>(s, ia, ib, g.d, sub);
                 }
                 __builtin_amdgcn_s_setprio(0);
-                running = M::step(g, pq, w.a, w.b, prm, o);
+                running = M::template step<G>(g, pq, w.a, w.b, prm, o);
             }
             if (!running) {
                 if (sub == 0) M::write(g, pq, pid, prm, o);

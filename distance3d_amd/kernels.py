@@ -159,9 +159,11 @@ def mpr_batch(scene, pair_a, pair_b, centers, tolerance=0.0001, max_iterations=1
                          % (scene.n_shapes, c.shape[0]))
     status = torch.empty(n, dtype=torch.int32, device=scene.device)
     out = torch.empty((n, 7), dtype=torch.float64, device=scene.device) if penetration else None
-    check(lib().d3d_mpr_batch(scene.c, ptr(a), ptr(b), ptr(c), n, float(tolerance),
-                              int(max_iterations), 1 if penetration else 0, ptr(status), ptr(out),
-                              stream_ptr(stream)), "d3d_mpr_batch")
+    ws = _workspace(gjk_workspace_bytes(n), scene.device, stream)
+    check(lib().d3d_mpr_batch_ws(scene.c, ptr(a), ptr(b), ptr(c), n, float(tolerance),
+                                 int(max_iterations), 1 if penetration else 0, ptr(status),
+                                 ptr(out), ptr(ws), ws.numel(), stream_ptr(stream)),
+          "d3d_mpr_batch_ws")
     return status, out
 
 

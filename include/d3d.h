@@ -356,6 +356,16 @@ int d3d_mpr_batch(const d3d_scene *scene, const int32_t *pair_a, const int32_t *
                   int32_t penetration, int32_t *status, double *out, void *stream);
 
 /*
+ * d3d_mpr_batch through the sorted pair queue of the GJK distance pipeline
+ * (same results): faster for all but the smallest batches, with a caller-owned
+ * workspace of d3d_gjk_workspace_bytes(n) bytes.
+ */
+int d3d_mpr_batch_ws(const d3d_scene *scene, const int32_t *pair_a, const int32_t *pair_b,
+                     const double *centers, int64_t n, double tolerance, int32_t max_iterations,
+                     int32_t penetration, int32_t *status, double *out, void *workspace,
+                     int64_t workspace_bytes, void *stream);
+
+/*
  * Hydroelastic contact of m tetrahedron pairs (hydroelastic_contact/
  * _tetrahedron_intersection.py:7-85 intersect_tetrahedron_pairs, 89-139
  * intersect_tetrahedron_pair and the contact plane / polygon routines it

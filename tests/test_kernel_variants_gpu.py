@@ -7,7 +7,7 @@ import pytest
 import torch
 
 from distance3d_amd import kernels, workloads
-from distance3d_amd.scene import SceneBuilder
+from distance3d_amd.scene import SceneBuilder, collider_centers
 from oracle import oracle
 from tests import geometry_brute as gb
 
@@ -172,3 +172,28 @@ def test_tet_pairs_by_batch_size(gpu, m):
         for g, w in zip(got, want):
             if g is not None:
                 assert np.array_equal(g.cpu().numpy(), w, equal_nan=True)
+
+
+@pytest.mark.parametrize("n", (1, 31, 32, 33, 300, 5000))
+@pytest.mark.parametrize("kind", ("mixed", "near", "same"))
+def test_mpr_by_batch_size(gpu, kind, n):
+    """Both MPR kernels at the line between them, over every work class, with
+    coinciding centres, a refinement cap and an invalid pair, with and without
+    penetration."""
+    host = workloads.mixed_pairs(seed=6, n_pairs=350).scene
+    host.shape_f64[:, 9:12] *= {"mixed": 1.0, "near": 0.4, "same": 0.0}[kind]
+    rs = np.random.RandomState(n)
+    a, b = rs.randint(0, host.n_shapes, (2, n)).astype(np.int32)
+    centers = collider_centers(host)
+    dev = host.to_device()
+    for cap in (100, 1):
+        want = oracle.mpr(host, a, b, centers, max_iterations=cap)
+        got = kernels.mpr_batch(dev, a, b, centers, max_iterations=cap)
+        for g, w in zip(got, want):
+            assert np.array_equal(g.cpu().numpy(), w, equal_nan=True)
+        status, out = kernels.mpr_batch(dev, a, b, centers, max_iterations=cap, penetration=False)
+        want = oracle.mpr(host, a, b, centers, max_iterations=cap, penetration=False)
+        assert out is None and np.array_equal(status.cpu().numpy(), want[0])
+    a[-1] = host.n_shapes
+    status, out = kernels.mpr_batch(dev, a, b, centers)
+    assert int(status[-1]) == 0x200 and bool(torch.isnan(out[-1]).all())
