@@ -406,9 +406,23 @@ struct DistanceMode {
     static __device__ __forceinline__ void bad(int64_t pid, const Out &o) { gjk_write_bad(pid, o); }
 };
 
-// Occupancy 3 (<= 168 VGPRs): measured faster than occupancy 2 without the
-// register cap, at the cost of a few spilled registers.
+// Occupancy 3 (<= 168 VGPRs, a hundred of them spilled) hides more latency when
+// the chip is full; occupancy 2 spills nothing and is the faster one for a batch
+// that does not fill it.  3 and 2: 64 mixed pairs 242 and 127 us, 1,024 mixed 279
+// and 248, 4,096 mixed 418 and 424, 8,192 mixed 474 and 515, 1,048,576 mixed 5,318
+// and 5,778; pairs of 32-vertex hulls, 64 41 and 36 us, 4,096 71 and 65.
+constexpr int64_t kLooseMax = 4096;
+
 __global__ __launch_bounds__(kQBlock) __attribute__((amdgpu_waves_per_eu(3))) void gjk_all_kernel(
+    d3d_scene s, const int32_t *__restrict__ pa, const int32_t *__restrict__ pb,
+    const int32_t *__restrict__ order, const int32_t *__restrict__ cls_begin,
+    const int32_t *__restrict__ cls_count, int32_t *__restrict__ cls_cursor, d3d_gjk_params prm,
+    GjkOut o) {
+    __shared__ double pq_lds[24 * kQBlock];
+    run_all<DistanceMode>(s, pa, pb, order, cls_begin, cls_count, cls_cursor, prm, o, pq_lds);
+}
+
+__global__ __launch_bounds__(kQBlock) __attribute__((amdgpu_waves_per_eu(2))) void gjk_small_kernel(
     d3d_scene s, const int32_t *__restrict__ pa, const int32_t *__restrict__ pb,
     const int32_t *__restrict__ order, const int32_t *__restrict__ cls_begin,
     const int32_t *__restrict__ cls_count, int32_t *__restrict__ cls_cursor, d3d_gjk_params prm,
@@ -500,12 +514,26 @@ struct IntersectMode {
 // Bound like gjk_all_kernel (latency of the hull sweeps and of the FP64 chains),
 // with about a quarter of its rounds.  262,144 mixed pairs: 401 us with the
 // sort, against 740 us one lane per pair in list order, where a wavefront sweeps
-// the hulls of its lanes one after the other in every round.
-__global__ __launch_bounds__(kQBlock) __attribute__((amdgpu_waves_per_eu(3))) void
-gjk_intersect_all_kernel(d3d_scene s, const int32_t *__restrict__ pa, const int32_t *__restrict__ pb,
-                         const int32_t *__restrict__ order, const int32_t *__restrict__ cls_begin,
-                         const int32_t *__restrict__ cls_count, int32_t *__restrict__ cls_cursor,
-                         d3d_gjk_params prm, HitOut o) {
+// the hulls of its lanes one after the other in every round.  Occupancy 3 and 2
+// as for the distance, with a later line since the rounds are few: 1,024 mixed
+// pairs 71 and 56 us, 16,384 near ones 181 and 175, 65,536 302 and 302, 262,144
+// 557 and 593.
+constexpr int64_t kIntersectLooseMax = 65536;
+
+__global__ __launch_bounds__(kQBlock) __attribute__((amdgpu_waves_per_eu(3))) void gjk_intersect_all_kernel(
+    d3d_scene s, const int32_t *__restrict__ pa, const int32_t *__restrict__ pb,
+    const int32_t *__restrict__ order, const int32_t *__restrict__ cls_begin,
+    const int32_t *__restrict__ cls_count, int32_t *__restrict__ cls_cursor, d3d_gjk_params prm,
+    HitOut o) {
+    __shared__ double pq_lds[24 * kQBlock];
+    run_all<IntersectMode>(s, pa, pb, order, cls_begin, cls_count, cls_cursor, prm, o, pq_lds);
+}
+
+__global__ __launch_bounds__(kQBlock) __attribute__((amdgpu_waves_per_eu(2))) void gjk_intersect_small_kernel(
+    d3d_scene s, const int32_t *__restrict__ pa, const int32_t *__restrict__ pb,
+    const int32_t *__restrict__ order, const int32_t *__restrict__ cls_begin,
+    const int32_t *__restrict__ cls_count, int32_t *__restrict__ cls_cursor, d3d_gjk_params prm,
+    HitOut o) {
     __shared__ double pq_lds[24 * kQBlock];
     run_all<IntersectMode>(s, pa, pb, order, cls_begin, cls_count, cls_cursor, prm, o, pq_lds);
 }
@@ -647,10 +675,12 @@ static int launch_all(const d3d_scene &s, const int32_t *pa, const int32_t *pb, 
     const bool timed = stage_events(ev);
     if (timed) D3D_CHECK_HIP(hipEventRecord(ev[0], stream));
     if (int rc = queue_sort(s, pa, pb, n, w, stream, epa ? epa->count : nullptr)) return rc;
-    const d3d_gjk_params rp = queue_params(prm);
+    d3d_gjk_params rp = queue_params(prm);
     if (timed) D3D_CHECK_HIP(hipEventRecord(ev[1], stream));
-    hipLaunchKernelGGL(gjk_all_kernel, dim3(queue_grid(rp)), dim3(kQBlock), 0, stream, s, pa, pb,
-                       w.order, w.cls_begin, w.cls_count, w.cls_cursor, rp, o);
+    const bool loose = n <= kLooseMax;
+    if (loose && rp.blocks_per_cu > 2) rp.blocks_per_cu = 2;  // as many as are resident
+    hipLaunchKernelGGL(loose ? gjk_small_kernel : gjk_all_kernel, dim3(queue_grid(rp)), dim3(kQBlock), 0,
+                       stream, s, pa, pb, w.order, w.cls_begin, w.cls_count, w.cls_cursor, rp, o);
     D3D_CHECK_LAUNCH("gjk_all_kernel");
     if (timed) D3D_CHECK_HIP(hipEventRecord(ev[2], stream));
     if (epa) {
@@ -822,11 +852,12 @@ extern "C" int d3d_gjk_distance_batch_ws(const d3d_scene *scene, const int32_t *
                              simplex, n_points, workspace, workspace_bytes, nullptr, stream);
 }
 
-// Pairs below which the sort's launches cost more than they save: with hulls in
-// the scene 16 mixed pairs take 33 us in the lane-per-pair kernel and 51 us
-// here, 64 pairs 91 and 51 us, 262,144 pairs 740 and 401 us.  A scene without
-// hulls has nothing to sort for (262,144 pairs of boxes 49 and 75 us).
-constexpr int64_t kIntersectQueueMin = 32;
+// Pairs below which the sort costs more than it saves: with hulls in the scene 1
+// mixed pair takes 9 us in the lane-per-pair kernel and 14 us here, 16 pairs 33
+// and at most the 25 us that 64 pairs take here (90 us there), 262,144 pairs 747
+// and 409 us.  A scene without hulls has nothing to sort for (262,144 pairs of
+// boxes 49 and 75 us).
+constexpr int64_t kIntersectQueueMin = 16;
 
 extern "C" int d3d_gjk_intersection_batch_ws(const d3d_scene *scene, const int32_t *pair_a,
                                              const int32_t *pair_b, int64_t n, double tolerance,
@@ -847,11 +878,13 @@ extern "C" int d3d_gjk_intersection_batch_ws(const d3d_scene *scene, const int32
     d3d_gjk_params prm = default_params();
     prm.tolerance = tolerance;
     prm.max_iterations = max_iterations;
+    const bool loose = n <= kIntersectLooseMax;
+    prm.blocks_per_cu = loose ? 2 : 3;
     const d3d_gjk_params rp = queue_params(prm);
     const QueueWs w = ws_view(workspace, n);
     if (int rc = queue_sort(*scene, pair_a, pair_b, n, w, (hipStream_t)stream, nullptr)) return rc;
-    hipLaunchKernelGGL(gjk_intersect_all_kernel, dim3(queue_grid(rp)), dim3(kQBlock), 0,
-                       (hipStream_t)stream, *scene, pair_a, pair_b, w.order, w.cls_begin, w.cls_count,
+    hipLaunchKernelGGL(loose ? gjk_intersect_small_kernel : gjk_intersect_all_kernel,
+                       dim3(queue_grid(rp)), dim3(kQBlock), 0, (hipStream_t)stream, *scene, pair_a, pair_b, w.order, w.cls_begin, w.cls_count,
                        w.cls_cursor, rp, HitOut{hit, status});
     D3D_CHECK_LAUNCH("gjk_intersect_all_kernel");
     return D3D_OK;

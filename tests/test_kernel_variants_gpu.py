@@ -97,7 +97,7 @@ def test_box_query_list_lengths(gpu, k):
     assert np.array_equal(got, np.stack([np.zeros(k, int), np.arange(k)], 1))
 
 
-@pytest.mark.parametrize("n", (1, 31, 32, 33, 300, 5000))
+@pytest.mark.parametrize("n", (1, 15, 16, 17, 300, 5000))
 @pytest.mark.parametrize("kind", ("mixed", "near", "analytic"))
 def test_intersection_by_batch_size(gpu, kind, n):
     """Both intersection kernels at the line between them, over every work
@@ -197,3 +197,13 @@ def test_mpr_by_batch_size(gpu, kind, n):
     a[-1] = host.n_shapes
     status, out = kernels.mpr_batch(dev, a, b, centers)
     assert int(status[-1]) == 0x200 and bool(torch.isnan(out[-1]).all())
+
+
+@pytest.mark.parametrize("n", (65535, 65536, 65537))
+def test_intersection_large_batches(gpu, n):
+    """The intersection's two occupancies at the line between them."""
+    host = workloads.mixed_pairs(seed=11, n_pairs=100).scene
+    rs = np.random.RandomState(n)
+    a, b = rs.randint(0, host.n_shapes, (2, n)).astype(np.int32)
+    hit, _ = kernels.gjk_intersection_batch(host.to_device(), a, b)
+    assert np.array_equal(hit.cpu().numpy(), oracle.gjk_intersection(host, a, b)[0])
