@@ -96,6 +96,7 @@ _SIGNATURES = {
     "d3d_bvh_query_sorted_finish": [_I64, _P, _I64, _P, _P, _I64, _P],
     "d3d_bvh_refit": [_P, _I64, _P, _I64, _P],
     "d3d_overlap_dense": [_P, _I64, _P, _I64, _P, _I64, _P, _P, _I64, _P],
+    "d3d_overlap_dense_write": [_P, _I64, _P, _I64, _P, _I64, _P, _P, _I64, _P],
     "d3d_mpr_batch": [_P, _P, _P, _P, _I64, _D, _I32, _I32, _P, _P, _P],
     "d3d_mpr_batch_ws": [_P, _P, _P, _P, _I64, _D, _I32, _I32, _P, _P, _P, _I64, _P],
     "d3d_tet_pairs_batch": [_P, _P, _P, _P, _P, _P, _P, _I64, _D, _D, _P, _P, _P, _P, _P, _I64,

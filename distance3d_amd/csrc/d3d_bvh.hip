@@ -734,11 +734,18 @@ __device__ __forceinline__ bool box_overlap(const double (&q)[6], const double *
 template <bool kWrite>
 __global__ __launch_bounds__(kDenseBlock) void dense_overlap_kernel(
     const double *__restrict__ a, int64_t n, const double *__restrict__ b, int64_t m,
-    unsigned long long *__restrict__ counts, int32_t *__restrict__ pairs, int64_t cap) {
+    unsigned long long *__restrict__ counts, const unsigned long long *__restrict__ total,
+    int32_t *__restrict__ pairs, int64_t cap) {
     const int lane = lane_id();
     const int64_t wave = ((int64_t)blockIdx.x * kDenseBlock + threadIdx.x) / kWave;
     const int64_t row0 = wave * kDenseRows;
     if (row0 >= n) return;
+    if (kWrite) {
+        // nothing to write: no hits in these rows, or their place is past the room
+        const unsigned long long first = counts[row0];
+        const unsigned long long end = row0 + kDenseRows < n ? counts[row0 + kDenseRows] : *total;
+        if (first == end || first >= (unsigned long long)cap) return;
+    }
     double q[kDenseRows][6];
     unsigned long long off[kDenseRows];
 #pragma unroll
@@ -1015,15 +1022,30 @@ extern "C" int d3d_overlap_dense(const double *a, int64_t n, const double *b, in
     const int64_t waves = (n + kDenseRows - 1) / kDenseRows;
     const unsigned blocks = (unsigned)((waves * kWave + kDenseBlock - 1) / kDenseBlock);
     hipLaunchKernelGGL(dense_overlap_kernel<false>, dim3(blocks), dim3(kDenseBlock), 0, st, a, n, b,
-                       m, counts, pairs, cap);
+                       m, counts, nullptr, pairs, cap);
     D3D_CHECK_LAUNCH("dense_overlap_kernel<count>");
     hipLaunchKernelGGL(dense_scan_kernel, dim3(1), dim3(1024), 0, st, counts, n,
                        (unsigned long long *)n_pairs);
     D3D_CHECK_LAUNCH("dense_scan_kernel");
-    if (cap > 0) {
-        hipLaunchKernelGGL(dense_overlap_kernel<true>, dim3(blocks), dim3(kDenseBlock), 0, st, a, n,
-                           b, m, counts, pairs, cap);
-        D3D_CHECK_LAUNCH("dense_overlap_kernel<write>");
-    }
+    if (cap > 0)
+        return d3d_overlap_dense_write(a, n, b, m, pairs, cap, n_pairs, workspace, workspace_bytes,
+                                       stream);
+    return D3D_OK;
+}
+
+extern "C" int d3d_overlap_dense_write(const double *a, int64_t n, const double *b, int64_t m,
+                                       int32_t *pairs, int64_t cap, const uint64_t *n_pairs,
+                                       void *workspace, int64_t workspace_bytes, void *stream) {
+    clear_error();
+    D3D_CHECK_ARG(n >= 1 && n < (int64_t)0x7fffffff && m >= 1 && m < (int64_t)0x7fffffff,
+                  "n and m must be in [1, 2^31)");
+    D3D_CHECK_ARG(a && b && n_pairs && workspace && cap >= 1 && pairs, "NULL buffer");
+    D3D_CHECK_ARG(workspace_bytes >= d3d_overlap_dense_workspace_bytes(n), "workspace too small");
+    const int64_t waves = (n + kDenseRows - 1) / kDenseRows;
+    const unsigned blocks = (unsigned)((waves * kWave + kDenseBlock - 1) / kDenseBlock);
+    hipLaunchKernelGGL(dense_overlap_kernel<true>, dim3(blocks), dim3(kDenseBlock), 0,
+                       (hipStream_t)stream, a, n, b, m, (unsigned long long *)workspace,
+                       (const unsigned long long *)n_pairs, pairs, cap);
+    D3D_CHECK_LAUNCH("dense_overlap_kernel<write>");
     return D3D_OK;
 }

@@ -372,7 +372,7 @@ def overlap_dense(a, b, cap=None, counter=None, stream=None):
     """All (i, j) with closed-interval overlap of a[i] and b[j], by testing
     every pair (d3d_overlap_dense), row-major (i, then j ascending), as an
     (k, 2) int32 device tensor.  Reads the pair count back (one host
-    synchronisation); a second pass runs when ``cap`` was too small."""
+    synchronisation); the writing pass runs again when ``cap`` was too small."""
     import torch
     a = _dev64(a, (-1, 3, 2))
     b = _dev64(b, (-1, 3, 2)).to(a.device)
@@ -383,14 +383,16 @@ def overlap_dense(a, b, cap=None, counter=None, stream=None):
                      dtype=torch.uint8, device=a.device)
     if cap is None:
         cap = 4 * n + 1024
-    while True:
-        pairs = torch.empty((max(cap, 1), 2), dtype=torch.int32, device=a.device)
-        check(lib().d3d_overlap_dense(ptr(a), n, ptr(b), m, ptr(pairs), cap, ptr(counter), ptr(ws),
-                                      ws.numel(), stream_ptr(stream)), "d3d_overlap_dense")
-        k = int(counter.item())
-        if k <= cap:
-            return pairs[:k]
-        cap = k
+    pairs = torch.empty((max(cap, 1), 2), dtype=torch.int32, device=a.device)
+    check(lib().d3d_overlap_dense(ptr(a), n, ptr(b), m, ptr(pairs), cap, ptr(counter), ptr(ws),
+                                  ws.numel(), stream_ptr(stream)), "d3d_overlap_dense")
+    k = int(counter.item())
+    if k > cap:
+        pairs = torch.empty((k, 2), dtype=torch.int32, device=a.device)
+        check(lib().d3d_overlap_dense_write(ptr(a), n, ptr(b), m, ptr(pairs), k, ptr(counter),
+                                            ptr(ws), ws.numel(), stream_ptr(stream)),
+              "d3d_overlap_dense_write")
+    return pairs[:k]
 
 
 def bvh_query(bvh, queries, cap=None, counter=None, stream=None, sort=True):

@@ -493,6 +493,15 @@ int d3d_overlap_dense(const double *a, int64_t n, const double *b, int64_t m, in
                       void *stream);
 
 /*
+ * The pairs again with more room: after d3d_overlap_dense on the same boxes,
+ * whose count and workspace it takes as that call left them, writes the first
+ * cap pairs without testing for the counts anew.  n, m and cap must be >= 1.
+ */
+int d3d_overlap_dense_write(const double *a, int64_t n, const double *b, int64_t m, int32_t *pairs,
+                            int64_t cap, const uint64_t *n_pairs, void *workspace,
+                            int64_t workspace_bytes, void *stream);
+
+/*
  * d3d_bvh_refit(aabbs (n,3,2) f64, n, bvh, bytes, stream): new boxes for the
  * leaves of a BVH that d3d_bvh_build built over n boxes (box i keeps leaf
  * slot i), keeping its topology: the node boxes are recomputed bottom-up and
