@@ -67,13 +67,15 @@ def _check(status):
         raise AssertionError("more half-plane intersection points than the reference reserves")
 
 
-def _intersecting(T1, e1, X1, T2, e2, X2, pairs, E1, E2, forces, checked=True):
+def _intersecting(T1, e1, X1, T2, e2, X2, pairs, E1, E2, forces, checked=True, polygons=True):
     """The intersecting pairs of a pair list, in list order, on the GPU: a
     status-only pass over all pairs, the hit (and overflow) rows compacted on
     the device, then planes, polygons (and forces) for the hits only.
     Returns host arrays (hit pairs (k,2), planes (k,4), n_vertices (k,),
     polygons (k,24,3), forces (k,7) or None).  ``checked=False``: the pairs
-    are known to be in range (produced by this library's broad phase)."""
+    are known to be in range (produced by this library's broad phase).
+    ``polygons=False``: the forces alone, the rest of the tuple None (the
+    polygons of a fine contact are megabytes)."""
     import torch
     pr = torch.as_tensor(pairs)
     pr = (pr if pr.is_cuda else pr.cuda()).to(torch.int32).reshape(-1, 2).contiguous()
@@ -84,12 +86,16 @@ def _intersecting(T1, e1, X1, T2, e2, X2, pairs, E1, E2, forces, checked=True):
     _check(sel.cpu().numpy())
     hp = pr[rows[(sel & 1) != 0]]
     if hp.shape[0] == 0:
+        if not polygons:
+            return None, None, None, None, np.empty((0, 7))
         return (np.empty((0, 2), dtype=np.int64), np.empty((0, 4)), np.empty(0, dtype=np.int32),
                 np.empty((0, kernels.TET_MAX_POLY, 3)), np.empty((0, 7)) if forces else None)
     st2, planes, nv, polys = kernels.tet_pairs_batch(T1, e1, X1, T2, e2, X2, hp, E1, E2,
                                                      checked=False)
     F = (kernels.tet_contact_forces(T1, e1, hp, st2, planes, nv, polys, E1, checked=False)
          if forces else None)
+    if not polygons:
+        return None, None, None, None, F.cpu().numpy()
     return (hp.cpu().numpy().astype(np.int64), planes.cpu().numpy(), nv.cpu().numpy(),
             polys.cpu().numpy(), F.cpu().numpy() if forces else None)
 
@@ -382,11 +388,10 @@ class ContactSurface:
                 _transform_points(frame2world, t2.reshape(n * 4, 3)).reshape(n, 4, 3))
 
 
-def find_contact_surface(rigid_body1, rigid_body2, use_aabb_trees=False):
-    """Contact surface of two rigid bodies (_interface.py:52-101); like the
-    reference it re-expresses rigid_body1 in rigid_body2's frame.  Broad phase
-    over the tetrahedron boxes, then every overlapping tetrahedron pair on
-    the GPU."""
+def _contact_inputs(rigid_body1, rigid_body2, use_aabb_trees):
+    """Both bodies' tetrahedra on the GPU in rigid_body2's frame (rigid_body1 is
+    re-expressed in it), their transforms and the candidate pairs of the broad
+    phase over the tetrahedron boxes."""
     import torch
     rigid_body1.express_in(rigid_body2.body2origin_)
     T1 = torch.from_numpy(np.ascontiguousarray(rigid_body1.tetrahedra_points)).cuda()
@@ -402,6 +407,15 @@ def find_contact_surface(rigid_body1, rigid_body2, use_aabb_trees=False):
         pairs = kernels.bvh_query(kernels.bvh_build(ab2), ab1)
     else:
         pairs = np.empty((0, 2), dtype=np.int64)
+    return T1, X1, T2, X2, pairs
+
+
+def find_contact_surface(rigid_body1, rigid_body2, use_aabb_trees=False):
+    """Contact surface of two rigid bodies (_interface.py:52-101); like the
+    reference it re-expresses rigid_body1 in rigid_body2's frame.  Broad phase
+    over the tetrahedron boxes, then every overlapping tetrahedron pair on
+    the GPU."""
+    T1, X1, T2, X2, pairs = _contact_inputs(rigid_body1, rigid_body2, use_aabb_trees)
     E1, E2 = rigid_body1.youngs_modulus, rigid_body2.youngs_modulus
     if len(pairs) == 0:
         surface = ContactSurface(rigid_body2.body2origin_, False, np.empty((0, 4)), [], [], [])
@@ -456,12 +470,15 @@ def compute_contact_force(tetrahedron, epsilon, contact_plane_hnf, contact_polyg
 def accumulate_wrenches(contact_surface, rigid_body1, rigid_body2):
     """Net wrenches of the polygon forces about each body's centre of mass,
     in the world frame (_forces.py:114-139)."""
-    f = contact_surface.contact_forces
-    c = contact_surface.contact_coms
+    return _wrenches(contact_surface.contact_forces, contact_surface.contact_coms,
+                     contact_surface.frame2world, rigid_body1, rigid_body2)
+
+
+def _wrenches(f, c, frame2world, rigid_body1, rigid_body2):
     force21 = np.sum(f, axis=0)
     torque21 = np.sum(np.cross(c - rigid_body1.com, f), axis=0)
     torque12 = np.sum(np.cross(c - rigid_body2.com, -f), axis=0)
-    adj = _adjoint_from_transform(contact_surface.frame2world)
+    adj = _adjoint_from_transform(frame2world)
     wrench21 = adj.T.dot(np.hstack((force21, torque21)))
     wrench12 = adj.T.dot(np.hstack((-force21, torque12)))
     return wrench12, wrench21
@@ -470,12 +487,21 @@ def accumulate_wrenches(contact_surface, rigid_body1, rigid_body2):
 def contact_forces(rigid_body1, rigid_body2, return_details=False):
     """(intersection, wrench12_in_world, wrench21_in_world[, details]) of two
     rigid bodies (_interface.py:8-49)."""
+    if not return_details:
+        # the wrenches need the polygons' centres and forces, not the polygons
+        T1, X1, T2, X2, pairs = _contact_inputs(rigid_body1, rigid_body2, False)
+        F = np.empty((0, 7))
+        if len(pairs):
+            F = _intersecting(T1, rigid_body1.tetrahedra_potentials, X1, T2,
+                              rigid_body2.tetrahedra_potentials, X2, pairs,
+                              rigid_body1.youngs_modulus, rigid_body2.youngs_modulus, True,
+                              checked=False, polygons=False)[4]
+        return (len(F) > 0,) + _wrenches(F[:, 3:6], F[:, 0:3], rigid_body2.body2origin_,
+                                         rigid_body1, rigid_body2)
     surface = find_contact_surface(rigid_body1, rigid_body2)
     wrench12, wrench21 = accumulate_wrenches(surface, rigid_body1, rigid_body2)
-    if return_details:
-        details = surface.make_details(rigid_body1.tetrahedra_points, rigid_body2.tetrahedra_points)
-        return surface.intersection, wrench12, wrench21, details
-    return surface.intersection, wrench12, wrench21
+    details = surface.make_details(rigid_body1.tetrahedra_points, rigid_body2.tetrahedra_points)
+    return surface.intersection, wrench12, wrench21, details
 
 
 class HydroelasticBoundingVolumeHierarchy(BoundingVolumeHierarchy):
