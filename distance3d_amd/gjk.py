@@ -53,10 +53,18 @@ def gjk_distance_jolt(collider1, collider2, tolerance=1e-10, max_distance_square
     than ``sqrt(max_distance_squared)``.  ``simplex`` is the (4, 3) array of
     Minkowski-difference support points the loop ended with.
     """
+    import torch
     scene, i1, i2 = _pair_scene(collider1, collider2)
-    r = kernels.gjk_distance_batch(scene, [i1], [i2], tolerance, max_distance_squared,
-                                   sanity_check, want_simplex=True)
-    status = int(r.status.cpu().item())
+    pair = torch.tensor([i1, i2], dtype=torch.int32).to(scene.device)
+    # every output in one device row, so that one copy brings them back: distance,
+    # closest points, simplex, then status, iterations and point count as int32
+    row = torch.empty(45, dtype=torch.float64, device=scene.device)
+    ints = row[43:].view(torch.int32)
+    out = kernels.GjkResult(row[0:1], row[1:4], row[4:7], ints[0:1], ints[1:2], row[7:43], ints[2:3])
+    kernels.gjk_distance_batch(scene, pair[:1], pair[1:], tolerance, max_distance_squared,
+                               sanity_check, out=out)
+    host = row.cpu().numpy()
+    status, _, n_points, _ = (int(x) for x in host[43:].view(np.int32))
     if status & 0xFF == _native.CLIPPED:
         return MAX_FLOAT, None, None, None
     if status & _native.BAD_INPUT:
@@ -65,12 +73,9 @@ def gjk_distance_jolt(collider1, collider2, tolerance=1e-10, max_distance_square
         raise AssertionError("Sanity check failed")
     if status & 0xFF == _native.ITER_CAP:
         raise RuntimeError("GJK did not terminate within the iteration cap")
-    dist = float(r.dist.cpu().item())
-    cp1 = r.cp_a.cpu().numpy()[0]
-    cp2 = r.cp_b.cpu().numpy()[0]
-    S = r.simplex.cpu().numpy()[0]
-    simplex = GjkSimplex(S[0], S[1], S[2], int(r.n_points.cpu().item()))
-    return dist, cp1, cp2, simplex
+    S = host[7:43].reshape(3, 4, 3)
+    return (float(host[0]), host[1:4].copy(), host[4:7].copy(),
+            GjkSimplex(S[0], S[1], S[2], n_points))
 
 
 def gjk_intersection_jolt(collider1, collider2, tolerance=1e-10):

@@ -32,6 +32,9 @@ F64_COLS = 16
 I32_COLS = 4
 _ULP_MARGIN = 1.0 + 2.0 ** -20
 CLUSTER_MIN_VERTICES = 64
+# a scene of at most this many bytes is uploaded in one copy, staged in one host
+# array; a large one array by array, without a second host copy of it
+PACKED_UPLOAD_MAX = 1 << 20
 
 
 def plane_basis_from_normal(plane_normal):
@@ -145,6 +148,34 @@ def cluster_layout(host, min_vertices=CLUSTER_MIN_VERTICES, threads=0):
     return out
 
 
+def _upload(layout, device):
+    """The arrays of a scene layout as device tensors (None stays None, an empty
+    array becomes one zero row).  The eight arrays of a small scene are views of
+    one tensor, each at a multiple of 256 bytes, so that one copy brings all."""
+    import torch
+    arrays = {}
+    for name, a in layout.items():
+        if a is not None:
+            a = np.ascontiguousarray(a) if len(a) else np.zeros((1,) + a.shape[1:], a.dtype)
+        arrays[name] = a
+    total = sum((a.nbytes + 255) // 256 * 256 for a in arrays.values() if a is not None)
+    if total > PACKED_UPLOAD_MAX:
+        return {name: None if a is None else torch.from_numpy(a).to(device)
+                for name, a in arrays.items()}
+    host = np.zeros(total, np.uint8)
+    at = {}
+    end = 0
+    for name, a in arrays.items():
+        if a is not None:
+            at[name] = end
+            host[end:end + a.nbytes] = a.reshape(-1).view(np.uint8)
+            end += (a.nbytes + 255) // 256 * 256
+    packed = torch.from_numpy(host).to(device)
+    return {name: None if a is None else
+            packed[at[name]:at[name] + a.nbytes].view(getattr(torch, a.dtype.name)).view(a.shape)
+            for name, a in arrays.items()}
+
+
 class DeviceScene:
     """A scene resident in HBM (torch tensors) plus its C descriptor.
 
@@ -158,24 +189,13 @@ class DeviceScene:
         self.device = dev
         self.host = host
 
-        def up(a, dtype):
-            if len(a) == 0:
-                a = np.zeros((1,) + a.shape[1:], dtype=a.dtype)
-            return torch.from_numpy(np.ascontiguousarray(a)).to(dev, dtype=dtype)
-
         if cluster_min and cluster_min > 0:
             lay = cluster_layout(host, cluster_min)
         else:
             lay = {"shape_f64": host.shape_f64, "shape_i32": host.shape_i32, "vx": host.vx,
                    "vy": host.vy, "vz": host.vz, "v64": host.v64, "vorig": None, "clusters": None}
-        self.shape_f64 = up(lay["shape_f64"], torch.float64)
-        self.shape_i32 = up(lay["shape_i32"], torch.int32)
-        self.vx = up(lay["vx"], torch.float32)
-        self.vy = up(lay["vy"], torch.float32)
-        self.vz = up(lay["vz"], torch.float32)
-        self.v64 = up(lay["v64"], torch.float64)
-        self.vorig = None if lay["vorig"] is None else up(lay["vorig"], torch.int32)
-        self.clusters = None if lay["clusters"] is None else up(lay["clusters"], torch.float32)
+        for name, tensor in _upload(lay, dev).items():
+            setattr(self, name, tensor)
         self.n_shapes = host.n_shapes
         self.n_vertices = len(lay["vx"])
         self.n_vertices64 = len(lay["v64"])
