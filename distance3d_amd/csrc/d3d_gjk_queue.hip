@@ -32,18 +32,48 @@ __global__ void queue_clear_kernel(int32_t *hdr, int n) {
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) hdr[i] = 0;
 }
 
-__global__ __launch_bounds__(kQBlock) void queue_hist_kernel(d3d_scene s,
-                                                             const int32_t *__restrict__ pa,
-                                                             const int32_t *__restrict__ pb,
-                                                             int64_t n, int32_t *__restrict__ hist) {
+// Counting and scattering go over tiles of kSortThreads * kItems pairs, a tile
+// per block: every block adds its counts of the keys it met to a few hundred
+// global counters, so a large batch takes large tiles (see queue_sort).
+constexpr int kSortThreads = 512;
+
+// The keys of a thread's pairs of a tile (-1 past the end), with the loads of
+// all of them out together.
+template <int kItems>
+__device__ __forceinline__ void tile_keys(const d3d_scene &s, const int32_t *__restrict__ pa,
+                                          const int32_t *__restrict__ pb, int64_t n, int64_t base,
+                                          int (&key)[kItems]) {
+    int a[kItems], b[kItems];
+#pragma unroll
+    for (int j = 0; j < kItems; ++j) {
+        const int64_t i = base + j * kSortThreads + threadIdx.x;
+        a[j] = i < n ? pa[i] : -1;
+        b[j] = i < n ? pb[i] : -1;
+    }
+#pragma unroll
+    for (int j = 0; j < kItems; ++j) {
+        const int64_t i = base + j * kSortThreads + threadIdx.x;
+        const int k = pair_key(s, a[j], b[j]);
+        key[j] = i < n ? k : -1;
+    }
+}
+
+template <int kItems>
+__global__ __launch_bounds__(kSortThreads) void queue_hist_kernel(d3d_scene s,
+                                                                  const int32_t *__restrict__ pa,
+                                                                  const int32_t *__restrict__ pb,
+                                                                  int64_t n,
+                                                                  int32_t *__restrict__ hist) {
     __shared__ int32_t h[kNumKeys];
-    for (int i = threadIdx.x; i < kNumKeys; i += kQBlock) h[i] = 0;
+    for (int i = threadIdx.x; i < kNumKeys; i += kSortThreads) h[i] = 0;
+    int key[kItems];
+    tile_keys<kItems>(s, pa, pb, n, (int64_t)blockIdx.x * kSortThreads * kItems, key);
     __syncthreads();
-    for (int64_t i = (int64_t)blockIdx.x * kQBlock + threadIdx.x; i < n;
-         i += (int64_t)gridDim.x * kQBlock)
-        atomicAdd(&h[pair_key(s, pa[i], pb[i])], 1);
+#pragma unroll
+    for (int j = 0; j < kItems; ++j)
+        if (key[j] >= 0) atomicAdd(&h[key[j]], 1);
     __syncthreads();
-    for (int i = threadIdx.x; i < kNumKeys; i += kQBlock)
+    for (int i = threadIdx.x; i < kNumKeys; i += kSortThreads)
         if (h[i]) atomicAdd(&hist[i], h[i]);
 }
 
@@ -88,28 +118,28 @@ __global__ __launch_bounds__(kQBlock) void queue_scan_kernel(int32_t *__restrict
     }
 }
 
-__global__ __launch_bounds__(kQBlock) void queue_scatter_kernel(
+template <int kItems>
+__global__ __launch_bounds__(kSortThreads) void queue_scatter_kernel(
     d3d_scene s, const int32_t *__restrict__ pa, const int32_t *__restrict__ pb, int64_t n,
     const int32_t *__restrict__ key_off, int32_t *__restrict__ key_cur,
     int32_t *__restrict__ order) {
     __shared__ int32_t h[kNumKeys];
-    __shared__ int32_t base[kNumKeys];
-    for (int64_t b0 = (int64_t)blockIdx.x * kQBlock; b0 < n; b0 += (int64_t)gridDim.x * kQBlock) {
-        for (int i = threadIdx.x; i < kNumKeys; i += kQBlock) h[i] = 0;
-        __syncthreads();
-        const int64_t i = b0 + threadIdx.x;
-        int key = 0, rank = 0;
-        if (i < n) {
-            key = pair_key(s, pa[i], pb[i]);
-            rank = atomicAdd(&h[key], 1);
-        }
-        __syncthreads();
-        for (int k = threadIdx.x; k < kNumKeys; k += kQBlock)
-            if (h[k]) base[k] = atomicAdd(&key_cur[k], h[k]);
-        __syncthreads();
-        if (i < n) order[key_off[key] + base[key] + rank] = (int32_t)i;
-        __syncthreads();
-    }
+    for (int i = threadIdx.x; i < kNumKeys; i += kSortThreads) h[i] = 0;
+    const int64_t base = (int64_t)blockIdx.x * kSortThreads * kItems;
+    int key[kItems], rank[kItems];
+    tile_keys<kItems>(s, pa, pb, n, base, key);
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < kItems; ++j) rank[j] = key[j] >= 0 ? atomicAdd(&h[key[j]], 1) : 0;
+    __syncthreads();
+    // the tile's place among the pairs of each key it met
+    for (int k = threadIdx.x; k < kNumKeys; k += kSortThreads)
+        if (h[k]) h[k] = key_off[k] + atomicAdd(&key_cur[k], h[k]);
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < kItems; ++j)
+        if (key[j] >= 0)
+            order[h[key[j]] + rank[j]] = (int32_t)(base + j * kSortThreads + threadIdx.x);
 }
 
 // the EPA list counter and the EPA claim cursor
@@ -635,17 +665,23 @@ int queue_sort(const d3d_scene &s, const int32_t *pa, const int32_t *pb, int64_t
     hipLaunchKernelGGL(queue_clear_kernel, dim3(4), dim3(kQBlock), 0, stream, w.hist,
                        (int)ws_header_ints());
     D3D_CHECK_LAUNCH("queue_clear_kernel");
-    int64_t g = (n + kQBlock - 1) / kQBlock;
-    if (g > 2048) g = 2048;
-    hipLaunchKernelGGL(queue_hist_kernel, dim3((unsigned)g), dim3(kQBlock), 0, stream, s, pa, pb, n,
-                       w.hist);
-    D3D_CHECK_LAUNCH("queue_hist_kernel");
-    hipLaunchKernelGGL(queue_scan_kernel, dim3(1), dim3(kQBlock), 0, stream, w.hist, w.key_off,
-                       w.cls_begin, w.cls_count);
-    D3D_CHECK_LAUNCH("queue_scan_kernel");
-    hipLaunchKernelGGL(queue_scatter_kernel, dim3((unsigned)g), dim3(kQBlock), 0, stream, s, pa, pb,
-                       n, w.key_off, w.key_cur, w.order);
-    D3D_CHECK_LAUNCH("queue_scatter_kernel");
+    auto sort = [&](auto hist, auto scatter, int items) {
+        const int64_t tile = (int64_t)kSortThreads * items;
+        const unsigned blocks = (unsigned)((n + tile - 1) / tile);
+        hipLaunchKernelGGL(hist, dim3(blocks), dim3(kSortThreads), 0, stream, s, pa, pb, n, w.hist);
+        hipLaunchKernelGGL(queue_scan_kernel, dim3(1), dim3(kQBlock), 0, stream, w.hist, w.key_off,
+                           w.cls_begin, w.cls_count);
+        hipLaunchKernelGGL(scatter, dim3(blocks), dim3(kSortThreads), 0, stream, s, pa, pb, n, w.key_off,
+                           w.key_cur, w.order);
+    };
+    // the whole sort with 1 / 2 / 4 / 8 pairs per thread: 16,384 mixed pairs 19 / 21
+    // / 25 / 33 us, 131,072 pairs 28 / 25 / 26 / 33, 262,144 pairs 40 / 31 / 29 / 34,
+    // 1,048,576 pairs 98 / 65 / 53 / 47 (129 us with 256-pair tiles)
+    if (n < 65536) sort(queue_hist_kernel<1>, queue_scatter_kernel<1>, 1);
+    else if (n < 196608) sort(queue_hist_kernel<2>, queue_scatter_kernel<2>, 2);
+    else if (n < 786432) sort(queue_hist_kernel<4>, queue_scatter_kernel<4>, 4);
+    else sort(queue_hist_kernel<8>, queue_scatter_kernel<8>, 8);
+    D3D_CHECK_LAUNCH("queue sort");
     return D3D_OK;
 }
 

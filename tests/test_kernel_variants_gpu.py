@@ -128,10 +128,11 @@ def test_intersection_by_batch_size(gpu, kind, n):
     assert int(hit[-1]) == 0 and int(status[-1]) == 0x200
 
 
-@pytest.mark.parametrize("n", (1, 1023, 1025, 4095, 4096, 4097))
+@pytest.mark.parametrize("n", (1, 1023, 1025, 4095, 4096, 4097, 65535, 65537, 196607, 196609, 786431,
+                               786433))
 def test_pair_sort_by_batch_size(gpu, n):
-    """GJK distance and intersection on both sides of the one-block sort, with
-    invalid pairs: every pair is taken exactly once."""
+    """GJK distance and intersection on both sides of the one-block sort and of
+    the tile sizes, with invalid pairs: every pair is taken exactly once."""
     host = workloads.mixed_pairs(seed=9, n_pairs=200).scene
     rs = np.random.RandomState(n)
     a, b = rs.randint(0, host.n_shapes, (2, n)).astype(np.int32)
