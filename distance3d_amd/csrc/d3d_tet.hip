@@ -87,12 +87,16 @@ __device__ __forceinline__ bool plane_cuts(const double *__restrict__ T, const d
 // A wavefront per block goes over 64 pairs at a time, one per lane: the plane,
 // and whether it cuts both tetrahedra.  Only the pairs it cuts (40% of random
 // pairs, 60% of a contact's candidates) have a polygon to clip, by far the
-// longer part, so they wait in an LDS queue until 64 of them fill the lanes.
+// longer part, so they wait in an LDS queue, with their planes, until 64 of them
+// fill the lanes.
 // Polygon rows are first filled with NaN by the whole wavefront in consecutive
 // stores; a lane that filled its own row stored 8 bytes every 576.
 // Bound: FP64 instructions of the clipping, and with polygons the 576 bytes a
 // pair takes.  524,289 random pairs, planes and polygons: 277 us one pair per
-// lane throughout, now 196 us; status only 168 and 143 us.
+// lane throughout, 196 us where the queue held the pairs only and their planes
+// were computed again, 186 us now; status only 168, 143 and 137 us.  Where the
+// planes cut most pairs the queue has little to gain: the whole contact of two
+// deeply overlapping bodies, 5,094,572 candidates, 1.01, 1.09 and 1.03 ms.
 __global__ __launch_bounds__(kTetBlock) void tet_pair_kernel(
     const double *__restrict__ T1, const double *__restrict__ e1, const double *__restrict__ X1,
     const double *__restrict__ T2, const double *__restrict__ e2, const double *__restrict__ X2,
@@ -101,30 +105,38 @@ __global__ __launch_bounds__(kTetBlock) void tet_pair_kernel(
     double *__restrict__ polys, double *__restrict__ work) {
     __shared__ double ang_s[kTetMaxPoly][kTetBlock];
     __shared__ unsigned char ord_s[kTetMaxPoly][kTetBlock];
+    // a ring of the waiting pairs, their tetrahedra and their planes; a pair of
+    // the contact_plane-is-true case is stored as ~k
     __shared__ int64_t queue[2 * kTetBlock];
+    __shared__ int2 queue_ij[2 * kTetBlock];
+    __shared__ double queue_h[4][2 * kTetBlock];
     const int lane = threadIdx.x;
     const unsigned long long lt = lane == 0 ? 0ull : (~0ull >> (kWave - lane));
     // the 2-D polygon points of the lane's current pair live in its own
     // workspace row
     double *pts = work + 2 * kTetMaxPoly * ((int64_t)blockIdx.x * kTetBlock + lane);
-    int waiting = 0;  // pairs in the queue
+    int first = 0, waiting = 0;  // pairs in the queue
 
     // the polygons of the first `count` pairs of the queue
     auto clip = [&](int count) {
     // the NaN rows are in memory before polygon points go over them
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    if (polys) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     if (lane < count) {
-    const int64_t k = queue[lane];
-    const int64_t i = pairs[2 * k], j = pairs[2 * k + 1];
+    const int slot = (first + lane) & (2 * kTetBlock - 1);
+    const int64_t item = queue[slot], k = item < 0 ? ~item : item;
+    const int2 ij = queue_ij[slot];
+    const int64_t i = ij.x, j = ij.y;
     const double *t2 = T2 + 12 * j;
     const double *x1 = X1 + 16 * i, *x2 = X2 + 16 * j;
-    const double *p1 = e1 + 4 * i, *p2 = e2 + 4 * j;
+    const double *p2 = e2 + 4 * j;
     // planes and polygons are optional outputs (NULL: status and vertex
     // count only)
     double *poly = polys ? polys + 3 * kTetMaxPoly * k : nullptr;
     int status = 0, nv = 0;
     double h[4];
-    if (contact_plane(p1, x1, E1, p2, x2, E2, h)) {
+#pragma unroll
+    for (int c = 0; c < 4; ++c) h[c] = queue_h[c][slot];
+    if (item < 0) {
         // _handle_same_tetrahedron (:142-159)
         double sum = 0.0;
 #pragma unroll
@@ -261,25 +273,27 @@ __global__ __launch_bounds__(kTetBlock) void tet_pair_kernel(
     status_out[k] = status;
     nv_out[k] = nv;
     }
-    // the pairs behind them move up
-    const int left = waiting - count;
-    const int64_t next = lane < left ? queue[count + lane] : 0;
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    if (lane < left) queue[lane] = next;
+    // their slots are free for what is queued next
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    waiting = left;
+    first = (first + count) & (2 * kTetBlock - 1);
+    waiting -= count;
     };
 
+    // the pairs of the next 64 are loaded ahead
+    auto load_pair = [&](int64_t k) { return k < m ? make_int2(pairs[2 * k], pairs[2 * k + 1]) : make_int2(0, 0); };
+    int2 ij = load_pair((int64_t)blockIdx.x * kTetBlock + lane);
     for (int64_t base = (int64_t)blockIdx.x * kTetBlock; base < m || waiting > 0;
          base += (int64_t)gridDim.x * kTetBlock) {
         const int64_t k = base + lane;
-        bool clipped = false;
+        const int2 here = ij;
+        ij = load_pair(k + (int64_t)gridDim.x * kTetBlock);
+        bool same = false, clipped = false;
+        double h[4];
         if (k < m) {
-            const int64_t i = pairs[2 * k], j = pairs[2 * k + 1];
-            double h[4];
-            clipped = contact_plane(e1 + 4 * i, X1 + 16 * i, E1, e2 + 4 * j, X2 + 16 * j, E2, h) ||
-                      (plane_cuts(T1 + 12 * i, h) && plane_cuts(T2 + 12 * j, h));
+            const int64_t i = here.x, j = here.y;
+            same = contact_plane(e1 + 4 * i, X1 + 16 * i, E1, e2 + 4 * j, X2 + 16 * j, E2, h);
+            clipped = same || (plane_cuts(T1 + 12 * i, h) && plane_cuts(T2 + 12 * j, h));
             if (!clipped) {
                 if (planes) {
                     double *plane = planes + 4 * k;
@@ -295,7 +309,13 @@ __global__ __launch_bounds__(kTetBlock) void tet_pair_kernel(
             for (int64_t q = lane; q < values; q += kTetBlock) fill[q] = NAN;
         }
         const unsigned long long mask = __ballot(clipped);
-        if (clipped) queue[waiting + __popcll(mask & lt)] = k;
+        if (clipped) {
+            const int slot = (first + waiting + __popcll(mask & lt)) & (2 * kTetBlock - 1);
+            queue[slot] = same ? ~k : k;
+            queue_ij[slot] = here;
+#pragma unroll
+            for (int c = 0; c < 4; ++c) queue_h[c][slot] = h[c];
+        }
         waiting += __popcll(mask);
         // the lanes read what the others queued
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
