@@ -910,11 +910,11 @@ extern "C" int d3d_gjk_intersection_batch_ws(const d3d_scene *scene, const int32
     if (int rc = check_scene(scene)) return rc;
     D3D_CHECK_ARG(n >= 0, "n must be >= 0");
     if (n == 0) return D3D_OK;
-    D3D_CHECK_ARG(n < (int64_t)0x7fffffff, "n must fit in int32");
     D3D_CHECK_ARG(pair_a && pair_b && hit && workspace, "NULL buffer");
     D3D_CHECK_ARG(max_iterations > 0, "max_iterations must be > 0");
     D3D_CHECK_ARG(workspace_bytes >= d3d_gjk_workspace_bytes(n), "workspace too small");
-    if (n < kIntersectQueueMin || scene->n_vertices == 0)
+    // (the queue holds pair indices as int32)
+    if (n < kIntersectQueueMin || n >= (int64_t)0x7fffffff || scene->n_vertices == 0)
         return d3d_gjk_intersection_batch(scene, pair_a, pair_b, n, tolerance, max_iterations, hit,
                                           status, stream);
     d3d_gjk_params prm = default_params();

@@ -82,8 +82,9 @@ def gjk_distance_batch(scene, pair_a, pair_b, tolerance=1e-10, max_distance_squa
     ``out`` may hold preallocated tensors (dist, cp_a, cp_b, status,
     iterations, simplex, n_points) and ``workspace`` a uint8 device tensor of
     at least :func:`gjk_workspace_bytes` bytes, so a loop allocates nothing.
-    ``lanes_per_pair`` (8 entries, one per work class) and ``launch`` (dict:
-    ``blocks_per_cu``, ``claim_factor``) override the launch tuning."""
+    ``lanes_per_pair`` (16 entries, one per work class, or 8, one per size
+    class) and ``launch`` (dict: ``blocks_per_cu``, ``claim_factor``) override
+    the launch tuning."""
     import torch
     a = _dev_i32(pair_a, scene.device)
     b = _dev_i32(pair_b, scene.device)
@@ -325,7 +326,7 @@ def epa_batch(scene, pair_a, pair_b, simplex, n_points, max_iterations=64, max_f
 
 
 class Bvh:
-    """A linear BVH over ``aabbs`` (n,3,2) float64 device tensor, held in a
+    """A box tree over ``aabbs`` (n,3,2) float64 device tensor, held in a
     device buffer (uint8 tensor).  The boxes must stay unchanged while the
     BVH is queried."""
 
@@ -353,7 +354,7 @@ def bvh_build(aabbs, stream=None):
 
 def bvh_refit(bvh, aabbs, stream=None):
     """New (n,3,2) float64 boxes for the leaves of ``bvh`` (box i keeps leaf
-    slot i, the topology stays); the boxes are copied into ``bvh.aabbs``."""
+    slot i, the tree's shape stays); the boxes are copied into ``bvh.aabbs``."""
     import torch
     a = torch.as_tensor(aabbs, dtype=torch.float64).reshape(-1, 3, 2)
     if a.shape[0] != bvh.n:
@@ -405,7 +406,7 @@ def bvh_query(bvh, queries, cap=None, counter=None, stream=None, sort=True):
     q = torch.as_tensor(queries, dtype=torch.float64)
     q = q.to(bvh.aabbs.device).reshape(-1, 3, 2).contiguous()
     m = q.shape[0]
-    if sort and m > 0:
+    if sort and 0 < m <= SORTED_QUERY_MAX_QUERIES:
         pairs = _bvh_query_sorted(bvh, q, cap, counter, stream)
         if pairs is not None:
             return pairs
@@ -431,6 +432,8 @@ def bvh_query(bvh, queries, cap=None, counter=None, stream=None, sort=True):
 # longest list of one query that is ordered by counting (quadratic in its
 # length) instead of a sort of all pairs
 SORTED_QUERY_MAX_LIST = 1024
+# its scratch takes 80 bytes per query beside the pairs: 5 GB at this many
+SORTED_QUERY_MAX_QUERIES = 1 << 26
 
 
 def _bvh_query_sorted(bvh, q, cap, counter, stream):
