@@ -1,5 +1,5 @@
 """AABB tree with the reference's interface (aabb_tree.py:15-191, 465-527),
-backed by a linear BVH built and queried on the GPU.
+backed by a packed box tree built and queried on the GPU.
 
 Leaf rows are numbered exactly as the reference numbers them (a bulk insert
 into an empty tree puts leaves at rows 0..n-1, later inserts append n leaf

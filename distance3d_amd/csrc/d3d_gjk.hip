@@ -1,9 +1,10 @@
-// d3d_gjk.hip -- batched GJK distance / intersection, support points and
-// AABBs for gfx950.
+// d3d_gjk.hip -- GJK intersection of small batches, support points and AABBs
+// for gfx950.
 //
-// (The batched GJK distance pipeline is in d3d_gjk_queue.hip.)
+// (GJK distance, and the intersection of larger batches, run through the sorted
+// pair queue in d3d_gjk_queue.hip.)
 //
-// Kernel shape: one lane per pair, 64 pairs per wavefront.  The FP64 simplex
+// Shape of the intersection kernel: one lane per pair, 64 pairs per wavefront.  The FP64 simplex
 // (Y, P, Q of up to four points) lives in VGPRs of its lane; support points of
 // analytic colliders and of small hulls are computed by the lane itself, while
 // large hulls are swept by the whole wavefront (coalesced FP32 SoA rows, see

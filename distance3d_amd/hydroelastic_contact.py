@@ -4,7 +4,7 @@ _forces.py, _tetrahedron_intersection.py:7-139, _barycentric_transform.py,
 _mesh_processing.py), evaluated by the gfx950 kernels:
 
 - d3d_tet_mesh_prep: per-tetrahedron AABBs and barycentric transforms;
-- the LBVH broad phase (all_aabbs_overlap / AabbTree) over those AABBs;
+- the broad phase (all_aabbs_overlap / AabbTree) over those AABBs;
 - d3d_tet_pairs_batch: per tetrahedron pair the contact plane where the two
   Young's-modulus-weighted pressure fields agree, and the contact polygon;
 - d3d_tet_contact_forces: centre, force and area of each polygon.

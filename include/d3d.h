@@ -115,12 +115,13 @@ typedef struct d3d_scene {
  *   5: <= 2048, 6: <= 4096, 7: > 4096;
  *   work class = size class, plus 8 when both colliders are hulls (D3D_NUM_CLASSES).
  * lanes_per_pair[c] lanes (a power of two <= 64; 0 = built-in default
- * 1,4,16,8,16,16,32,64 for one hull and 1,8,16,8,64,16,64,64 for two) work on
- * each pair of class c (class 0: 1, 2 or 4; larger values use 4).  For hull classes with 4 or more lanes, a pair whose hull
- * vertices fit the group's LDS slot (44, 85, 216, 456 or 1008 vertices with
- * 4, 8, 16, 32 or 64 lanes) has them copied there once and is swept from LDS;
- * when both colliders are hulls the two halves of the group sweep A and B
- * concurrently.
+ * 1,4,16,8,16,16,32,64 for one hull and 1,8,16,8,64,16,64,64 for two, widened
+ * on the device for a class whose pairs do not fill the chip) work on each
+ * pair of class c (class 0: 1, 2 or 4; larger values use 4).  For hull classes
+ * with 4 or more lanes, a pair whose hull vertices fit the group's LDS slot
+ * (44, 85, 216, 456 or 1008 vertices with 4, 8, 16, 32 or 64 lanes) has them
+ * copied there once and is swept from LDS; when both colliders are hulls the
+ * two halves of the group sweep A and B concurrently.
  * Launch shape (0 = built-in default): blocks_per_cu persistent GJK blocks of
  * four wavefronts per compute unit (1..3, default 3); claim_factor: a
  * wavefront claims claim_factor * 64 / G pairs of a class at a time (1..8,
@@ -504,7 +505,7 @@ int d3d_overlap_dense_write(const double *a, int64_t n, const double *b, int64_t
 /*
  * d3d_bvh_refit(aabbs (n,3,2) f64, n, bvh, bytes, stream): new boxes for the
  * leaves of a BVH that d3d_bvh_build built over n boxes (box i keeps leaf
- * slot i), keeping its topology: the node boxes are recomputed bottom-up and
+ * slot i), keeping the tree's shape: the node boxes are recomputed bottom-up and
  * queries stay exact (a node box only has to contain its leaves' boxes).
  * `aabbs` replaces the array the build was given.  Replaces the full
  * rebuild by serial insertion on every pose update in
