@@ -208,3 +208,19 @@ def test_intersection_large_batches(gpu, n):
     a, b = rs.randint(0, host.n_shapes, (2, n)).astype(np.int32)
     hit, _ = kernels.gjk_intersection_batch(host.to_device(), a, b)
     assert np.array_equal(hit.cpu().numpy(), oracle.gjk_intersection(host, a, b)[0])
+
+
+@pytest.mark.parametrize("boxes, queries, spread", [(1, 1, 0.0), (40, 300, 0.1), (600, 9, 0.1), (20000, 9001, 3.0),
+                                                    (3000, 50001, 8.0)])
+def test_unordered_query_is_the_ordered_set(boxes, queries, spread):
+    """A block's hits below, at and far above what it gathers at once, for each
+    number of lanes per query, with room for all pairs and for few at first."""
+    rng = np.random.default_rng(boxes)
+    lo = rng.uniform(-spread, spread, (boxes + queries, 3))
+    ab = np.stack([lo, lo + rng.uniform(0.05, 0.5, lo.shape)], axis=2)
+    bvh = kernels.bvh_build(torch.from_numpy(ab[:boxes]).cuda())
+    q = torch.from_numpy(ab[boxes:]).cuda()
+    want = kernels.bvh_query(bvh, q).cpu().numpy()
+    for cap in (None, 5):
+        got = kernels.bvh_query(bvh, q, cap=cap, sort=False).cpu().numpy()
+        np.testing.assert_array_equal(got[np.lexsort((got[:, 1], got[:, 0]))], want)
