@@ -1,6 +1,10 @@
 """Batched entry points over a device-resident scene (torch tensors in, torch
-tensors out).  Each function is one call into libd3d_hip on the current
-stream; none of them synchronises."""
+tensors out).  Each function is one call into libd3d_hip on the current stream,
+or on the one given as ``stream``, where its inputs must be ready; only those
+that read a count back to size their result synchronise with it."""
+import functools
+import inspect
+
 import numpy as np
 
 from . import _native
@@ -20,15 +24,53 @@ def _dev_f64(x, device):
                            dtype=torch.float64).to(device).contiguous()
 
 
-def _workspace(n_bytes, device, stream):
-    """A scratch tensor of one call, safe to drop when it runs on ``stream``."""
+def _workspace(n_bytes, device):
+    """A scratch tensor of one call on the current stream, dropped on return."""
     import torch
-    ws = torch.empty(max(int(n_bytes), 1), dtype=torch.uint8, device=device)
-    if stream is not None:
-        ws.record_stream(stream)
-    return ws
+    return torch.empty(max(int(n_bytes), 1), dtype=torch.uint8, device=device)
 
 
+def _tensors(out):
+    """The tensors of a batch function's result."""
+    import torch
+    if isinstance(out, torch.Tensor):
+        return [out]
+    if isinstance(out, (tuple, list)):
+        return [t for x in out for t in _tensors(x)]
+    return [t for t in getattr(out, "__dict__", {}).values() if isinstance(t, torch.Tensor)]
+
+
+def _on_stream(fn):
+    """Makes the ``stream`` argument of a batch function the current stream while
+    it runs.  Memory taken on a stream may still be in use by that stream's
+    earlier work, which only the stream itself is ordered behind: scratch taken
+    on the caller's stream and used on another one would be written under a
+    batch still running on the first.  The results are marked as used by the
+    caller's stream too, so that dropping them does not hand their memory to
+    the next call while the caller still reads it."""
+    at = list(inspect.signature(fn).parameters).index("stream")
+
+    @functools.wraps(fn)
+    def run(*args, **kwargs):
+        stream = args[at] if len(args) > at else kwargs.get("stream")
+        if stream is None:
+            return fn(*args, **kwargs)
+        import torch
+        if not isinstance(stream, torch.cuda.Stream):
+            stream = torch.cuda.ExternalStream(stream.cuda_stream)
+        caller = torch.cuda.current_stream(stream.device)
+        with torch.cuda.stream(stream):
+            out = fn(*args, **kwargs)
+        if caller != stream:
+            for t in _tensors(out):
+                if t.is_cuda:
+                    t.record_stream(caller)
+        return out
+
+    return run
+
+
+@_on_stream
 def support_batch(scene, shape_ids, dirs, stream=None):
     """Support points of ``scene`` colliders ``shape_ids`` along ``dirs``
     (n, 3) -> (n, 3) float64 tensor."""
@@ -44,6 +86,7 @@ def support_batch(scene, shape_ids, dirs, stream=None):
     return out
 
 
+@_on_stream
 def aabb_batch(scene, shape_ids, stream=None):
     """AABBs (n, 3, 2) of ``scene`` colliders ``shape_ids``."""
     import torch
@@ -73,6 +116,7 @@ class GjkResult:
         return self.dist == 0.0
 
 
+@_on_stream
 def gjk_distance_batch(scene, pair_a, pair_b, tolerance=1e-10, max_distance_squared=100000.0,
                        sanity_check=1e-8, max_iterations=128, lanes_per_pair=None,
                        want_simplex=False, want_iterations=True, out=None, workspace=None,
@@ -123,6 +167,7 @@ def gjk_workspace_bytes(n):
     return int(_native.load_library().d3d_gjk_workspace_bytes(int(n)))
 
 
+@_on_stream
 def gjk_intersection_batch(scene, pair_a, pair_b, tolerance=1e-10, max_iterations=128,
                            want_status=False, stream=None):
     """GJK intersection test over pairs -> (hit uint8 tensor, status or None)."""
@@ -134,13 +179,14 @@ def gjk_intersection_batch(scene, pair_a, pair_b, tolerance=1e-10, max_iteration
         raise ValueError("pair_a and pair_b differ in length")
     hit = torch.empty(n, dtype=torch.uint8, device=scene.device)
     status = torch.empty(n, dtype=torch.int32, device=scene.device) if want_status else None
-    ws = _workspace(gjk_workspace_bytes(n), scene.device, stream)
+    ws = _workspace(gjk_workspace_bytes(n), scene.device)
     check(lib().d3d_gjk_intersection_batch_ws(
         scene.c, ptr(a), ptr(b), n, float(tolerance), int(max_iterations), ptr(hit),
         ptr(status), ptr(ws), ws.numel(), stream_ptr(stream)), "d3d_gjk_intersection_batch_ws")
     return hit, status
 
 
+@_on_stream
 def mpr_batch(scene, pair_a, pair_b, centers, tolerance=0.0001, max_iterations=100,
               penetration=True, stream=None):
     """MPR over pairs (d3d_mpr_batch).  ``centers``: (n_shapes, 3) collider
@@ -160,7 +206,7 @@ def mpr_batch(scene, pair_a, pair_b, centers, tolerance=0.0001, max_iterations=1
                          % (scene.n_shapes, c.shape[0]))
     status = torch.empty(n, dtype=torch.int32, device=scene.device)
     out = torch.empty((n, 7), dtype=torch.float64, device=scene.device) if penetration else None
-    ws = _workspace(gjk_workspace_bytes(n), scene.device, stream)
+    ws = _workspace(gjk_workspace_bytes(n), scene.device)
     check(lib().d3d_mpr_batch_ws(scene.c, ptr(a), ptr(b), ptr(c), n, float(tolerance),
                                  int(max_iterations), 1 if penetration else 0, ptr(status),
                                  ptr(out), ptr(ws), ws.numel(), stream_ptr(stream)),
@@ -171,6 +217,7 @@ def mpr_batch(scene, pair_a, pair_b, centers, tolerance=0.0001, max_iterations=1
 TET_MAX_POLY = 24
 
 
+@_on_stream
 def tet_pairs_batch(T1, e1, X1, T2, e2, X2, pairs, youngs_modulus1=1.0, youngs_modulus2=1.0,
                     stream=None, geometry=True, checked=True):
     """Contact plane and polygon of tetrahedron pairs (d3d_tet_pairs_batch).
@@ -198,8 +245,7 @@ def tet_pairs_batch(T1, e1, X1, T2, e2, X2, pairs, youngs_modulus1=1.0, youngs_m
     planes = torch.empty((m, 4), dtype=torch.float64, device="cuda") if geometry else None
     nv = torch.empty(m, dtype=torch.int32, device="cuda")
     polys = torch.empty((m, TET_MAX_POLY, 3), dtype=torch.float64, device="cuda") if geometry else None
-    ws = torch.empty(max(int(_native.load_library().d3d_tet_pairs_workspace_bytes(m)), 1),
-                     dtype=torch.uint8, device="cuda")
+    ws = _workspace(_native.load_library().d3d_tet_pairs_workspace_bytes(m), "cuda")
     check(lib().d3d_tet_pairs_batch(ptr(T1), ptr(e1), ptr(X1), ptr(T2), ptr(e2), ptr(X2), ptr(pr),
                                     m, float(youngs_modulus1), float(youngs_modulus2), ptr(status),
                                     ptr(planes), ptr(nv), ptr(polys), ptr(ws), ws.numel(),
@@ -219,6 +265,7 @@ def _dev32(a, shape):
     return (t if t.is_cuda else t.cuda()).reshape(shape).contiguous()
 
 
+@_on_stream
 def polygon_angles(y, x, stream=None):
     """atan2(y, x) rounded correctly, elementwise (d3d_polygon_angles): the
     angle the contact-polygon ordering uses.  Returns a device tensor."""
@@ -233,6 +280,7 @@ def polygon_angles(y, x, stream=None):
     return out
 
 
+@_on_stream
 def tet_mesh_prep(T, aabbs=True, transforms=True, stream=None):
     """AABBs (n,3,2) and barycentric transforms (n,4,4) of tetrahedra T
     (n,4,3) (d3d_tet_mesh_prep).  Returns device tensors (aabbs or None, X or
@@ -249,6 +297,7 @@ def tet_mesh_prep(T, aabbs=True, transforms=True, stream=None):
     return ab, X, flags
 
 
+@_on_stream
 def tet_contact_forces(T1, e1, pairs, status, planes, n_vertices, polygons, youngs_modulus1=1.0,
                        stream=None, checked=True):
     """Centre, force and area of each intersecting pair's contact polygon
@@ -297,6 +346,7 @@ class EpaResult:
         return self.status == 1
 
 
+@_on_stream
 def epa_batch(scene, pair_a, pair_b, simplex, n_points, max_iterations=64, max_faces=128,
               epsilon=1e-8, stream=None, want_faces=False):
     """EPA over pairs seeded from GJK simplices ((n,3,4,3) Y/P/Q rows and
@@ -336,6 +386,7 @@ class Bvh:
         self.n = n
 
 
+@_on_stream
 def bvh_build(aabbs, stream=None):
     """Build a BVH over (n,3,2) float64 boxes (tensor or array)."""
     import torch
@@ -352,6 +403,7 @@ def bvh_build(aabbs, stream=None):
     return Bvh(a, buf, n)
 
 
+@_on_stream
 def bvh_refit(bvh, aabbs, stream=None):
     """New (n,3,2) float64 boxes for the leaves of ``bvh`` (box i keeps leaf
     slot i, the tree's shape stays); the boxes are copied into ``bvh.aabbs``."""
@@ -447,7 +499,9 @@ def _bvh_query_sorted(bvh, q, cap, counter, stream):
     result = torch.empty(3, dtype=torch.int64, device=q.device)
     while True:
         pairs = torch.empty((cap, 2), dtype=torch.int32, device=q.device)
-        ws = _workspace(lib().d3d_bvh_query_sorted_workspace_bytes(m, cap), q.device, stream)
+        ws = _workspace(lib().d3d_bvh_query_sorted_workspace_bytes(m, cap), q.device)
+        if stream is not None:
+            ws.record_stream(stream)
         check(lib().d3d_bvh_query_sorted(ptr(bvh.buffer), bvh.n, ptr(bvh.aabbs), ptr(q), m,
                                          ptr(pairs), cap, ptr(result), ptr(ws), ws.numel(),
                                          stream_ptr(stream)), "d3d_bvh_query_sorted")
@@ -489,6 +543,7 @@ class SceneView:
         return ctypes.byref(self._c)
 
 
+@_on_stream
 def instance_pairs(scene, pair_a, pair_b, pose_a=None, pose_b=None, pose_idx_a=None,
                    pose_idx_b=None, n_poses=0, out=None, stream=None):
     """Posed pair instances of ``scene`` colliders (see d3d_instance_pairs).
@@ -537,6 +592,7 @@ class GjkEpaResult:
                             torch.empty(n, dtype=torch.int32, device=device))
 
 
+@_on_stream
 def gjk_epa_batch(scene, pair_a, pair_b, out=None, workspace=None, lanes_per_pair=None,
                   epa_max_iterations=64, epa_max_faces=128, epa_epsilon=1e-8, stream=None,
                   iterations=None, **gjk_kw):
@@ -552,7 +608,7 @@ def gjk_epa_batch(scene, pair_a, pair_b, out=None, workspace=None, lanes_per_pai
     if out is None:
         out = GjkEpaResult.empty(n, scene.device)
     if workspace is None:
-        workspace = torch.empty(gjk_epa_workspace_bytes(n), dtype=torch.uint8, device=scene.device)
+        workspace = _workspace(gjk_epa_workspace_bytes(n), scene.device)
     prm = _native.gjk_params(lanes_per_pair=lanes_per_pair, **gjk_kw)
     check(lib().d3d_gjk_epa_batch_ws(
         scene.c, ptr(a), ptr(b), n, ctypes.byref(prm), int(epa_max_iterations),

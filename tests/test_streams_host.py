@@ -1,0 +1,81 @@
+"""A batch call on another stream takes its memory and makes its conversions,
+launches and read-backs on that stream: with the streams, the library and the
+allocations replaced, on the CPU."""
+import contextlib
+import types
+
+import numpy as np
+import pytest
+import torch
+
+from distance3d_amd import kernels
+
+
+class Stream:
+    device = "cpu"
+    cuda_stream = 7
+
+
+@pytest.fixture
+def calls(monkeypatch):
+    """Events of a call, each with the stream that was current: allocations by
+    their place of use and library functions by name."""
+    current = [Stream()]
+    seen = []
+
+    @contextlib.contextmanager
+    def on(stream):
+        current.append(stream)
+        yield
+        current.pop()
+
+    def recorded(name, fn, device=None):
+        def run(*args, **kwargs):
+            seen.append((name, current[-1]))
+            if device is not None:
+                kwargs["device"] = device
+            return fn(*args, **kwargs)
+        return run
+
+    class Lib:
+        def __getattr__(self, name):
+            if name.endswith("_bytes"):
+                return lambda *a: 4096
+            return recorded(name, lambda *a: 0)
+
+    monkeypatch.setattr(torch.cuda, "Stream", Stream)
+    monkeypatch.setattr(torch.cuda, "stream", on)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda device=None: current[-1])
+    monkeypatch.setattr(torch.Tensor, "cuda", lambda self: self)
+    monkeypatch.setattr(torch.Tensor, "record_stream", lambda self, stream: None)
+    monkeypatch.setattr(torch.Tensor, "item", recorded("item", torch.Tensor.item))
+    monkeypatch.setattr(torch.Tensor, "tolist", recorded("tolist", torch.Tensor.tolist))
+    for name in ("empty", "zeros"):
+        monkeypatch.setattr(torch, name, recorded(name, getattr(torch, name), "cpu"))
+    monkeypatch.setattr(kernels, "lib", Lib)
+    monkeypatch.setattr(kernels._native, "load_library", Lib)
+    return seen
+
+
+PAIRS = np.zeros(40, dtype=np.int32)
+SCENE = types.SimpleNamespace(device="cpu", n_shapes=3, c=None)
+TETS = [np.zeros((2, 4, 3)), np.zeros((2, 4)), np.zeros((2, 4, 4))]
+
+CALLS = {
+    "gjk_intersection_batch": lambda s: kernels.gjk_intersection_batch(SCENE, PAIRS, PAIRS, stream=s),
+    "mpr_batch": lambda s: kernels.mpr_batch(SCENE, PAIRS, PAIRS, np.zeros((3, 3)), stream=s),
+    "gjk_epa_batch": lambda s: kernels.gjk_epa_batch(SCENE, PAIRS, PAIRS, stream=s),
+    "gjk_distance_batch": lambda s: kernels.gjk_distance_batch(SCENE, PAIRS, PAIRS, stream=s),
+    "tet_pairs_batch": lambda s: kernels.tet_pairs_batch(*TETS, *TETS, np.zeros((5, 2)), checked=False,
+                                                         stream=s),
+    "bvh_build": lambda s: kernels.bvh_build(np.zeros((4, 3, 2)), stream=s),
+}
+
+
+@pytest.mark.parametrize("name", sorted(CALLS))
+def test_memory_and_launches_are_the_streams(calls, name):
+    stream = Stream()
+    CALLS[name](stream)
+    assert any(what.startswith("d3d_") for what, _ in calls)
+    assert any(what in ("empty", "zeros") for what, _ in calls)
+    assert all(on is stream for _, on in calls), [what for what, on in calls if on is not stream]
