@@ -421,6 +421,7 @@ def bvh_refit(bvh, aabbs, stream=None):
 DENSE_OVERLAP_MAX_TESTS = 1 << 28
 
 
+@_on_stream
 def overlap_dense(a, b, cap=None, counter=None, stream=None):
     """All (i, j) with closed-interval overlap of a[i] and b[j], by testing
     every pair (d3d_overlap_dense), row-major (i, then j ascending), as an
@@ -432,8 +433,7 @@ def overlap_dense(a, b, cap=None, counter=None, stream=None):
     n, m = a.shape[0], b.shape[0]
     if counter is None:
         counter = torch.zeros(1, dtype=torch.int64, device=a.device)
-    ws = torch.empty(max(int(_native.load_library().d3d_overlap_dense_workspace_bytes(n)), 8),
-                     dtype=torch.uint8, device=a.device)
+    ws = _workspace(_native.load_library().d3d_overlap_dense_workspace_bytes(n), a.device)
     if cap is None:
         cap = 4 * n + 1024
     pairs = torch.empty((max(cap, 1), 2), dtype=torch.int32, device=a.device)
@@ -448,6 +448,7 @@ def overlap_dense(a, b, cap=None, counter=None, stream=None):
     return pairs[:k]
 
 
+@_on_stream
 def bvh_query(bvh, queries, cap=None, counter=None, stream=None, sort=True):
     """All (query, box) index pairs with closed-interval overlap, as an
     (k, 2) int32 device tensor (lexicographically sorted when ``sort``).
@@ -500,17 +501,10 @@ def _bvh_query_sorted(bvh, q, cap, counter, stream):
     while True:
         pairs = torch.empty((cap, 2), dtype=torch.int32, device=q.device)
         ws = _workspace(lib().d3d_bvh_query_sorted_workspace_bytes(m, cap), q.device)
-        if stream is not None:
-            ws.record_stream(stream)
         check(lib().d3d_bvh_query_sorted(ptr(bvh.buffer), bvh.n, ptr(bvh.aabbs), ptr(q), m,
                                          ptr(pairs), cap, ptr(result), ptr(ws), ws.numel(),
                                          stream_ptr(stream)), "d3d_bvh_query_sorted")
-        if stream is None:
-            k, longest, spilled = result.tolist()
-        else:
-            result.record_stream(stream)
-            with torch.cuda.stream(stream):
-                k, longest, spilled = result.tolist()
+        k, longest, spilled = result.tolist()
         if spilled and longest > SORTED_QUERY_MAX_LIST:
             return None
         if k <= cap:

@@ -61,3 +61,40 @@ def test_gjk_and_epa(streams, batches):
     want = [oracle.gjk_distance(host, a, b)["dist"] for a, b in lists]
     for k, out in _in_turn(streams, lists, lambda a, b, s: kernels.gjk_epa_batch(dev, a, b, stream=s)):
         assert np.array_equal(out.dist.cpu().numpy(), want[k])
+
+
+def _boxes(rs, n, size):
+    lo = rs.uniform(0.0, 10.0, (n, 3))
+    return np.stack([lo, lo + rs.uniform(0.1, size, (n, 3))], axis=2)
+
+
+@pytest.mark.parametrize("call", ("dense", "sorted", "unsorted", "long lists"))
+@pytest.mark.parametrize("cap", (None, 1))
+def test_box_overlaps(streams, call, cap):
+    """Counts read back from a stream that is behind the caller's: with room for
+    all pairs and for one at first."""
+    rs = np.random.RandomState(3)
+    boxes = [_boxes(rs, n, 0.7) for n in (900, 3000)]
+    queries = [_boxes(rs, n, 3.0 if call != "long lists" else 12.0) for n in (40, 200)]
+    for q, b in zip(queries, boxes):
+        q[0] = b[0]
+    ahead = torch.zeros(1 << 24, device="cuda")
+    for s in streams:
+        for q, b in zip(queries, boxes):
+            want, _ = oracle.all_aabbs_overlap(q, b)
+            want = want[np.lexsort((want[:, 1], want[:, 0]))]
+            db, dq = torch.from_numpy(b).cuda(), torch.from_numpy(q).cuda()
+            torch.cuda.synchronize()
+            with torch.cuda.stream(s):
+                for _ in range(20):
+                    ahead.add_(1.0)
+            if call == "dense":
+                got = kernels.overlap_dense(dq, db, cap=cap, stream=s)
+            else:
+                bvh = kernels.bvh_build(db, stream=s)
+                got = kernels.bvh_query(bvh, dq, cap=cap, sort=call != "unsorted", stream=s)
+            torch.cuda.synchronize()
+            got = got.cpu().numpy()
+            if call == "unsorted":
+                got = got[np.lexsort((got[:, 1], got[:, 0]))]
+            assert np.array_equal(got, want)

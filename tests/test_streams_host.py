@@ -60,6 +60,7 @@ def calls(monkeypatch):
 PAIRS = np.zeros(40, dtype=np.int32)
 SCENE = types.SimpleNamespace(device="cpu", n_shapes=3, c=None)
 TETS = [np.zeros((2, 4, 3)), np.zeros((2, 4)), np.zeros((2, 4, 4))]
+BVH = kernels.Bvh(torch.zeros((4, 3, 2), dtype=torch.float64), torch.zeros(4096, dtype=torch.uint8), 4)
 
 CALLS = {
     "gjk_intersection_batch": lambda s: kernels.gjk_intersection_batch(SCENE, PAIRS, PAIRS, stream=s),
@@ -68,6 +69,9 @@ CALLS = {
     "gjk_distance_batch": lambda s: kernels.gjk_distance_batch(SCENE, PAIRS, PAIRS, stream=s),
     "tet_pairs_batch": lambda s: kernels.tet_pairs_batch(*TETS, *TETS, np.zeros((5, 2)), checked=False,
                                                          stream=s),
+    "overlap_dense": lambda s: kernels.overlap_dense(np.zeros((4, 3, 2)), np.zeros((9, 3, 2)), stream=s),
+    "bvh_query": lambda s: kernels.bvh_query(BVH, np.zeros((9, 3, 2)), stream=s),
+    "bvh_query unsorted": lambda s: kernels.bvh_query(BVH, np.zeros((9, 3, 2)), sort=False, stream=s),
     "bvh_build": lambda s: kernels.bvh_build(np.zeros((4, 3, 2)), stream=s),
 }
 
