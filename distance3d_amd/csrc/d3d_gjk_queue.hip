@@ -262,8 +262,7 @@ __device__ __forceinline__ bool gjk_distance_step(GjkState &g, const PQ &pq, v3 
     // in registers took two dozen selects per step: 1,048,576 mixed pairs 5,240 us,
     // 5,131 us this way); the group's lanes see what its first lane wrote
     pq.put(g.S.n < 3 ? g.S.n : 3, p, q);
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    row_fence();
     load_y(g.S, pq);
     g.S.n += 1;
     v3 nvec;
@@ -511,8 +510,7 @@ struct IntersectMode {
         g.state = D3D_SEPARATED;
         if (dot(g.d, w) < -kEps) return false;
         pq.put_p(g.n < 3 ? g.n : 3, w);
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        row_fence();
         // rows past the new one are not used
         Simplex S;
         S.n = g.n + 1;

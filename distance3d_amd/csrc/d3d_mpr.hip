@@ -399,6 +399,8 @@ struct MprMode {
     template <int G>
     static __device__ __forceinline__ bool step(State &g, const PQ &pq, v3 p, v3 q,
                                                 const d3d_gjk_params &, const Out &o) {
+        // all lanes of the group read the rows its first lane wrote in earlier rounds
+        row_fence();
         const v3 w = p - q;
         if (g.phase == kMprV1) {
             pq.put(1, p, q);

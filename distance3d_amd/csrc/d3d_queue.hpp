@@ -9,7 +9,9 @@
 //   step<G>(...)    one round with the supports on A along d and on B along -d;
 //                   false once the pair has terminated
 //   write / bad     the pair's outputs, by one lane; those of an invalid pair
-// A pair's rows of support points live in LDS (PQ).
+// A pair's rows of support points live in LDS (PQ): the group's first lane
+// writes them and all its lanes read them, so a step puts a row_fence between
+// the last write (its own or an earlier step's) and its reads.
 #pragma once
 
 #include "d3d_device.hpp"
@@ -136,6 +138,14 @@ struct PQ {
         if (c.m > 2) move<kParts>(c.k2, 2);
     }
 };
+
+// Orders a group's LDS writes (rows, slots) before its lanes' reads for the compiler, which
+// may otherwise keep the old value on the lanes that did not write; the
+// hardware runs a wavefront's LDS operations in order.
+__device__ __forceinline__ void row_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
 
 // ------------------------------------------------------- group supports
 
@@ -443,8 +453,7 @@ __device__ __forceinline__ void run_class(const d3d_scene &s, const int32_t *__r
                                 }
                             }
                             // the group's lanes read what the others wrote
-                            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-                            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+                            row_fence();
                         }
                     } else if (sub == 0) {
                         M::bad(pid, o);
