@@ -355,15 +355,16 @@ extern "C" int d3d_aabb_batch(const d3d_scene *scene, const int32_t *shape, int6
     // large one has wavefronts to spare.  4 / 16 / 64 colliders per wavefront:
     // 16,384 mixed 37 / 67 / 89 us, 131,072 mixed 146 / 125 / 165 us, 262,144
     // mixed 272 / 250 / 241 us; boxes alone 20,000 10.5 / 10.4 / 10.3 us, 200,000
-    // 36 / 14 / 11 us, 1,048,576 165 / 52 / 32 us.
+    // 36 / 14 / 11 us, 1,048,576 165 / 52 / 32 us: a scene without hull vertices has
+    // no sweeps, and always takes 64.
     const int serial_max = default_params().hull_serial_max;
     auto launch = [&](auto kernel, int per_wave) {
         hipLaunchKernelGGL(kernel, dim3(grid_for(n, kBlock / kWave * per_wave)), dim3(kBlock), 0,
                            (hipStream_t)stream, *scene, shape, n, serial_max, out);
     };
-    if (n < 65536) launch(aabb_kernel<4>, 4);
-    else if (n < 524288) launch(aabb_kernel<16>, 16);
-    else launch(aabb_kernel<64>, 64);
+    if (n >= 524288 || scene->n_vertices == 0) launch(aabb_kernel<64>, 64);
+    else if (n >= 65536) launch(aabb_kernel<16>, 16);
+    else launch(aabb_kernel<4>, 4);
     D3D_CHECK_LAUNCH("aabb_kernel");
     return D3D_OK;
 }

@@ -224,3 +224,14 @@ def test_unordered_query_is_the_ordered_set(boxes, queries, spread):
     for cap in (None, 5):
         got = kernels.bvh_query(bvh, q, cap=cap, sort=False).cpu().numpy()
         np.testing.assert_array_equal(got[np.lexsort((got[:, 1], got[:, 0]))], want)
+
+
+@pytest.mark.parametrize("n", (1, 63, 64, 65, 255, 257, 65535, 65537, 524289))
+def test_aabbs_without_hulls(gpu, n):
+    """A scene without hull vertices, on both sides of the sizes at which one
+    with hulls changes its colliders per wavefront."""
+    host = workloads.broad_phase_scene(n_boxes=50, n_capsules=20, extent=4.0).scene
+    ids = (np.arange(n) * 7 % host.n_shapes).astype(np.int32)
+    got = kernels.aabb_batch(host.to_device(), ids).cpu().numpy()
+    want = oracle.aabbs(host, np.arange(host.n_shapes, dtype=np.int32))
+    assert np.array_equal(got, want[ids])
