@@ -517,7 +517,7 @@ constexpr int kBlockHits = 512;
 template <int QL, bool kSorted>
 __global__ __launch_bounds__(kBvhBlock) void bvh_query_kernel(
     BvhLevels lv, const BvhNode *__restrict__ nodes, const double *__restrict__ aabbs,
-    const double *__restrict__ q, int64_t m, int32_t *__restrict__ pairs, int64_t cap,
+    const double *__restrict__ q, int64_t first, int64_t m, int32_t *__restrict__ pairs, int64_t cap,
     unsigned long long *__restrict__ counter, QueryWs ws) {
     constexpr int kGroups = kBvhBlock / QL;
     constexpr int W = QL / 8;
@@ -533,7 +533,7 @@ __global__ __launch_bounds__(kBvhBlock) void bvh_query_kernel(
     const int slot = sub >> 3, child = sub & 7;
     const int lane = lane_id();
     if (t < kBvhMaxLevels) off[t] = lv.off[t];
-    const int64_t qi = (int64_t)blockIdx.x * kGroups + g;
+    const int64_t qi = first + (int64_t)blockIdx.x * kGroups + g;
     const bool valid = qi < m;
     double Q[6];
     float qlo[3], qhi[3];
@@ -943,8 +943,14 @@ static void query_launch(const BvhView &v, int64_t n, const double *aabbs, const
     const BvhLevels lv = bvh_levels(n);
     auto go = [&](auto kernel, int lanes) {
         const int per = kBvhBlock / lanes;
-        hipLaunchKernelGGL(kernel, dim3((unsigned)((m + per - 1) / per)), dim3(kBvhBlock), 0, st, lv,
-                           v.nodes, aabbs, queries, m, pairs, cap, counter, ws);
+        // a launch has less than 2^32 threads; more queries (of an unordered call)
+        // take several
+        const int64_t slice = query_slice(kBvhBlock, per);
+        for (int64_t first = 0; first < m; first += slice) {
+            const int64_t k = min(slice, m - first);
+            hipLaunchKernelGGL(kernel, dim3((unsigned)((k + per - 1) / per)), dim3(kBvhBlock), 0, st, lv,
+                               v.nodes, aabbs, queries, first, m, pairs, cap, counter, ws);
+        }
     };
     switch (query_lanes(m)) {
     case 8: go(bvh_query_kernel<8, kSorted>, 8); break;
@@ -1004,7 +1010,7 @@ extern "C" int d3d_bvh_query_sorted(const void *bvh, int64_t n, const double *aa
                                     void *stream) {
     clear_error();
     D3D_CHECK_ARG(n >= 1 && n < (int64_t)0x40000000, "n must be in [1, 2^30)");
-    D3D_CHECK_ARG(m >= 1 && m < (int64_t)0x7fffffff, "m must be in [1, 2^31)");
+    D3D_CHECK_ARG(m >= 1 && m < (int64_t)0x10000000, "m must be in [1, 2^28)");
     D3D_CHECK_ARG(cap >= 1, "cap must be >= 1");
     D3D_CHECK_ARG(bvh && aabbs && queries && pairs && result && workspace, "NULL buffer");
     D3D_CHECK_ARG(workspace_bytes >= query_layout(m, cap, nullptr, nullptr), "workspace too small");
@@ -1034,7 +1040,7 @@ extern "C" int d3d_bvh_query_sorted_finish(int64_t m, int32_t *pairs, int64_t ca
                                            const uint64_t *result, void *workspace,
                                            int64_t workspace_bytes, void *stream) {
     clear_error();
-    D3D_CHECK_ARG(m >= 1 && m < (int64_t)0x7fffffff, "m must be in [1, 2^31)");
+    D3D_CHECK_ARG(m >= 1 && m < (int64_t)0x10000000, "m must be in [1, 2^28)");
     D3D_CHECK_ARG(cap >= 1, "cap must be >= 1");
     D3D_CHECK_ARG(pairs && result && workspace, "NULL buffer");
     D3D_CHECK_ARG(workspace_bytes >= query_layout(m, cap, nullptr, nullptr), "workspace too small");

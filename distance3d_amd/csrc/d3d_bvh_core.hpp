@@ -39,6 +39,10 @@ __host__ __device__ inline BvhLevels bvh_levels(int64_t n) {
     return lv;
 }
 
+// Queries of one launch of blocks of `block` threads with `per` queries each,
+// whole blocks: fewer than 2^32 threads.
+constexpr int64_t query_slice(int block, int per) { return (((int64_t)1 << 32) / block - 1) * per; }
+
 __host__ __device__ inline int clz32(uint32_t v) { return v ? __builtin_clz(v) : 32; }
 
 // Length of the common prefix of sorted keys i and j; equal keys compare

@@ -469,7 +469,7 @@ int d3d_bvh_query(const void *bvh, int64_t n, const double *aabbs, const double 
  * result[2] > 0 d3d_bvh_query_sorted_finish, with the same arguments, adds the
  * long lists (quadratic in a list's length: past about a thousand pairs per
  * query sort the output of d3d_bvh_query instead); when result[0] > cap call
- * again with more room.  m and cap must be >= 1; the workspace
+ * again with more room.  m must be in [1, 2^28), cap >= 1; the workspace
  * (d3d_bvh_query_sorted_workspace_bytes(m, cap) bytes) is the caller's.
  */
 int64_t d3d_bvh_query_sorted_workspace_bytes(int64_t m, int64_t cap);

@@ -235,3 +235,16 @@ def test_aabbs_without_hulls(gpu, n):
     got = kernels.aabb_batch(host.to_device(), ids).cpu().numpy()
     want = oracle.aabbs(host, np.arange(host.n_shapes, dtype=np.int32))
     assert np.array_equal(got, want[ids])
+
+
+def test_query_of_more_than_one_launch(gpu):
+    """More unordered queries than one launch has threads for (8 lanes each):
+    the last ones, far away from the empty rest, are found."""
+    m = (1 << 29) + 5
+    q = torch.full((m, 3, 2), 100.0, dtype=torch.float64, device="cuda")
+    at = torch.tensor([0, 7, (1 << 29) - 33, (1 << 29) - 32, 1 << 29, m - 1], device="cuda")
+    q[at] = torch.tensor([[0.5, 0.6]] * 3, dtype=torch.float64, device="cuda")
+    boxes = np.array([[[0.0, 1.0]] * 3, [[2.0, 3.0]] * 3])
+    got = kernels.bvh_query(kernels.bvh_build(boxes), q, cap=64, sort=False)
+    del q
+    assert torch.equal(got[torch.argsort(got[:, 0])].long(), torch.stack([at, torch.zeros_like(at)], 1))
