@@ -331,6 +331,17 @@ __device__ __forceinline__ SupportPair support_pair_bounds(const d3d_scene &s, i
     return SupportPair{a, b};
 }
 
+// Items of a class of `count` pairs that a wavefront claims at a time: `full`, or
+// the class's fair share per wavefront when that is smaller; and the chunks the
+// class has.  A class may have up to 2^31 - 2 pairs: the sums are unsigned.
+__host__ __device__ constexpr uint32_t chunks_of(int count, int chunk) {
+    return ((uint32_t)count + (uint32_t)chunk - 1u) / (uint32_t)chunk;
+}
+__host__ __device__ constexpr int claim_chunk(int count, int n_waves, int full) {
+    const uint32_t fair = chunks_of(count, n_waves);
+    return fair < (uint32_t)full ? (int)fair : full;
+}
+
 // One work class, G lanes per pair, by one wavefront: groups of G lanes take
 // pairs of the class (chunked claims from the class cursor) until the class is
 // exhausted and every group of the wavefront has finished its pair.  The
@@ -376,8 +387,9 @@ __device__ __forceinline__ void run_class(const d3d_scene &s, const int32_t *__r
     const int64_t r = (wv - rot + n_waves) % n_waves;
     const int64_t fixed_end = (int64_t)n_waves * chunk;
     const bool dynamic = fixed_end < count;
-    int cb = (int)min(r * chunk, (int64_t)count), ce = cb + chunk;
-    // the wavefront's unclaimed items are [cb, ce) of the class
+    // the wavefront's unclaimed items are [cb, ce) of the class; past its end every
+    // wavefront claims one more chunk, which goes beyond 2^31 in a class close to it
+    uint32_t cb = (uint32_t)min(r * chunk, (int64_t)count), ce = cb + (uint32_t)chunk;
     while (true) {
         const bool need = !have && !exhausted;
         const unsigned long long m = __ballot(need && sub == 0);
@@ -387,30 +399,30 @@ __device__ __forceinline__ void run_class(const d3d_scene &s, const int32_t *__r
             // ranked past the items at hand wait for the next round.
             const int c = __popcll(m);
             const int rank = __popcll(m & lanemask_lt(leader));
-            const int avail = ce - cb;
-            int nb = 0;
+            const int avail = (int)(ce - cb);
+            uint32_t nb = 0;
             if (avail < c) {
                 const int first = __ffsll((long long)m) - 1;
                 if (dynamic) {
-                    if (lane == first) nb = (int)fixed_end + atomicAdd(cursor, chunk);
-                    nb = readlane_i32(nb, first);
+                    if (lane == first) nb = (uint32_t)fixed_end + (uint32_t)atomicAdd(cursor, chunk);
+                    nb = (uint32_t)readlane_i32((int)nb, first);
                 } else {
-                    nb = count;  // nothing past the fixed chunks
+                    nb = (uint32_t)count;  // nothing past the fixed chunks
                 }
             }
-            const int base = rank < avail ? cb : nb - avail;
+            const uint32_t base = rank < avail ? cb : nb - (uint32_t)avail;
             const bool served = rank < avail + (avail < c ? chunk : 0);
             if (avail < c) {
                 const int taken = c - avail < chunk ? c - avail : chunk;
-                cb = nb + taken;
-                ce = nb + chunk;
+                cb = nb + (uint32_t)taken;
+                ce = nb + (uint32_t)chunk;
             } else {
-                cb += c;
+                cb += (uint32_t)c;
             }
             if (need && served) {
-                const int idx = base + rank;
-                if (idx < count) {
-                    pid = order[begin + idx];
+                const uint32_t idx = base + (uint32_t)rank;
+                if (idx < (uint32_t)count) {
+                    pid = order[begin + (int)idx];
                     ia = pa[pid];
                     ib = pb[pid];
                     Shape A, B;
@@ -553,8 +565,7 @@ __device__ __forceinline__ void run_all(const d3d_scene &s, const int32_t *__res
         // wavefront when that is smaller, so a small batch spreads its pairs
         // over all wavefronts instead of a few wavefronts holding all of them
         const int full = prm.claim_factor * (kWave / G);
-        const int fair = (count + n_waves - 1) / n_waves;
-        const int chunk = fair < full ? fair : full;
+        const int chunk = claim_chunk(count, n_waves, full);
         if (cls == 0) {
             if (G <= 1) run_class<M, 1, false>(s, pa, pb, order, begin, count, cur, prm, o, pq_wave, chunk, rot);
             else if (G == 2) run_class<M, 2, false>(s, pa, pb, order, begin, count, cur, prm, o, pq_wave, chunk, rot);
@@ -570,8 +581,8 @@ __device__ __forceinline__ void run_all(const d3d_scene &s, const int32_t *__res
             default: run_class<M, 64, true>(s, pa, pb, order, begin, count, cur, prm, o, pq_wave, chunk, rot); break;
             }
         }
-        const int used = (count + chunk - 1) / chunk;
-        rot = (int)(((int64_t)rot + (used < n_waves ? used : n_waves)) % n_waves);
+        const uint32_t used = chunks_of(count, chunk);
+        rot = (int)(((int64_t)rot + (used < (uint32_t)n_waves ? (int)used : n_waves)) % n_waves);
     }
 }
 

@@ -1,14 +1,17 @@
-"""The hand-over of LDS rows inside a group of lanes, read from the sources: a
-group's first lane writes the rows of its pair and all its lanes read them, and
-without a fence between the two the compiler may keep the old row on the other
-lanes.  No run can show it missing while the compiler happens not to, so the
-step functions of the queue's modes are read instead."""
+"""The pair queue on the CPU.  The hand-over of LDS rows inside a group of lanes,
+read from the sources: a group's first lane writes the rows of its pair and all
+its lanes read them, and without a fence between the two the compiler may keep
+the old row on the other lanes.  No run can show it missing while the compiler
+happens not to, so the step functions of the queue's modes are read instead.
+And the queue's claims of pairs, run on the host."""
 import os
 import re
+import subprocess
 
 import pytest
 
-CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "distance3d_amd", "csrc")
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+CSRC = os.path.join(ROOT, "distance3d_amd", "csrc")
 
 
 def _bodies(path, name):
@@ -33,3 +36,15 @@ def test_steps_fence_before_they_read_rows(source, name, count):
         if read is not None:
             fence = re.search(r"\brow_fence\(\)", body)
             assert fence is not None and fence.start() < read.start()
+
+
+def test_claims_of_the_largest_classes(tmp_path):
+    exe = str(tmp_path / "queue_host_check")
+    try:
+        subprocess.run(["/opt/rocm/bin/hipcc", "-std=c++17", "-O1", "--offload-arch=gfx950", "-I", CSRC,
+                        "-I", os.path.join(ROOT, "include"), os.path.join(ROOT, "tests", "queue_host_check.hip"),
+                        "-o", exe], check=True, capture_output=True, timeout=300)
+    except FileNotFoundError:
+        pytest.skip("hipcc not available")
+    r = subprocess.run([exe], capture_output=True, text=True, timeout=60)
+    assert r.returncode == 0, r.stdout
