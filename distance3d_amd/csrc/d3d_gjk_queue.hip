@@ -689,20 +689,19 @@ int queue_sort(const d3d_scene &s, const int32_t *pa, const int32_t *pb, int64_t
     return D3D_OK;
 }
 
-d3d_gjk_params queue_params(const d3d_gjk_params &prm) {
+d3d_gjk_params queue_params(const d3d_gjk_params &prm, int64_t n, int64_t loose_max) {
     d3d_gjk_params rp = prm;
     for (int c = 0; c < kNumClasses; ++c) {
         int G = prm.lanes_per_pair[c] > 0 ? prm.lanes_per_pair[c] : -kDefaultLanes[c];
         if (c == 0 && G > 4) G = 4;
         rp.lanes_per_pair[c] = G;
     }
-    rp.blocks_per_cu = prm.blocks_per_cu > 0 ? prm.blocks_per_cu : 3;
+    rp.blocks_per_cu = batch_blocks(n, loose_max, prm.blocks_per_cu);
     rp.claim_factor = prm.claim_factor > 0 ? prm.claim_factor : 2;
     rp.epa_blocks_per_cu = prm.epa_blocks_per_cu > 0 ? prm.epa_blocks_per_cu : 8;
     return rp;
 }
 
-// resident at occupancy 3 (4 wavefronts per block) by default
 unsigned queue_grid(const d3d_gjk_params &resolved) {
     return (unsigned)(cu_count() * resolved.blocks_per_cu);
 }
@@ -715,10 +714,9 @@ static int launch_all(const d3d_scene &s, const int32_t *pa, const int32_t *pb, 
     const bool timed = stage_events(ev);
     if (timed) D3D_CHECK_HIP(hipEventRecord(ev[0], stream));
     if (int rc = queue_sort(s, pa, pb, n, w, stream, epa ? epa->count : nullptr)) return rc;
-    d3d_gjk_params rp = queue_params(prm);
+    const d3d_gjk_params rp = queue_params(prm, n, kLooseMax);
     if (timed) D3D_CHECK_HIP(hipEventRecord(ev[1], stream));
-    const bool loose = n <= kLooseMax;
-    if (loose && rp.blocks_per_cu > 2) rp.blocks_per_cu = 2;  // as many as are resident
+    const bool loose = batch_is_loose(n, kLooseMax, prm.blocks_per_cu);
     hipLaunchKernelGGL(loose ? gjk_small_kernel : gjk_all_kernel, dim3(queue_grid(rp)), dim3(kQBlock), 0,
                        stream, s, pa, pb, w.order, w.cls_begin, w.cls_count, w.cls_cursor, rp, o);
     D3D_CHECK_LAUNCH("gjk_all_kernel");
@@ -918,9 +916,8 @@ extern "C" int d3d_gjk_intersection_batch_ws(const d3d_scene *scene, const int32
     d3d_gjk_params prm = default_params();
     prm.tolerance = tolerance;
     prm.max_iterations = max_iterations;
-    const bool loose = n <= kIntersectLooseMax;
-    prm.blocks_per_cu = loose ? 2 : 3;
-    const d3d_gjk_params rp = queue_params(prm);
+    const bool loose = batch_is_loose(n, kIntersectLooseMax, 0);
+    const d3d_gjk_params rp = queue_params(prm, n, kIntersectLooseMax);
     const QueueWs w = ws_view(workspace, n);
     if (int rc = queue_sort(*scene, pair_a, pair_b, n, w, (hipStream_t)stream, nullptr)) return rc;
     hipLaunchKernelGGL(loose ? gjk_intersect_small_kernel : gjk_intersect_all_kernel,

@@ -580,7 +580,7 @@ extern "C" int d3d_mpr_batch_ws(const d3d_scene *scene, const int32_t *pair_a, c
                              status, out, stream);
     d3d_gjk_params prm = default_params();
     prm.blocks_per_cu = kMprBlocksPerCu;
-    const d3d_gjk_params rp = queue_params(prm);
+    const d3d_gjk_params rp = queue_params(prm, n, 0);
     const QueueWs w = ws_view(workspace, n);
     if (int rc = queue_sort(*scene, pair_a, pair_b, n, w, (hipStream_t)stream)) return rc;
     hipLaunchKernelGGL(mpr_all_kernel, dim3(queue_grid(rp)), dim3(kQBlock), 0, (hipStream_t)stream,

@@ -592,10 +592,21 @@ __device__ __forceinline__ void run_all(const d3d_scene &s, const int32_t *__res
 int queue_sort(const d3d_scene &s, const int32_t *pa, const int32_t *pb, int64_t n, const QueueWs &w,
                hipStream_t stream, unsigned long long *epa_count = nullptr);
 
+// Persistent blocks per compute unit for n pairs: the caller's where given, else
+// what is resident at the occupancy that suits the batch, 2 up to loose_max pairs
+// and 3 above.  A batch within loose_max runs the occupancy-2 kernel unless the
+// caller asks for more blocks than that holds.
+constexpr int batch_blocks(int64_t n, int64_t loose_max, int asked) {
+    return asked > 0 ? asked : n <= loose_max ? 2 : 3;
+}
+constexpr bool batch_is_loose(int64_t n, int64_t loose_max, int asked) {
+    return n <= loose_max && batch_blocks(n, loose_max, asked) <= 2;
+}
+
 // prm with the lanes per class (negative: the table's, which the kernel may
-// widen; positive: the caller's) and the launch shape resolved; the grid of a
-// persistent launch (kQBlock threads per block).
-d3d_gjk_params queue_params(const d3d_gjk_params &prm);
+// widen; positive: the caller's) and the launch shape resolved for n pairs; the
+// grid of a persistent launch (kQBlock threads per block).
+d3d_gjk_params queue_params(const d3d_gjk_params &prm, int64_t n, int64_t loose_max);
 unsigned queue_grid(const d3d_gjk_params &resolved);
 
 }  // namespace d3d

@@ -123,7 +123,8 @@ typedef struct d3d_scene {
  * copied there once and is swept from LDS; when both colliders are hulls the
  * two halves of the group sweep A and B concurrently.
  * Launch shape (0 = built-in default): blocks_per_cu persistent GJK blocks of
- * four wavefronts per compute unit (1..3, default 3); claim_factor: a
+ * four wavefronts per compute unit (1..3, default 2 up to 4,096 pairs and 3
+ * above); claim_factor: a
  * wavefront claims claim_factor * 64 / G pairs of a class at a time (1..8,
  * default 2; fewer when the class is small); epa_blocks_per_cu persistent EPA
  * wavefronts per compute unit in the fused pipeline (1..16, default 8). */

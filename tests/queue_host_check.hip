@@ -1,7 +1,8 @@
 // Host-side check of the pair queue's claims (d3d_queue.hpp), run on the CPU by
 // tests/test_queue_modes_host.py: for classes up to the largest, every chunk is
 // positive, the chunks cover the class, and no position a wavefront can claim
-// past the end leaves the 32 bits it is held in.
+// past the end leaves the 32 bits it is held in; and a caller's blocks per
+// compute unit are taken as given at every batch size.
 #include <cstdio>
 
 #include "d3d_queue.hpp"
@@ -27,6 +28,16 @@ int main() {
                     ++bad;
                 }
             }
+    for (int64_t n : {(int64_t)1, (int64_t)4096, (int64_t)4097, (int64_t)1 << 20})
+        for (int asked : {0, 1, 2, 3}) {
+            const int blocks = batch_blocks(n, 4096, asked);
+            // the occupancy-2 kernel holds two blocks per compute unit
+            if ((asked > 0 && blocks != asked) || blocks < 1 || blocks > 3 ||
+                (batch_is_loose(n, 4096, asked) && (blocks > 2 || n > 4096))) {
+                std::printf("FAIL %lld pairs, %d blocks asked: %d\n", (long long)n, asked, blocks);
+                ++bad;
+            }
+        }
     std::printf(bad ? "FAILED %d\n" : "OK\n", bad);
     return bad ? 1 : 0;
 }

@@ -248,3 +248,15 @@ def test_query_of_more_than_one_launch(gpu):
     got = kernels.bvh_query(kernels.bvh_build(boxes), q, cap=64, sort=False)
     del q
     assert torch.equal(got[torch.argsort(got[:, 0])].long(), torch.stack([at, torch.zeros_like(at)], 1))
+
+
+@pytest.mark.parametrize("n", (300, 4096, 4097))
+@pytest.mark.parametrize("blocks", (1, 2, 3))
+def test_distance_by_blocks_per_cu(gpu, n, blocks):
+    """A caller's blocks per compute unit, on both sides of the size at which the
+    default changes."""
+    host = workloads.mixed_pairs(seed=12, n_pairs=200).scene
+    a, b = np.random.RandomState(n).randint(0, host.n_shapes, (2, n)).astype(np.int32)
+    out = kernels.gjk_distance_batch(host.to_device(), a, b, launch={"blocks_per_cu": blocks})
+    want = oracle.gjk_distance(host, a, b)
+    assert np.array_equal(out.dist.cpu().numpy(), want["dist"])

@@ -3,7 +3,8 @@ read from the sources: a group's first lane writes the rows of its pair and all
 its lanes read them, and without a fence between the two the compiler may keep
 the old row on the other lanes.  No run can show it missing while the compiler
 happens not to, so the step functions of the queue's modes are read instead.
-And the queue's claims of pairs, run on the host."""
+And the queue's claims of pairs and the rule for its launch shape, run on the
+host."""
 import os
 import re
 import subprocess
@@ -38,7 +39,7 @@ def test_steps_fence_before_they_read_rows(source, name, count):
             assert fence is not None and fence.start() < read.start()
 
 
-def test_claims_of_the_largest_classes(tmp_path):
+def test_claims_and_launch_shape(tmp_path):
     exe = str(tmp_path / "queue_host_check")
     try:
         subprocess.run(["/opt/rocm/bin/hipcc", "-std=c++17", "-O1", "--offload-arch=gfx950", "-I", CSRC,
