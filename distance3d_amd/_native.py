@@ -50,6 +50,9 @@ class d3d_scene(ctypes.Structure):
 ABI_VERSION = 5
 CLUSTER_SIZE = 16
 NOALLOC_MAX_PAIRS = 16384  # D3D_NOALLOC_MAX_PAIRS
+# fewer pairs than these take the lane-per-pair kernels, which need no scratch
+INTERSECTION_QUEUE_MIN = 16  # D3D_INTERSECTION_QUEUE_MIN
+MPR_QUEUE_MIN = 32  # D3D_MPR_QUEUE_MIN
 
 
 class d3d_gjk_params(ctypes.Structure):

@@ -891,11 +891,11 @@ extern "C" int d3d_gjk_distance_batch_ws(const d3d_scene *scene, const int32_t *
 }
 
 // Pairs below which the sort costs more than it saves: with hulls in the scene 1
-// mixed pair takes 9 us in the lane-per-pair kernel and 14 us here, 16 pairs 33
-// and at most the 25 us that 64 pairs take here (90 us there), 262,144 pairs 747
-// and 409 us.  A scene without hulls has nothing to sort for (262,144 pairs of
+// mixed pair takes 9 us in the lane-per-pair kernel and 14 us here; 16 pairs take
+// 15 to 33 there, as their largest hull is, and 17 to 20 here, 24 pairs 29 and 20,
+// 64 pairs 90 and 25, 262,144 pairs 747 and 409 us.  A scene without hulls has nothing to sort for (262,144 pairs of
 // boxes 49 and 75 us).
-constexpr int64_t kIntersectQueueMin = 16;
+constexpr int64_t kIntersectQueueMin = D3D_INTERSECTION_QUEUE_MIN;
 
 extern "C" int d3d_gjk_intersection_batch_ws(const d3d_scene *scene, const int32_t *pair_a,
                                              const int32_t *pair_b, int64_t n, double tolerance,
@@ -906,13 +906,14 @@ extern "C" int d3d_gjk_intersection_batch_ws(const d3d_scene *scene, const int32
     if (int rc = check_scene(scene)) return rc;
     D3D_CHECK_ARG(n >= 0, "n must be >= 0");
     if (n == 0) return D3D_OK;
-    D3D_CHECK_ARG(pair_a && pair_b && hit && workspace, "NULL buffer");
+    D3D_CHECK_ARG(pair_a && pair_b && hit, "NULL buffer");
     D3D_CHECK_ARG(max_iterations > 0, "max_iterations must be > 0");
-    D3D_CHECK_ARG(workspace_bytes >= d3d_gjk_workspace_bytes(n), "workspace too small");
     // (the queue holds pair indices as int32)
     if (n < kIntersectQueueMin || n >= (int64_t)0x7fffffff || scene->n_vertices == 0)
         return d3d_gjk_intersection_batch(scene, pair_a, pair_b, n, tolerance, max_iterations, hit,
                                           status, stream);
+    D3D_CHECK_ARG(workspace, "NULL buffer");
+    D3D_CHECK_ARG(workspace_bytes >= d3d_gjk_workspace_bytes(n), "workspace too small");
     d3d_gjk_params prm = default_params();
     prm.tolerance = tolerance;
     prm.max_iterations = max_iterations;

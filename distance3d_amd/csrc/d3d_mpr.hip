@@ -560,7 +560,7 @@ extern "C" int d3d_mpr_batch(const d3d_scene *scene, const int32_t *pair_a, cons
 // take 13.7 and 19.0 us for 8 mixed pairs, 19.7 and 21.1 for 16, 35.8 and 23.7
 // for 32.  A scene without hulls has nothing to sort for (262,144 pairs of boxes
 // 56 and 77 us).
-constexpr int64_t kMprQueueMin = 32;
+constexpr int64_t kMprQueueMin = D3D_MPR_QUEUE_MIN;
 
 extern "C" int d3d_mpr_batch_ws(const d3d_scene *scene, const int32_t *pair_a, const int32_t *pair_b,
                                 const double *centers, int64_t n, double tolerance,
@@ -571,13 +571,14 @@ extern "C" int d3d_mpr_batch_ws(const d3d_scene *scene, const int32_t *pair_a, c
     if (int rc = check_scene(scene)) return rc;
     D3D_CHECK_ARG(n >= 0, "n must be >= 0");
     if (n == 0) return D3D_OK;
-    D3D_CHECK_ARG(pair_a && pair_b && centers && status && workspace, "NULL buffer");
+    D3D_CHECK_ARG(pair_a && pair_b && centers && status, "NULL buffer");
     D3D_CHECK_ARG(penetration == 0 || out, "out is NULL but penetration was requested");
     D3D_CHECK_ARG(max_iterations > 0, "max_iterations must be > 0");
-    D3D_CHECK_ARG(workspace_bytes >= d3d_gjk_workspace_bytes(n), "workspace too small");
     if (n < kMprQueueMin || n >= (int64_t)0x7fffffff || scene->n_vertices == 0)
         return d3d_mpr_batch(scene, pair_a, pair_b, centers, n, tolerance, max_iterations, penetration,
                              status, out, stream);
+    D3D_CHECK_ARG(workspace, "NULL buffer");
+    D3D_CHECK_ARG(workspace_bytes >= d3d_gjk_workspace_bytes(n), "workspace too small");
     d3d_gjk_params prm = default_params();
     prm.blocks_per_cu = kMprBlocksPerCu;
     const d3d_gjk_params rp = queue_params(prm, n, 0);

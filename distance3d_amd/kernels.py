@@ -167,6 +167,16 @@ def gjk_workspace_bytes(n):
     return int(_native.load_library().d3d_gjk_workspace_bytes(int(n)))
 
 
+def _queue_workspace(scene, n, queue_min):
+    """Scratch of a queued batch of n pairs and its size; none where the pairs are
+    not queued (fewer than queue_min, or no hulls), as the allocation is a tenth
+    of a small call."""
+    if n < queue_min or scene._c.n_vertices == 0:
+        return None, 0
+    ws = _workspace(gjk_workspace_bytes(n), scene.device)
+    return ws, ws.numel()
+
+
 @_on_stream
 def gjk_intersection_batch(scene, pair_a, pair_b, tolerance=1e-10, max_iterations=128,
                            want_status=False, stream=None):
@@ -179,10 +189,10 @@ def gjk_intersection_batch(scene, pair_a, pair_b, tolerance=1e-10, max_iteration
         raise ValueError("pair_a and pair_b differ in length")
     hit = torch.empty(n, dtype=torch.uint8, device=scene.device)
     status = torch.empty(n, dtype=torch.int32, device=scene.device) if want_status else None
-    ws = _workspace(gjk_workspace_bytes(n), scene.device)
+    ws, ws_bytes = _queue_workspace(scene, n, _native.INTERSECTION_QUEUE_MIN)
     check(lib().d3d_gjk_intersection_batch_ws(
         scene.c, ptr(a), ptr(b), n, float(tolerance), int(max_iterations), ptr(hit),
-        ptr(status), ptr(ws), ws.numel(), stream_ptr(stream)), "d3d_gjk_intersection_batch_ws")
+        ptr(status), ptr(ws), ws_bytes, stream_ptr(stream)), "d3d_gjk_intersection_batch_ws")
     return hit, status
 
 
@@ -206,10 +216,10 @@ def mpr_batch(scene, pair_a, pair_b, centers, tolerance=0.0001, max_iterations=1
                          % (scene.n_shapes, c.shape[0]))
     status = torch.empty(n, dtype=torch.int32, device=scene.device)
     out = torch.empty((n, 7), dtype=torch.float64, device=scene.device) if penetration else None
-    ws = _workspace(gjk_workspace_bytes(n), scene.device)
+    ws, ws_bytes = _queue_workspace(scene, n, _native.MPR_QUEUE_MIN)
     check(lib().d3d_mpr_batch_ws(scene.c, ptr(a), ptr(b), ptr(c), n, float(tolerance),
                                  int(max_iterations), 1 if penetration else 0, ptr(status),
-                                 ptr(out), ptr(ws), ws.numel(), stream_ptr(stream)),
+                                 ptr(out), ptr(ws), ws_bytes, stream_ptr(stream)),
           "d3d_mpr_batch_ws")
     return status, out
 

@@ -253,8 +253,11 @@ int d3d_gjk_intersection_batch(const d3d_scene *scene, const int32_t *pair_a,
 /*
  * d3d_gjk_intersection_batch through the sorted pair queue of the distance
  * pipeline (same results): faster for all but the smallest batches, with a
- * caller-owned workspace of d3d_gjk_workspace_bytes(n) bytes.
+ * caller-owned workspace of d3d_gjk_workspace_bytes(n) bytes.  Fewer than
+ * D3D_INTERSECTION_QUEUE_MIN pairs, and a scene without hull vertices, take
+ * d3d_gjk_intersection_batch and need no workspace (NULL, 0).
  */
+#define D3D_INTERSECTION_QUEUE_MIN 16
 int d3d_gjk_intersection_batch_ws(const d3d_scene *scene, const int32_t *pair_a,
                                   const int32_t *pair_b, int64_t n, double tolerance,
                                   int32_t max_iterations, uint8_t *hit, int32_t *status,
@@ -360,8 +363,11 @@ int d3d_mpr_batch(const d3d_scene *scene, const int32_t *pair_a, const int32_t *
 /*
  * d3d_mpr_batch through the sorted pair queue of the GJK distance pipeline
  * (same results): faster for all but the smallest batches, with a caller-owned
- * workspace of d3d_gjk_workspace_bytes(n) bytes.
+ * workspace of d3d_gjk_workspace_bytes(n) bytes.  Fewer than D3D_MPR_QUEUE_MIN
+ * pairs, and a scene without hull vertices, take d3d_mpr_batch and need no
+ * workspace (NULL, 0).
  */
+#define D3D_MPR_QUEUE_MIN 32
 int d3d_mpr_batch_ws(const d3d_scene *scene, const int32_t *pair_a, const int32_t *pair_b,
                      const double *centers, int64_t n, double tolerance, int32_t max_iterations,
                      int32_t penetration, int32_t *status, double *out, void *workspace,

@@ -2,6 +2,7 @@
 launches and read-backs on that stream: with the streams, the library and the
 allocations replaced, on the CPU."""
 import contextlib
+import os
 import types
 
 import numpy as np
@@ -58,7 +59,7 @@ def calls(monkeypatch):
 
 
 PAIRS = np.zeros(40, dtype=np.int32)
-SCENE = types.SimpleNamespace(device="cpu", n_shapes=3, c=None)
+SCENE = types.SimpleNamespace(device="cpu", n_shapes=3, c=None, _c=types.SimpleNamespace(n_vertices=8))
 TETS = [np.zeros((2, 4, 3)), np.zeros((2, 4)), np.zeros((2, 4, 4))]
 BVH = kernels.Bvh(torch.zeros((4, 3, 2), dtype=torch.float64), torch.zeros(4096, dtype=torch.uint8), 4)
 
@@ -83,3 +84,24 @@ def test_memory_and_launches_are_the_streams(calls, name):
     assert any(what.startswith("d3d_") for what, _ in calls)
     assert any(what in ("empty", "zeros") for what, _ in calls)
     assert all(on is stream for _, on in calls), [what for what, on in calls if on is not stream]
+
+
+@pytest.mark.parametrize("call, queue_min", [
+    (lambda scene, p: kernels.gjk_intersection_batch(scene, p, p), kernels._native.INTERSECTION_QUEUE_MIN),
+    (lambda scene, p: kernels.mpr_batch(scene, p, p, np.zeros((3, 3)), penetration=False),
+     kernels._native.MPR_QUEUE_MIN)])
+def test_no_scratch_where_pairs_are_not_queued(calls, call, queue_min):
+    """One allocation (the result) without the queue, two with it."""
+    hulls = types.SimpleNamespace(n_vertices=8)
+    none = types.SimpleNamespace(n_vertices=0)
+    for c, n, allocations in ((hulls, 1, 1), (hulls, queue_min - 1, 1), (hulls, queue_min, 2), (none, 4096, 1)):
+        del calls[:]
+        call(types.SimpleNamespace(device="cpu", n_shapes=3, c=None, _c=c), np.zeros(n, dtype=np.int32))
+        assert sum(what == "empty" for what, _ in calls) == allocations
+
+
+def test_queue_limits_match_the_header():
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    header = open(os.path.join(root, "include", "d3d.h")).read()
+    for name in ("INTERSECTION_QUEUE_MIN", "MPR_QUEUE_MIN"):
+        assert "#define D3D_%s %d\n" % (name, getattr(kernels._native, name)) in header
