@@ -148,6 +148,11 @@ def cluster_layout(host, min_vertices=CLUSTER_MIN_VERTICES, threads=0):
     return out
 
 
+# what the kernels read, whatever a caller has put in a HostScene's arrays
+_DTYPES = {"shape_f64": np.float64, "shape_i32": np.int32, "vx": np.float32, "vy": np.float32,
+           "vz": np.float32, "v64": np.float64, "vorig": np.int32, "clusters": np.float32}
+
+
 def _upload(layout, device):
     """The arrays of a scene layout as device tensors (None stays None, an empty
     array becomes one zero row).  The eight arrays of a small scene are views of
@@ -156,7 +161,7 @@ def _upload(layout, device):
     arrays = {}
     for name, a in layout.items():
         if a is not None:
-            a = np.ascontiguousarray(a) if len(a) else np.zeros((1,) + a.shape[1:], a.dtype)
+            a = np.ascontiguousarray(a if len(a) else np.zeros((1,) + a.shape[1:]), _DTYPES[name])
         arrays[name] = a
     total = sum((a.nbytes + 255) // 256 * 256 for a in arrays.values() if a is not None)
     if total > PACKED_UPLOAD_MAX:
