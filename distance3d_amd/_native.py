@@ -96,6 +96,7 @@ _SIGNATURES = {
     "d3d_bvh_build": [_P, _I64, _P, _I64, _P],
     "d3d_bvh_query": [_P, _I64, _P, _P, _I64, _P, _I64, _P, _P],
     "d3d_bvh_query_sorted": [_P, _I64, _P, _P, _I64, _P, _I64, _P, _P, _I64, _P],
+    "d3d_bvh_query_sorted_write": [_I64, _P, _I64, _I64, _P, _I64, _P],
     "d3d_bvh_query_sorted_finish": [_I64, _P, _I64, _P, _P, _I64, _P],
     "d3d_bvh_refit": [_P, _I64, _P, _I64, _P],
     "d3d_overlap_dense": [_P, _I64, _P, _I64, _P, _I64, _P, _P, _I64, _P],

@@ -686,11 +686,11 @@ __global__ __launch_bounds__(1024) void query_scan_kernel(unsigned long long *__
 
 // The pairs of kQueries queries (a block of the query kernel), 16 lanes each:
 // a list that fits the query's rows is ranked by counting the smaller indices
-// and written in order; of a longer one the rows are copied to its place in
-// `stage`, where query_spill_kernel adds the rest.
+// and written in order, to at most `room` rows; of a longer one the rows are
+// copied to its place in `stage`, where query_spill_kernel adds the rest.
 template <int kQueries>
-__global__ __launch_bounds__(kQueries * kHitRows) void query_write_kernel(int64_t m, int64_t cap,
-                                                                          QueryWs ws,
+__global__ __launch_bounds__(kQueries * kHitRows) void query_write_kernel(int64_t m, int64_t room,
+                                                                          int64_t cap, QueryWs ws,
                                                                           int32_t *__restrict__ pairs) {
     static_assert(kHitRows == 16 && kQueries >= 2 && kQueries <= 32, "16 lanes read at most two counts each");
     __shared__ int32_t cnt[32];
@@ -722,7 +722,7 @@ __global__ __launch_bounds__(kQueries * kHitRows) void query_write_kernel(int64_
 #pragma unroll
     for (int j = 0; j < kHitRows; ++j) rank += vals[g][j] < b ? 1 : 0;
     const unsigned long long pos = off + (unsigned long long)rank;
-    if (pos < (unsigned long long)cap) {
+    if (pos < (unsigned long long)room) {
         pairs[2 * pos] = (int32_t)q;
         pairs[2 * pos + 1] = b;
     }
@@ -999,6 +999,20 @@ static int64_t query_layout(int64_t m, int64_t cap, char *base, QueryWs *ws) {
     return b;
 }
 
+static int query_write(int64_t m, int32_t *pairs, int64_t room, int64_t cap, const QueryWs &ws,
+                       hipStream_t st) {
+    const int per = kBvhBlock / query_lanes(m);
+    auto go = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3((unsigned)((m + per - 1) / per)), dim3(per * kHitRows), 0, st, m,
+                           room, cap, ws, pairs);
+    };
+    if (per == 32) go(query_write_kernel<32>);
+    else if (per == 8) go(query_write_kernel<8>);
+    else go(query_write_kernel<4>);
+    D3D_CHECK_LAUNCH("query_write_kernel");
+    return D3D_OK;
+}
+
 extern "C" int64_t d3d_bvh_query_sorted_workspace_bytes(int64_t m, int64_t cap) {
     if (m < 0 || cap < 0) return -1;
     return query_layout(m, cap, nullptr, nullptr);
@@ -1012,7 +1026,7 @@ extern "C" int d3d_bvh_query_sorted(const void *bvh, int64_t n, const double *aa
     D3D_CHECK_ARG(n >= 1 && n < (int64_t)0x40000000, "n must be in [1, 2^30)");
     D3D_CHECK_ARG(m >= 1 && m < (int64_t)0x10000000, "m must be in [1, 2^28)");
     D3D_CHECK_ARG(cap >= 1, "cap must be >= 1");
-    D3D_CHECK_ARG(bvh && aabbs && queries && pairs && result && workspace, "NULL buffer");
+    D3D_CHECK_ARG(bvh && aabbs && queries && result && workspace, "NULL buffer");
     D3D_CHECK_ARG(workspace_bytes >= query_layout(m, cap, nullptr, nullptr), "workspace too small");
     hipStream_t st = (hipStream_t)stream;
     unsigned long long *res = (unsigned long long *)result;
@@ -1020,20 +1034,25 @@ extern "C" int d3d_bvh_query_sorted(const void *bvh, int64_t n, const double *aa
     query_layout(m, cap, (char *)workspace, &ws);
     hipLaunchKernelGGL(bvh_zero_counter, dim3(1), dim3(1), 0, st, res + 2);
     D3D_CHECK_LAUNCH("bvh_zero_counter");
-    query_launch<true>(bvh_view((void *)bvh, n), n, aabbs, queries, m, pairs, cap, res + 2, ws, st);
+    query_launch<true>(bvh_view((void *)bvh, n), n, aabbs, queries, m, nullptr, cap, res + 2, ws, st);
     D3D_CHECK_LAUNCH("bvh_query_kernel");
     const int per = kBvhBlock / query_lanes(m);
-    const int64_t blocks = (m + per - 1) / per;
-    hipLaunchKernelGGL(query_scan_kernel, dim3(1), dim3(1024), 0, st, ws.base, ws.most, blocks, res);
+    hipLaunchKernelGGL(query_scan_kernel, dim3(1), dim3(1024), 0, st, ws.base, ws.most, (m + per - 1) / per,
+                       res);
     D3D_CHECK_LAUNCH("query_scan_kernel");
-    auto write = [&](auto kernel) {
-        hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(per * kHitRows), 0, st, m, cap, ws, pairs);
-    };
-    if (per == 32) write(query_write_kernel<32>);
-    else if (per == 8) write(query_write_kernel<8>);
-    else write(query_write_kernel<4>);
-    D3D_CHECK_LAUNCH("query_write_kernel");
-    return D3D_OK;
+    return pairs ? query_write(m, pairs, cap, cap, ws, st) : D3D_OK;
+}
+
+extern "C" int d3d_bvh_query_sorted_write(int64_t m, int32_t *pairs, int64_t room, int64_t cap,
+                                          void *workspace, int64_t workspace_bytes, void *stream) {
+    clear_error();
+    D3D_CHECK_ARG(m >= 1 && m < (int64_t)0x10000000, "m must be in [1, 2^28)");
+    D3D_CHECK_ARG(cap >= 1 && room >= 1, "cap and room must be >= 1");
+    D3D_CHECK_ARG(pairs && workspace, "NULL buffer");
+    D3D_CHECK_ARG(workspace_bytes >= query_layout(m, cap, nullptr, nullptr), "workspace too small");
+    QueryWs ws;
+    query_layout(m, cap, (char *)workspace, &ws);
+    return query_write(m, pairs, room, cap, ws, (hipStream_t)stream);
 }
 
 extern "C" int d3d_bvh_query_sorted_finish(int64_t m, int32_t *pairs, int64_t cap,

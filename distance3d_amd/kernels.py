@@ -497,6 +497,9 @@ def bvh_query(bvh, queries, cap=None, counter=None, stream=None, sort=True):
 SORTED_QUERY_MAX_LIST = 1024
 # its scratch takes 80 bytes per query beside the pairs: 5 GB at this many
 SORTED_QUERY_MAX_QUERIES = 1 << 26
+# most room that is written before the number of pairs is known (1 MiB), as a
+# caller who keeps the result may keep all of it
+SORTED_QUERY_MAX_ROOM = 1 << 17
 
 
 def _bvh_query_sorted(bvh, q, cap, counter, stream):
@@ -509,7 +512,11 @@ def _bvh_query_sorted(bvh, q, cap, counter, stream):
     cap = 4 * m + min(12 * m, 1 << 22) + 1024 if cap is None else max(int(cap), 1)
     result = torch.empty(3, dtype=torch.int64, device=q.device)
     while True:
-        pairs = torch.empty((cap, 2), dtype=torch.int32, device=q.device)
+        # a small room is written before the number of pairs is known: the GPU would
+        # idle from the read-back to the launch (6,001 queries with their tree's
+        # refit 118 and 126 us)
+        room = cap if cap <= SORTED_QUERY_MAX_ROOM else 0
+        pairs = torch.empty((room, 2), dtype=torch.int32, device=q.device) if room else None
         ws = _workspace(lib().d3d_bvh_query_sorted_workspace_bytes(m, cap), q.device)
         check(lib().d3d_bvh_query_sorted(ptr(bvh.buffer), bvh.n, ptr(bvh.aabbs), ptr(q), m,
                                          ptr(pairs), cap, ptr(result), ptr(ws), ws.numel(),
@@ -517,9 +524,17 @@ def _bvh_query_sorted(bvh, q, cap, counter, stream):
         k, longest, spilled = result.tolist()
         if spilled and longest > SORTED_QUERY_MAX_LIST:
             return None
-        if k <= cap:
+        # short lists are all in their queries' rows
+        if not spilled or k <= cap:
             break
         cap = k
+    # a caller keeps at most 8 times its pairs, or 64 KiB (one query of 35 pairs 49 us
+    # and, written twice, 62)
+    if k > room or max(8 * k, 8192) < room:
+        pairs = torch.empty((k, 2), dtype=torch.int32, device=q.device)
+        if k:
+            check(lib().d3d_bvh_query_sorted_write(m, ptr(pairs), k, cap, ptr(ws), ws.numel(),
+                                                   stream_ptr(stream)), "d3d_bvh_query_sorted_write")
     if spilled:
         check(lib().d3d_bvh_query_sorted_finish(m, ptr(pairs), cap, ptr(result), ptr(ws), ws.numel(),
                                                 stream_ptr(stream)), "d3d_bvh_query_sorted_finish")

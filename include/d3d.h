@@ -478,11 +478,18 @@ int d3d_bvh_query(const void *bvh, int64_t n, const double *aabbs, const double 
  * query sort the output of d3d_bvh_query instead); when result[0] > cap call
  * again with more room.  m must be in [1, 2^28), cap >= 1; the workspace
  * (d3d_bvh_query_sorted_workspace_bytes(m, cap) bytes) is the caller's.
+ * With pairs == NULL the first call only finds and counts the pairs, and
+ * d3d_bvh_query_sorted_write, on the same m, cap and workspace, writes the first
+ * `room` of them, once or again: room may be result[0] exactly, and more than
+ * cap as long as result[2] == 0.  d3d_bvh_query_sorted_finish follows it where
+ * needed, into at least result[0] rows.
  */
 int64_t d3d_bvh_query_sorted_workspace_bytes(int64_t m, int64_t cap);
 int d3d_bvh_query_sorted(const void *bvh, int64_t n, const double *aabbs, const double *queries,
                          int64_t m, int32_t *pairs, int64_t cap, uint64_t *result, void *workspace,
                          int64_t workspace_bytes, void *stream);
+int d3d_bvh_query_sorted_write(int64_t m, int32_t *pairs, int64_t room, int64_t cap, void *workspace,
+                               int64_t workspace_bytes, void *stream);
 int d3d_bvh_query_sorted_finish(int64_t m, int32_t *pairs, int64_t cap, const uint64_t *result,
                                 void *workspace, int64_t workspace_bytes, void *stream);
 

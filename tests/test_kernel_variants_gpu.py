@@ -260,3 +260,31 @@ def test_distance_by_blocks_per_cu(gpu, n, blocks):
     out = kernels.gjk_distance_batch(host.to_device(), a, b, launch={"blocks_per_cu": blocks})
     want = oracle.gjk_distance(host, a, b)
     assert np.array_equal(out.dist.cpu().numpy(), want["dist"])
+
+
+@pytest.mark.parametrize("hits", (0, 1, 5, 40, 550, 1050, 2000))
+def test_ordered_pairs_hold_little_spare_room(gpu, hits):
+    """What a caller keeps of an ordered query is at most 8 times its pairs or 64
+    KiB, for short, long and sorted lists."""
+    boxes = np.zeros((max(hits, 1), 3, 2))
+    boxes[:, :, 1] = 1.0
+    queries = np.full((3000, 3, 2), 50.0)
+    if hits:
+        queries[7] = [0.5, 0.6]
+    pairs = kernels.bvh_query(kernels.bvh_build(boxes), queries)
+    assert np.array_equal(pairs.cpu().numpy(), np.stack([np.full(hits, 7), np.arange(hits)], 1))
+    assert pairs.untyped_storage().nbytes() <= max(64 * hits, 1 << 16)
+
+
+def test_ordered_pairs_of_a_large_batch(gpu):
+    """Enough queries for the smaller room per query, with short and long lists."""
+    m = 400003
+    rs = np.random.RandomState(4)
+    boxes = _boxes(rs, 500, 30.0, 0.8)
+    boxes[:30] = [[4.0, 4.5]] * 3
+    queries = _boxes(rs, m, 30.0, 0.8)
+    queries[::50000] = [[4.2, 4.3]] * 3
+    bvh = kernels.bvh_build(boxes)
+    pairs = kernels.bvh_query(bvh, queries)
+    assert np.array_equal(pairs.cpu().numpy(), kernels.overlap_dense(queries, boxes).cpu().numpy())
+    assert pairs.untyped_storage().nbytes() <= 8 * len(pairs) + (1 << 20)
