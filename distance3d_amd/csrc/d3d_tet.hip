@@ -73,7 +73,7 @@ __device__ __forceinline__ bool contact_plane(const double *__restrict__ p1,
 
 // check_tetrahedra_intersect_contact_plane (:232-258), tolerance 1e-6: the
 // plane has points of T on both sides.
-__device__ __forceinline__ bool plane_cuts(const double *__restrict__ T, const double (&h)[4]) {
+__device__ __forceinline__ bool plane_cuts(const double *T, const double (&h)[4]) {
     double mn = 0.0, mx = 0.0;
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
@@ -88,21 +88,32 @@ __device__ __forceinline__ bool plane_cuts(const double *__restrict__ T, const d
 // and whether it cuts both tetrahedra.  Only the pairs it cuts (40% of random
 // pairs, 60% of a contact's candidates) have a polygon to clip, by far the
 // longer part, so they wait in an LDS queue, with their planes, until 64 of them
-// fill the lanes.
+// fill the lanes.  kGeometry: planes and polygons are wanted.  Without them the
+// pairs are candidates as a broad phase lists them, where neighbours share a
+// tetrahedron and are cut or missed together: 64 pairs of which kDirect are cut
+// are clipped at once by their own lanes, whose data are still at hand.
 // Polygon rows are first filled with NaN by the whole wavefront in consecutive
 // stores; a lane that filled its own row stored 8 bytes every 576.
 // Bound: FP64 instructions of the clipping, and with polygons the 576 bytes a
-// pair takes.  524,289 random pairs, planes and polygons: 277 us one pair per
+// pair takes.  524,289 random pairs, planes and polygons: 273 us one pair per
 // lane throughout, 196 us where the queue held the pairs only and their planes
-// were computed again, 186 us now; status only 168, 143 and 137 us.  Where the
-// planes cut most pairs the queue has little to gain: the whole contact of two
-// deeply overlapping bodies, 5,094,572 candidates, 1.01, 1.09 and 1.03 ms.
+// were computed again, 179 us now.  Status only, one pair per lane throughout,
+// all cut pairs queued, and now: 524,289 random pairs 166, 136 and 139 us;
+// candidates of two bodies, less deep from one to the next, 18,158,524 1,200,
+// 1,206 and 1,077 us, 12,344,112 915, 965 and 870 us, 5,094,572 565, 590 and 567
+// us, 1,686,636 241, 270 and 246 us, 453,088 88, 97 and 88 us.  With kDirect 48
+// they take 1,084, 880, 575, 244 and 88 us, with 32 1,126, 898, 583, 247 and 89.
+constexpr int kDirect = 62;
+
+template <bool kGeometry>
 __global__ __launch_bounds__(kTetBlock) void tet_pair_kernel(
     const double *__restrict__ T1, const double *__restrict__ e1, const double *__restrict__ X1,
     const double *__restrict__ T2, const double *__restrict__ e2, const double *__restrict__ X2,
     const int32_t *__restrict__ pairs, int64_t m, double E1, double E2,
-    int32_t *__restrict__ status_out, double *__restrict__ planes, int32_t *__restrict__ nv_out,
-    double *__restrict__ polys, double *__restrict__ work) {
+    int32_t *__restrict__ status_out, double *__restrict__ planes_out, int32_t *__restrict__ nv_out,
+    double *__restrict__ polys_out, double *__restrict__ work) {
+    double *const planes = kGeometry ? planes_out : nullptr;
+    double *const polys = kGeometry ? polys_out : nullptr;
     __shared__ double ang_s[kTetMaxPoly][kTetBlock];
     __shared__ unsigned char ord_s[kTetMaxPoly][kTetBlock];
     // a ring of the waiting pairs, their tetrahedra and their planes; a pair of
@@ -117,14 +128,12 @@ __global__ __launch_bounds__(kTetBlock) void tet_pair_kernel(
     double *pts = work + 2 * kTetMaxPoly * ((int64_t)blockIdx.x * kTetBlock + lane);
     int first = 0, waiting = 0;  // pairs in the queue
 
-    // the polygons of the first `count` pairs of the queue
-    auto clip = [&](int count) {
+    // the polygons of the active lanes' pairs, items as in the queue
+    auto clip = [&](bool active, int64_t item, int2 ij, double (&h)[4]) {
     // the NaN rows are in memory before polygon points go over them
     if (polys) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    if (lane < count) {
-    const int slot = (first + lane) & (2 * kTetBlock - 1);
-    const int64_t item = queue[slot], k = item < 0 ? ~item : item;
-    const int2 ij = queue_ij[slot];
+    if (active) {
+    const int64_t k = item < 0 ? ~item : item;
     const int64_t i = ij.x, j = ij.y;
     const double *t2 = T2 + 12 * j;
     const double *x1 = X1 + 16 * i, *x2 = X2 + 16 * j;
@@ -133,9 +142,6 @@ __global__ __launch_bounds__(kTetBlock) void tet_pair_kernel(
     // count only)
     double *poly = polys ? polys + 3 * kTetMaxPoly * k : nullptr;
     int status = 0, nv = 0;
-    double h[4];
-#pragma unroll
-    for (int c = 0; c < 4; ++c) h[c] = queue_h[c][slot];
     if (item < 0) {
         // _handle_same_tetrahedron (:142-159)
         double sum = 0.0;
@@ -273,27 +279,37 @@ __global__ __launch_bounds__(kTetBlock) void tet_pair_kernel(
     status_out[k] = status;
     nv_out[k] = nv;
     }
-    // their slots are free for what is queued next
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    first = (first + count) & (2 * kTetBlock - 1);
-    waiting -= count;
     };
 
-    // the pairs of the next 64 are loaded ahead
+    // with geometry the pairs of the next 64 are loaded ahead (181 and 179 us for the
+    // random pairs, but 1,078 and 1,100 us for 18,158,524 candidates without)
     auto load_pair = [&](int64_t k) { return k < m ? make_int2(pairs[2 * k], pairs[2 * k + 1]) : make_int2(0, 0); };
-    int2 ij = load_pair((int64_t)blockIdx.x * kTetBlock + lane);
+    int2 next = kGeometry ? load_pair((int64_t)blockIdx.x * kTetBlock + lane) : make_int2(0, 0);
     for (int64_t base = (int64_t)blockIdx.x * kTetBlock; base < m || waiting > 0;
          base += (int64_t)gridDim.x * kTetBlock) {
         const int64_t k = base + lane;
-        const int2 here = ij;
-        ij = load_pair(k + (int64_t)gridDim.x * kTetBlock);
+        const int2 here = kGeometry ? next : load_pair(k);
+        if (kGeometry) next = load_pair(k + (int64_t)gridDim.x * kTetBlock);
         bool same = false, clipped = false;
         double h[4];
         if (k < m) {
             const int64_t i = here.x, j = here.y;
-            same = contact_plane(e1 + 4 * i, X1 + 16 * i, E1, e2 + 4 * j, X2 + 16 * j, E2, h);
-            clipped = same || (plane_cuts(T1 + 12 * i, h) && plane_cuts(T2 + 12 * j, h));
+            if constexpr (kGeometry) {
+                same = contact_plane(e1 + 4 * i, X1 + 16 * i, E1, e2 + 4 * j, X2 + 16 * j, E2, h);
+                clipped = same || (plane_cuts(T1 + 12 * i, h) && plane_cuts(T2 + 12 * j, h));
+            } else {
+                // all loads go out together; random pairs, which geometry is asked of
+                // too, are better off without those they do not need
+                double t1[12], t2[12];
+#pragma unroll
+                for (int c = 0; c < 12; ++c) {
+                    t1[c] = T1[12 * i + c];
+                    t2[c] = T2[12 * j + c];
+                }
+                same = contact_plane(e1 + 4 * i, X1 + 16 * i, E1, e2 + 4 * j, X2 + 16 * j, E2, h);
+                const bool cuts1 = plane_cuts(t1, h), cuts2 = plane_cuts(t2, h);
+                clipped = same || (cuts1 && cuts2);
+            }
             if (!clipped) {
                 if (planes) {
                     double *plane = planes + 4 * k;
@@ -309,19 +325,40 @@ __global__ __launch_bounds__(kTetBlock) void tet_pair_kernel(
             for (int64_t q = lane; q < values; q += kTetBlock) fill[q] = NAN;
         }
         const unsigned long long mask = __ballot(clipped);
-        if (clipped) {
-            const int slot = (first + waiting + __popcll(mask & lt)) & (2 * kTetBlock - 1);
-            queue[slot] = same ? ~k : k;
-            queue_ij[slot] = here;
+        int64_t item = same ? ~k : k;
+        int2 clip_ij = here;
+        bool active = clipped, now = !kGeometry && __popcll(mask) >= kDirect;
+        if (!now) {
+            if (clipped) {
+                const int slot = (first + waiting + __popcll(mask & lt)) & (2 * kTetBlock - 1);
+                queue[slot] = item;
+                queue_ij[slot] = here;
 #pragma unroll
-            for (int c = 0; c < 4; ++c) queue_h[c][slot] = h[c];
+                for (int c = 0; c < 4; ++c) queue_h[c][slot] = h[c];
+            }
+            waiting += __popcll(mask);
+            // the lanes read what the others queued
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            now = waiting >= kTetBlock || base + (int64_t)gridDim.x * kTetBlock >= m;
+            if (now) {
+                const int count = min(waiting, kTetBlock);
+                active = lane < count;
+                if (active) {
+                    const int slot = (first + lane) & (2 * kTetBlock - 1);
+                    item = queue[slot];
+                    clip_ij = queue_ij[slot];
+#pragma unroll
+                    for (int c = 0; c < 4; ++c) h[c] = queue_h[c][slot];
+                }
+                // their slots are free for what is queued next
+                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+                first = (first + count) & (2 * kTetBlock - 1);
+                waiting -= count;
+            }
         }
-        waiting += __popcll(mask);
-        // the lanes read what the others queued
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        if (waiting >= kTetBlock || base + (int64_t)gridDim.x * kTetBlock >= m)
-            clip(min(waiting, kTetBlock));
+        if (now) clip(active, item, clip_ij, h);
     }
 }
 
@@ -577,8 +614,11 @@ __global__ __launch_bounds__(kTetBlock) void angle_kernel(const double *__restri
 
 using namespace d3d;
 
-// blocks the workspace has rows for (one per lane), and the blocks launched:
-// what the chip holds (256 CUs x 8), so that a large batch fills its queues
+// Blocks the workspace has rows for (one per lane), and blocks launched: with
+// geometry what the chip holds (256 CUs x 8), so that a large batch fills its
+// queues (524,289 random pairs 179 us, with 4,096 blocks 189 us); without it all,
+// which even out the candidate lists' dense and sparse parts (1,686,636
+// candidates 246 us, with 2,048 blocks 257 us).
 constexpr int64_t kTetMaxBlocks = 4096;
 constexpr int64_t kTetGrid = 2048;
 
@@ -600,10 +640,13 @@ extern "C" int d3d_tet_pairs_batch(const double *T1, const double *e1, const dou
     D3D_CHECK_ARG(T1 && e1 && X1 && T2 && e2 && X2 && pairs && status && n_vertices && workspace,
                   "NULL buffer");
     D3D_CHECK_ARG(workspace_bytes >= d3d_tet_pairs_workspace_bytes(m), "workspace too small");
-    const unsigned blocks = (unsigned)min((int64_t)grid_for(m, kTetBlock), kTetGrid);
-    hipLaunchKernelGGL(tet_pair_kernel, dim3(blocks), dim3(kTetBlock), 0,
-                       (hipStream_t)stream, T1, e1, X1, T2, e2, X2, pairs, m, youngs_modulus1,
-                       youngs_modulus2, status, planes, n_vertices, polygons, (double *)workspace);
+    const bool geometry = planes || polygons;
+    const int64_t most = geometry ? kTetGrid : kTetMaxBlocks;
+    const unsigned blocks = (unsigned)min((int64_t)grid_for(m, kTetBlock), most);
+    hipLaunchKernelGGL(geometry ? tet_pair_kernel<true> : tet_pair_kernel<false>, dim3(blocks),
+                       dim3(kTetBlock), 0, (hipStream_t)stream, T1, e1, X1, T2, e2, X2, pairs, m,
+                       youngs_modulus1, youngs_modulus2, status, planes, n_vertices, polygons,
+                       (double *)workspace);
     D3D_CHECK_LAUNCH("tet_pair_kernel");
     return D3D_OK;
 }

@@ -288,3 +288,35 @@ def test_ordered_pairs_of_a_large_batch(gpu):
     pairs = kernels.bvh_query(bvh, queries)
     assert np.array_equal(pairs.cpu().numpy(), kernels.overlap_dense(queries, boxes).cpu().numpy())
     assert pairs.untyped_storage().nbytes() <= 8 * len(pairs) + (1 << 20)
+
+
+@pytest.mark.parametrize("dense", (40, 61, 62, 63, 64))
+@pytest.mark.parametrize("tiles", (1, 2, 9, 4097))
+def test_tet_status_of_dense_and_sparse_tiles(gpu, dense, tiles):
+    """Status-only pairs in tiles of 64 of which ``dense`` are cut, on both sides
+    of the line for clipping a tile at once, each with a sparse tile after it
+    whose pairs wait, coinciding tetrahedra among both."""
+    rs = np.random.RandomState(5)
+    n = 40
+    bodies = []
+    for _ in range(2):
+        T = rs.uniform(-0.6, 0.6, (n, 1, 3)) + 0.5 * rs.randn(n, 4, 3)
+        e = rs.uniform(0.0, 1.0, (n, 4))
+        bodies.append([T, e])
+    bodies[1][0][:10], bodies[1][1][:10] = bodies[0][0][:10], bodies[0][1][:10]
+    (T1, e1), (T2, e2) = bodies
+    X = [oracle.tet_mesh_prep(T)[1] for T, _ in bodies]
+    every = np.stack(np.meshgrid(np.arange(n), np.arange(n), indexing="ij"), -1).reshape(-1, 2).astype(np.int32)
+    every = every[rs.permutation(len(every))]
+    status, _, nv, _ = oracle.tet_pairs(T1, e1, X[0], T2, e2, X[1], every)
+    cut, missed = np.nonzero(status)[0], np.nonzero(status == 0)[0]
+    assert len(cut) > 100 and len(missed) > 100
+    rows = []
+    for t in range(tiles):
+        k = dense if t % 2 == 0 else 5
+        tile = np.concatenate([rs.choice(cut, k), rs.choice(missed, 64 - k)])
+        rows.append(tile[rs.permutation(64)])
+    rows = np.concatenate(rows)[:64 * tiles - 3]
+    got = kernels.tet_pairs_batch(T1, e1, X[0], T2, e2, X[1], every[rows], geometry=False)
+    assert np.array_equal(got[0].cpu().numpy(), status[rows])
+    assert np.array_equal(got[2].cpu().numpy(), nv[rows])
