@@ -122,45 +122,6 @@ __global__ __launch_bounds__(kBvhBlock) void bvh_bounds_partial(const double *__
     if (threadIdx.x < 6) part[6 * blockIdx.x + threadIdx.x] = red[threadIdx.x][0];
 }
 
-__device__ __forceinline__ uint32_t spread10(uint32_t v) {
-    v &= 0x3ffu;
-    v = (v | (v << 16)) & 0x030000FFu;
-    v = (v | (v << 8)) & 0x0300F00Fu;
-    v = (v | (v << 4)) & 0x030C30C3u;
-    v = (v | (v << 2)) & 0x09249249u;
-    return v;
-}
-
-// Position along a Hilbert curve of 10 bits per axis (J. Skilling, "Programming
-// the Hilbert curve", AIP Conf. Proc. 707, 2004: undo the excess rotations from
-// the top bit down, Gray-encode, interleave).  Consecutive positions are
-// neighbouring cells, so 8 rows in a row make tighter boxes than along a Morton
-// curve with its jumps: 65,536 queries of 1,048,576 boxes 130 us in Morton order
-// and 84 us in this one, 5,003 queries 24 and 19 us; the build 2 us longer.
-__device__ __forceinline__ uint32_t hilbert30(uint32_t x, uint32_t y, uint32_t z) {
-    auto turn = [&](uint32_t &v, uint32_t q) {
-        const uint32_t p = q - 1;
-        const uint32_t t = (v & q) ? 0u : (x ^ v) & p;
-        x ^= (v & q) ? p : t;
-        v ^= t;
-    };
-#pragma unroll
-    for (uint32_t q = 512; q > 1; q >>= 1) {
-        x ^= (x & q) ? q - 1 : 0u;
-        turn(y, q);
-        turn(z, q);
-    }
-    y ^= x;
-    z ^= y;
-    uint32_t t = 0;
-#pragma unroll
-    for (uint32_t q = 512; q > 1; q >>= 1) t ^= (z & q) ? q - 1 : 0u;
-    x ^= t;
-    y ^= t;
-    z ^= t;
-    return (spread10(x) << 2) | (spread10(y) << 1) | spread10(z);
-}
-
 __device__ __forceinline__ int item_digit(uint64_t item, int pass) {
     return (int)(item >> (32 + kDigitBits * pass)) & (kDigits - 1);
 }
@@ -375,8 +336,6 @@ __global__ __launch_bounds__(kBvhBlock) void rs_scatter_kernel(const uint64_t *_
 // of 8.  Bound: the gather of the boxes in curve order (1,048,576 boxes: 32
 // us, 48 bytes at random per box; the refit of the pointer tree this replaced
 // took 62 launches and 595 us).
-constexpr int kLevelBlock = 512;
-
 __device__ __forceinline__ void put_node(BvhNode *nd, const float (&lo)[3], const float (&hi)[3], int id) {
     float4 *p = reinterpret_cast<float4 *>(nd);
     p[0] = make_float4(lo[0], lo[1], lo[2], __int_as_float(id));
@@ -463,11 +422,8 @@ __global__ __launch_bounds__(kLevelBlock) void bvh_level_kernel(BvhLevels lv, in
 static void level_launches(const BvhView &v, const double *aabbs, int64_t n, const int32_t *order,
                            hipStream_t st) {
     const BvhLevels lv = bvh_levels(n);
-    for (int base = 0; base == 0 || base < lv.top; base += 3) {
-        // a block makes 512, 64, 8 and 1 rows of the four levels, so whole groups of
-        // 8 rows (with their padding) of the last one take a multiple of 8 blocks
-        int64_t blocks = (round8(lv.count[base]) + kLevelBlock - 1) / kLevelBlock;
-        if (base + 3 <= lv.top) blocks = round8(blocks);
+    for (int base = 0; base == 0 || base < lv.top; base += kLevelStep) {
+        const int64_t blocks = level_blocks(lv, base);
         if (base == 0)
             hipLaunchKernelGGL(bvh_level_kernel<true>, dim3((unsigned)blocks), dim3(kLevelBlock), 0, st, lv, base,
                                aabbs, order, v.nodes);
@@ -506,12 +462,6 @@ struct QueryWs {
 // their place in `pairs` with one atomic, later ones are appended as they are
 // found.  With an atomic per find 65,536 queries of 1,048,576 boxes (160,306
 // pairs) took 844 us, the atomics on the one counter; now 89 us.
-//
-// The stack: popping one node of level k at a time never leaves more than
-// 7 k + 1 entries above its own place (each of its 8 children is finished
-// before the next is taken), so QL = 8 needs 7 kBvhMaxLevels + 1 rows.  Wider
-// groups take more than one node only while what they could push stays within
-// kWide rows, and one at a time above that.
 constexpr int kBlockHits = 512;
 
 template <int QL, bool kSorted>
@@ -521,8 +471,7 @@ __global__ __launch_bounds__(kBvhBlock) void bvh_query_kernel(
     unsigned long long *__restrict__ counter, QueryWs ws) {
     constexpr int kGroups = kBvhBlock / QL;
     constexpr int W = QL / 8;
-    constexpr int kWide = W == 1 ? 0 : 20 * W;
-    constexpr int kStack = kWide + 7 * kBvhMaxLevels + 1;
+    constexpr int kStack = query_stack(W);
     __shared__ int32_t stack[kGroups][kStack];
     __shared__ int64_t off[kBvhMaxLevels];
     __shared__ int32_t found[kGroups];
@@ -552,7 +501,7 @@ __global__ __launch_bounds__(kBvhBlock) void bvh_query_kernel(
     int sp = valid ? 1 : 0;
     int cnt = 0;
     while (sp > 0) {
-        const int take = sp + 7 * W <= kWide ? min(sp, W) : 1;
+        const int take = query_take(sp, W);
         const int e = slot < take ? st[sp - 1 - slot] : -1;
         sp -= take;
         bool push = false, hit = false;
