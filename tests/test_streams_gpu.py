@@ -98,3 +98,34 @@ def test_box_overlaps(streams, call, cap):
             if call == "unsorted":
                 got = got[np.lexsort((got[:, 1], got[:, 0]))]
             assert np.array_equal(got, want)
+
+
+@pytest.mark.parametrize("n", (20, 300, 9000))
+def test_captured_batches(batches, n):
+    """Intersection and MPR in a captured graph, scratch and all: replays with new
+    pairs, and eager calls of another size between them."""
+    host, dev, _, centers = batches
+    c = torch.from_numpy(centers).cuda()
+    rs = np.random.RandomState(n)
+    a, b = (torch.from_numpy(rs.randint(0, host.n_shapes, n).astype(np.int32)).cuda() for _ in range(2))
+    stream = torch.cuda.Stream()
+    stream.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(stream):
+        kernels.gjk_intersection_batch(dev, a, b)
+        kernels.mpr_batch(dev, a, b, c)
+    stream.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        hit, _ = kernels.gjk_intersection_batch(dev, a, b)
+        status, out = kernels.mpr_batch(dev, a, b, c)
+    for _ in range(4):
+        pa, pb = rs.randint(0, host.n_shapes, (2, n)).astype(np.int32)
+        a.copy_(torch.from_numpy(pa))
+        b.copy_(torch.from_numpy(pb))
+        graph.replay()
+        kernels.gjk_intersection_batch(dev, np.repeat(pa, 2), np.repeat(pb, 2))
+        torch.cuda.synchronize()
+        assert np.array_equal(hit.cpu().numpy(), oracle.gjk_intersection(host, pa, pb)[0])
+        want = oracle.mpr(host, pa, pb, centers)
+        assert np.array_equal(status.cpu().numpy(), want[0])
+        assert np.array_equal(out.cpu().numpy(), want[1], equal_nan=True)
