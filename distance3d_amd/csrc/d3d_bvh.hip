@@ -879,10 +879,11 @@ extern "C" int d3d_bvh_refit(const double *aabbs, int64_t n, void *bvh, int64_t 
 
 // Lanes per query: few queries take wide groups (fewer rounds in a row each),
 // many fill the chip with narrow ones.  A sorted query of a tree of 1,048,576
-// boxes with 8 / 16 / 32 / 64 lanes (in Morton order, where all take longer): 300 queries 46 / 31 / 22 / 18 us, 5,003
-// queries 56 / 37 / 28 / 24, 16,384 queries 81 / 55 / 46 / 50, 32,768 queries
-// 94 / 73 / 74 / 88, 65,536 queries 130 / 132 / 138 / 173, 131,072 queries 232 /
-// 236 / 262 / 329 (the same order on trees of 5,003 and 100,003 boxes).
+// boxes with 8 / 16 / 32 / 64 lanes: 300 queries 34 / 23 / 19 / 17 us, 5,003
+// queries 38 / 27 / 21 / 20, 8,192 queries 40 / 29 / 23 / 24, 16,384 queries 55 /
+// 39 / 33 / 39, 32,768 queries 65 / 50 / 53 / 71, 49,152 queries 75 / 73 / 73 /
+// 98, 65,536 queries 84 / 93 / 97 / 139, 131,072 queries 148 / 155 / 185 / 264
+// (the same order on trees of 5,003 and 100,003 boxes).
 static int query_lanes(int64_t m) { return m < 8192 ? 64 : m < 49152 ? 32 : 8; }
 
 template <bool kSorted>

@@ -2,18 +2,19 @@
 // queue-fed pipeline (d3d_queue.hpp).
 //
 // 1. classify + counting sort (device): every pair gets a key
-//        work class (total hull vertices of the pair, 8 classes)
+//        work class (8 size classes of the pair's hull vertices, for pairs of
+//        at most one hull and for pairs of two)
 //        x collider type of A x collider type of B
 //    and the pair indices are scattered into `order`, grouped by key.  Pairs
 //    of one class have similar support-sweep cost and, within a class, run
 //    next to pairs of the same type combination, so the type switch of the
 //    analytic supports stays wave-uniform.
-// 2. one persistent kernel per class, G lanes per pair (G from the tuning
-//    table; 1 for analytic and small-hull pairs, more for big hulls).  The G
-//    lanes of a pair hold identical FP64 simplex state; hull sweeps stride
-//    over the vertices by G and reduce inside the group.  Each group takes
-//    its next pair from the class's device cursor as soon as its current
-//    pair terminates, so lanes do not idle on the slowest pair of a wave.
+// 2. one persistent kernel over all classes, G lanes per pair (G from the tuning
+//    table; 1 for analytic pairs, more for big hulls).  The G lanes of a pair
+//    hold identical FP64 simplex state; hull sweeps stride over the vertices by
+//    G and reduce inside the group.  Each group takes its next pair from its
+//    wavefront's claim on the class as soon as its current pair terminates, so
+//    lanes do not idle on the slowest pair of a wave.
 // Counts and offsets stay on the device: no host synchronisation inside a
 // batch.
 #include <array>

@@ -495,7 +495,8 @@ def bvh_query(bvh, queries, cap=None, counter=None, stream=None, sort=True):
 # longest list of one query that is ordered by counting (quadratic in its
 # length) instead of a sort of all pairs
 SORTED_QUERY_MAX_LIST = 1024
-# its scratch takes 80 bytes per query beside the pairs: 5 GB at this many
+# its scratch takes about 80 bytes per query and 16 per pair it has room for (4 per
+# query and 4,195,328 by default): 10 GB at this many
 SORTED_QUERY_MAX_QUERIES = 1 << 26
 # most room that is written before the number of pairs is known (1 MiB), as a
 # caller who keeps the result may keep all of it
