@@ -740,21 +740,20 @@ static int launch_all(const d3d_scene &s, const int32_t *pa, const int32_t *pb, 
 // pose_b[i]; NULL poses keep the scene's.  Vertex offsets are copied, so the
 // instances share the scene's resident vertex pools.
 __global__ __launch_bounds__(kQBlock) void instance_kernel(
-    d3d_scene s, const int32_t *__restrict__ a, const int32_t *__restrict__ b,
-    const double *__restrict__ pose_a, const double *__restrict__ pose_b,
-    const int32_t *__restrict__ pidx_a, const int32_t *__restrict__ pidx_b, int64_t n_poses,
-    int64_t n, double *__restrict__ f64, int32_t *__restrict__ i32, int32_t *__restrict__ inst_a,
-    int32_t *__restrict__ inst_b) {
+    d3d_scene s, const int32_t *a, const int32_t *b, const double *__restrict__ pose_a,
+    const double *__restrict__ pose_b, const int32_t *pidx_a, const int32_t *pidx_b, int64_t n_poses,
+    int64_t n, double *__restrict__ f64, int32_t *__restrict__ i32, int32_t *inst_a, int32_t *inst_b) {
     const int64_t t = (int64_t)blockIdx.x * kQBlock + threadIdx.x;
     if (t >= 2 * n) return;
     const int64_t pair = t >> 1;
     const int side = (int)(t & 1);
-    if (inst_a && inst_b) (side ? inst_b : inst_a)[pair] = (int32_t)t;
     const int k = side ? b[pair] : a[pair];
     const double *pose = side ? pose_b : pose_a;
     const int32_t *pidx = side ? pidx_b : pidx_a;
     int64_t prow = pair;
     if (pidx) prow = pidx[pair];
+    // after the reads: the lists written may be the ones read
+    if (inst_a && inst_b) (side ? inst_b : inst_a)[pair] = (int32_t)t;
     double *dst = f64 + 16 * t;
     int32_t *di = i32 + 4 * t;
     if (k < 0 || (int64_t)k >= s.n_shapes || (pose && pidx && (prow < 0 || prow >= n_poses))) {

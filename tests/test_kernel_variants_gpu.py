@@ -320,3 +320,27 @@ def test_tet_status_of_dense_and_sparse_tiles(gpu, dense, tiles):
     got = kernels.tet_pairs_batch(T1, e1, X[0], T2, e2, X[1], every[rows], geometry=False)
     assert np.array_equal(got[0].cpu().numpy(), status[rows])
     assert np.array_equal(got[2].cpu().numpy(), nv[rows])
+
+
+@pytest.mark.parametrize("n", (1, 129, 5000))
+def test_instances_written_over_their_pair_lists(gpu, n):
+    """Pair lists that are their own output: every instance is made from the list
+    as it was."""
+    host = workloads.mixed_pairs(seed=3, n_pairs=60).scene
+    dev = host.to_device()
+    rs = np.random.RandomState(n)
+    a, b = rs.randint(0, host.n_shapes, (2, n)).astype(np.int32)
+    poses = rs.uniform(-1.0, 1.0, (50, 12))
+    rows = rs.randint(0, 50, (2, n)).astype(np.int32)
+    cuda = lambda x: torch.from_numpy(x).cuda()
+    ia, ib, pa, pb = cuda(a), cuda(b), cuda(rows[0]), cuda(rows[1])
+    out = (torch.empty((2 * n, 16), dtype=torch.float64, device="cuda"),
+           torch.empty((2 * n, 4), dtype=torch.int32, device="cuda"), ia, ib)
+    view, va, vb = kernels.instance_pairs(dev, ia, ib, cuda(poses), cuda(poses), pa, pb, 50, out=out)
+    ids = np.stack([a, b], 1).reshape(-1)
+    want = host.shape_f64[ids].copy()
+    want[:, :12] = poses[rows.T.reshape(-1)]
+    assert np.array_equal(view.shape_i32[:, 0].cpu().numpy(), host.shape_i32[ids, 0])
+    assert np.array_equal(view.shape_f64[:, :12].cpu().numpy(), want[:, :12])
+    assert np.array_equal(va.cpu().numpy(), 2 * np.arange(n))
+    assert np.array_equal(vb.cpu().numpy(), 2 * np.arange(n) + 1)
